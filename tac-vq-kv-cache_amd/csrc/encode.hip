@@ -10,8 +10,10 @@
 //    tile of codewords x rows with exact products and fp32 accumulation; the
 //    argmin is a min over keys that carry the codeword index in their low
 //    bits.
-//  * rvq_encode_generic<DT,DMAX>: any dtype, d<=128, K<=256, any S, optional
-//    whitener; one thread per row, fp32 distances in the reference's
+//  * rvq_encode_generic<DT,DMAX>: what the MFMA kernels do not take (fp32
+//    states, other d, K or S; encode_grouped.hip and encode_bf16.hip hold the
+//    unwhitened 16-bit ones): d<=128, K<=256, any S, optional whitener; one
+//    thread per row, fp32 distances in the reference's
 //    |r|^2 + |c|^2 - 2 r.c form.
 #include "encode_args.h"
 
@@ -797,11 +799,11 @@ static int launch_mfma(const EncodeArgs& e, hipStream_t stream) {
   return launch_mfma<D, S>(e, nullptr, stream);
 }
 
-// Whether rvq_encode_mfma takes these arguments: fp16 states, d in {4, 8},
-// K = 256, S <= 2, no whitener, 16-byte aligned states and reconstructions,
-// and offsets that fit the kernel's 32-bit (24-bit for token strides)
-// arithmetic.
-static bool mfma_eligible(const EncodeArgs& a, int32_t states_dtype) {
+// Whether the grouped MFMA kernels take these arguments for 16-bit states:
+// d in {4, 8}, K = 256, S <= 2, no whitener, 16-byte aligned states and
+// reconstructions, and offsets that fit the kernels' 32-bit (24-bit for token
+// strides) arithmetic.
+static bool mfma_shape(const EncodeArgs& a) {
   const int64_t B = a.B, H = a.H, T = a.T, G = a.G, d = a.d, S = a.S;
   const bool aligned16 = (((uintptr_t)a.states) % 16 == 0) && a.sb % 8 == 0 && a.sh % 8 == 0 && a.st % 8 == 0;
   const bool codes_aligned =
@@ -818,9 +820,13 @@ static bool mfma_eligible(const EncodeArgs& a, int32_t states_dtype) {
                          x_span < ((int64_t)1 << 31) && c_span < ((int64_t)1 << 31) &&
                          B * H * T * G * d < ((int64_t)1 << 31) && a.st < ((int64_t)1 << 24) &&
                          a.ct < ((int64_t)1 << 24) && G * d < ((int64_t)1 << 24);
-  return offsets32 && states_dtype == JKV_F16 && a.whiteners == nullptr && a.K == 256 &&
+  return offsets32 && a.whiteners == nullptr && a.K == 256 &&
          (d == 8 || d == 4) && (S == 1 || S == 2) && aligned16 && codes_aligned && recon_aligned &&
          distinct_exits && B * T < ((int64_t)1 << 31) && T < ((int64_t)1 << 31);
+}
+// rvq_encode_mfma and rvq_encode_grouped multiply fp16 states
+static bool mfma_eligible(const EncodeArgs& a, int32_t states_dtype) {
+  return states_dtype == JKV_F16 && mfma_shape(a);
 }
 
 }  // namespace jkv
@@ -895,6 +901,10 @@ int jkv_rvq_encode(const void* states, int32_t states_dtype, int64_t B, int64_t 
       mfma_eligible(plain, states_dtype))
     return d == 4 ? launch_mfma<4, 1>(a, stream) : launch_mfma<8, 1>(a, stream);
   if (fast) return launch_grouped(a, nullptr, stream);
+  // bf16 states of the same geometries: their own MFMA kernel, at any row
+  // count (the one-row-per-thread kernel takes 370 us for a few rows, 866 us
+  // for 4,094; this one under 10 and 27 us)
+  if (states_dtype == JKV_BF16 && mfma_shape(a) && ((uintptr_t)tables) % 4 == 0) return launch_bf16(a, stream);
   // full-vector codebooks on MFMA (fp16-deployed tables in the workspace),
   // plain or whitened
   const bool full = states_dtype == JKV_F16 && d == 128 && K == 256 && S <= 32 && aligned16 &&

@@ -70,4 +70,7 @@ int launch_grouped(const EncodeArgs& e, const EncodeArgs* e2, hipStream_t stream
 // buffers (states, tables, codes, reconstructions).
 int launch_grouped_many(const EncodeArgs* jobs, int n, hipStream_t stream);
 
+// The same geometries for bf16 states, one job (encode_bf16.hip).
+int launch_bf16(const EncodeArgs& e, hipStream_t stream);
+
 }  // namespace jkv

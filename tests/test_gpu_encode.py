@@ -439,3 +439,57 @@ def test_rvq_decode_lds_runs_match_oracle(device, groups, stages, depth, tables_
     got = jkv.closed_loop_vq._ops.rvq_decode(codes.to(device), given.to(device), depth=depth, dtype=dtype)
     want = ref.frozen_decode(codes, tables, depth, dtype)
     assert torch.equal(got.cpu(), want)
+
+
+# bf16 states on the grouped MFMA kernel: slabs of 64 rows, 256 per workgroup
+# pass; one row, tile and slab edges, rows that straddle batch entries, strided
+# [B,T,H,D] views, both group widths, codebooks far from unit scale
+@pytest.mark.parametrize("batch,tokens,dim,stages,scale,strided", [
+    (1, 1, 8, 2, 1.0, False),
+    (3, 21, 8, 2, 1.0, True),
+    (2, 65, 8, 1, 1.0, False),
+    (1, 257, 4, 1, 1.0, False),
+    (5, 130, 4, 2, 1.0, True),
+    (1, 511, 8, 2, 2.0 ** -20, False),
+    (1, 511, 8, 2, 2.0 ** 9, False),
+    (2, 2048, 8, 2, 1.0, False),
+])
+def test_bf16_grouped_encode(device, batch, tokens, dim, stages, scale, strided):
+    print(f"bf16 encode B={batch} T={tokens} d={dim} S={stages} scale={scale} strided={strided}", flush=True)
+    gen = _gen(5100 + tokens + dim)
+    heads, groups = 2, 128 // dim
+    states = (ref.synthetic_states(gen, batch, heads, tokens).float() * scale).bfloat16()
+    tables = ref.synthetic_tables(gen, (heads, groups, stages, 256, dim), (1.0, 0.5)[:stages], stage_axis=2) * scale
+    given = states.transpose(1, 2).contiguous().transpose(1, 2) if strided else states
+    prefixes = tuple(range(1, stages + 1))
+    exits, codes = jkv.hard_grouped_residual_vq(given.to(device), tables.to(device), prefixes=prefixes)
+    r_exits, r_codes, d1, d2 = ref.grouped_residual_vq(states, tables, prefixes=prefixes, return_margins=True)
+    res = assert_codes(codes, r_codes, d1, d2)
+    rows = res["prefix_ok"]
+    # the one-row-per-thread fp32 search of the same values: the same codes
+    _, same = jkv.hard_grouped_residual_vq(states.float().to(device), tables.to(device), prefixes=prefixes)
+    assert torch.equal(codes, same)
+    for depth in prefixes:
+        assert exits[depth].dtype == torch.bfloat16
+        got = exits[depth].cpu().reshape(batch, heads, tokens, groups, dim)
+        want = r_exits[depth].detach().reshape(batch, heads, tokens, groups, dim)
+        assert torch.equal(got[rows], want[rows])
+
+
+def test_bf16_grouped_encode_outside_fp16(device):
+    # rows the kernel's fp16 words cannot carry (and a codebook of a problem
+    # that overflows them) take its fp32 scan, and the other rows the same
+    # codes: every code is the fp32 search's over the same values
+    gen = _gen(5200)
+    states = ref.synthetic_states(gen, 1, 2, 300).float()
+    states[0, 0, 3] *= 3e5
+    states[0, 0, 64:70] *= 1e20
+    states[0, 1, 7, 8:16] = float("inf")
+    states[0, 1, 9, 0] = float("nan")
+    states = states.bfloat16()
+    tables = ref.synthetic_tables(gen, (2, 16, 2, 256, 8), (1.0, 0.5), stage_axis=2)
+    tables[1, 5] *= 2e4
+    _, codes = jkv.hard_grouped_residual_vq(states.to(device), tables.to(device), prefixes=(2,))
+    _, want = jkv.hard_grouped_residual_vq(states.float().to(device), tables.to(device), prefixes=(2,))
+    codes, want = codes.cpu(), want.cpu()
+    assert torch.equal(codes, want)
