@@ -4,13 +4,18 @@
 // fp32 and not deployed to fp16, distance (|x|^2 + |c|^2) - 2 x.c, the lowest
 // index on ties (torch.argmin's rule).
 //
-// One 256-thread block takes 64 rows of one head and walks the head's table
+// D = 128 (a head) runs on the fp32 matrix instructions below; other
+// dimensions on nearest_f32_kernel.
+//
+// nearest_f32_kernel: one 256-thread block takes 64 rows of one head and walks the head's table
 // in 64-codeword tiles.  Rows and codewords are staged in LDS with a row
 // pitch of D rounded up to 4 plus 4 floats, so the 16 codeword rows a wave
 // reads at one k fall in distinct banks.  Thread (r, c) of the 16 x 16 grid
 // accumulates x.c for rows 4r..4r+3 and codewords 4c..4c+3 of the tile with
 // float4 LDS reads and keeps each row's best (distance, index); the 16
 // threads that share a row then reduce over lane shuffles.
+#include <algorithm>
+
 #include "jkv_common.h"
 
 namespace jkv {
@@ -146,6 +151,185 @@ __global__ __launch_bounds__(256) void nearest_f32_kernel(NearestArgs a) {
   }
 }
 
+
+// D = 128 and K <= 256: x.c on v_mfma_f32_32x32x2_f32 (fp32 products and
+// sums).  A 512-thread block holds the head's whole table in LDS, staged
+// once; each of its eight waves keeps 32 rows in registers as the B operand
+// and takes every SPLIT-th 32-codeword chunk, so a block covers 256 / SPLIT
+// rows.  Two chunks accumulate side by side.  The contraction's order is
+// free as long as A and B share it: lane half h takes dims 8m + 4h .. +3 of
+// step group m, so one 16-byte LDS read feeds four products.
+//
+// Bound: the fp32 matrix rate (64 cycles per product, 2 waves per SIMD); LDS
+// reads are 4 bytes per cycle and SIMD.  [8,8192,128] against 256 codewords:
+// 186 us on nearest_f32_kernel (23 TFLOP/s, bound by its LDS reads),
+// 43 us here (27 us of products; the rows' load and the table's staging lead).
+// Pitch 132 floats puts eight consecutive codewords' 16-byte pieces in
+// distinct banks.
+static const int kNmThreads = 512;
+static const int kNmCodes = 256;
+static const int kNmPitch = 132;
+static const int kNmLdsBytes = (kNmCodes * kNmPitch + kNmCodes) * 4;
+
+template <int SPLIT>
+__global__ __launch_bounds__(kNmThreads) void nearest_mfma_kernel(NearestArgs a) {
+  static_assert(SPLIT == 1 || SPLIT == 2 || SPLIT == 4 || SPLIT == 8, "waves per row tile");
+  extern __shared__ __align__(16) float nm_lds[];
+  float* cs = nm_lds;                       // [256][132]
+  float* s_cc = nm_lds + kNmCodes * kNmPitch;  // |c|^2, +inf past K
+  __shared__ float s_best[8][32];
+  __shared__ int s_idx[8][32];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, hf = lane >> 5;
+  const int K = (int)a.K;
+  const int chunks = (K + 31) >> 5;
+  const int64_t h = blockIdx.y;
+  constexpr int kTiles = 8 / SPLIT;  // 32-row tiles per block
+  const int tile = wave / SPLIT, part = wave % SPLIT;
+  const int64_t row = ((int64_t)blockIdx.x * kTiles + tile) * 32 + j;
+  const int64_t at = row < a.N ? row : a.N - 1;  // rows past N repeat the last
+
+  // this lane's half of its row: dims 8m + 4 hf .. +3
+  const float4* xsrc = (const float4*)(a.states + (h * a.N + at) * 128) + hf;
+  float4 x[16];
+#pragma unroll
+  for (int m = 0; m < 16; ++m) x[m] = xsrc[2 * m];
+
+  // the table, zero rows past K (up to a whole chunk), 16 bytes per thread
+  const float4* csrc = (const float4*)(a.tables + h * a.K * 128);
+  for (int i = tid; i < chunks * 32 * 32; i += kNmThreads) {
+    const int r = i >> 5, q = i & 31;
+    float4 v = {0.f, 0.f, 0.f, 0.f};
+    if (r < K) v = csrc[i];
+    *(float4*)(cs + r * kNmPitch + 4 * q) = v;
+  }
+  float xx = 0.f;
+#pragma unroll
+  for (int m = 0; m < 16; ++m) {
+    xx = fmaf(x[m].x, x[m].x, xx);
+    xx = fmaf(x[m].y, x[m].y, xx);
+    xx = fmaf(x[m].z, x[m].z, xx);
+    xx = fmaf(x[m].w, x[m].w, xx);
+  }
+  xx += __shfl_xor(xx, 32, 64);
+  __syncthreads();
+  if (tid < chunks * 32) {
+    float acc = __builtin_inff();
+    if (tid < K) {
+      acc = 0.f;
+      const float* c = cs + tid * kNmPitch;
+      for (int q = 0; q < 128; q += 4) {
+        const float4 v = *(const float4*)(c + q);
+        acc = fmaf(v.x, v.x, acc);
+        acc = fmaf(v.y, v.y, acc);
+        acc = fmaf(v.z, v.z, acc);
+        acc = fmaf(v.w, v.w, acc);
+      }
+    }
+    s_cc[tid] = acc;
+  }
+  __syncthreads();
+
+  float best = __builtin_inff();
+  int bidx = 0;
+  // chunks part, part + SPLIT, ...: two at a time
+  for (int c0 = part; c0 < chunks; c0 += 2 * SPLIT) {
+    const int c1 = c0 + SPLIT;
+    const bool two = c1 < chunks;
+    const float* ap0 = cs + (32 * c0 + j) * kNmPitch + 4 * hf;
+    const float* ap1 = two ? cs + (32 * c1 + j) * kNmPitch + 4 * hf : ap0;
+    float16v acc0 = {}, acc1 = {};
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      const float4 a0 = *(const float4*)(ap0 + 8 * m);
+      const float4 a1 = *(const float4*)(ap1 + 8 * m);
+      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, x[m].x, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, x[m].x, acc1, 0, 0, 0);
+      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, x[m].y, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, x[m].y, acc1, 0, 0, 0);
+      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, x[m].z, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, x[m].z, acc1, 0, 0, 0);
+      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, x[m].w, acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, x[m].w, acc1, 0, 0, 0);
+    }
+    // element el of lane (hf, j) is codeword 8 (el / 4) + 4 hf + el % 4 of the
+    // chunk: indices rise within the lane, so strict < keeps the first of
+    // equal distances
+    auto fold = [&](int c, const float16v& acc) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k0 = 32 * c + 8 * q + 4 * hf;
+        const float4 cc = *(const float4*)(s_cc + k0);
+        const float cv[4] = {cc.x, cc.y, cc.z, cc.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float dist = (xx + cv[e]) - 2.f * acc[4 * q + e];
+          if (dist < best) {
+            best = dist;
+            bidx = k0 + e;
+          }
+        }
+      }
+    };
+    fold(c0, acc0);
+    if (two) fold(c1, acc1);
+  }
+  // the other lane half holds the row's other codewords; the lower index wins ties
+  {
+    const float ob = __shfl_xor(best, 32, 64);
+    const int oi = __shfl_xor(bidx, 32, 64);
+    if (ob < best || (ob == best && oi < bidx)) {
+      best = ob;
+      bidx = oi;
+    }
+  }
+  if constexpr (SPLIT > 1) {
+    if (hf == 0) {
+      s_best[wave][j] = best;
+      s_idx[wave][j] = bidx;
+    }
+    __syncthreads();
+    if (part != 0) return;
+#pragma unroll
+    for (int q = 1; q < SPLIT; ++q) {
+      const float ob = s_best[wave + q][j];
+      const int oi = s_idx[wave + q][j];
+      if (ob < best || (ob == best && oi < bidx)) {
+        best = ob;
+        bidx = oi;
+      }
+    }
+  }
+  if (hf == 0 && row < a.N) a.indices[h * a.N + row] = bidx;
+}
+
+// The split with the least estimated time: rounds of 256 one-per-CU blocks,
+// each its share of the eight chunks plus about a tenth of the whole search
+// for its staging: [8,N,128] with N = 1,500 takes 16 waves'-worth of chunks in
+// parallel at SPLIT 4 where SPLIT 1 would leave 200 CUs idle.
+static int nearest_split(int64_t H, int64_t N) {
+  int best = 1;
+  double least = 0.0;
+  for (int split = 1; split <= 8; split *= 2) {
+    const double rounds = (double)ceil_div(H * ceil_div(N, (int64_t)(256 / split)), 256);
+    const double t = rounds * (1.0 / split + 0.1);
+    if (split == 1 || t < least) {
+      best = split;
+      least = t;
+    }
+  }
+  return best;
+}
+
+template <int SPLIT>
+static int launch_nearest_mfma(const NearestArgs& a, hipStream_t stream) {
+  const dim3 grid((uint32_t)ceil_div(a.N, (int64_t)(256 / SPLIT)), (uint32_t)a.H);
+  hipLaunchKernelGGL(nearest_mfma_kernel<SPLIT>, grid, dim3(kNmThreads), kNmLdsBytes, stream, a);
+  JKV_CHECK_LAUNCH();
+  return JKV_OK;
+}
 
 // The M nearest codewords of every row, nearest first (equal distances in
 // index order), optionally skipping one index per row (`excluded`, [H][N]):
@@ -312,6 +496,17 @@ extern "C" int jkv_nearest_f32(const float* states, int64_t H, int64_t N, int64_
   if (N == 0) return JKV_OK;
   JKV_CHECK_ARG(states && tables && indices, "null buffer");
   NearestArgs a = {states, tables, indices, H, N, D, K};
+  // whole heads against 8-bit stages, 16-byte rows: the matrix kernel (its
+  // grid counts 512-thread blocks of 32 rows at least)
+  if (D == 128 && K <= kNmCodes && (((uintptr_t)states | (uintptr_t)tables) % 16) == 0 &&
+      ceil_div(N, (int64_t)32) * kNmThreads < ((int64_t)1 << 32)) {
+    switch (nearest_split(H, N)) {
+      case 1: return launch_nearest_mfma<1>(a, stream);
+      case 2: return launch_nearest_mfma<2>(a, stream);
+      case 4: return launch_nearest_mfma<4>(a, stream);
+      default: return launch_nearest_mfma<8>(a, stream);
+    }
+  }
   dim3 grid((uint32_t)ceil_div(N, (int64_t)kNrRows), (uint32_t)H);
   hipLaunchKernelGGL(nearest_f32_kernel, grid, dim3(256), 0, stream, a);
   JKV_CHECK_LAUNCH();

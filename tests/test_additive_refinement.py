@@ -204,6 +204,34 @@ def test_block_refinement_argument_errors(kwargs, match):
         jkv.multi_exit_additive_block_refinement(states, tables, init, **kwargs)
 
 
+# the matrix kernel's four wave splits (8 down to 1 waves per 32 rows), ragged
+# row tiles and codeword chunks; 32-bit sums: a differing index must be a
+# near-tie (the 1e-4 that the difference of two 128-term fp32 sums allows)
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,rows,clusters", [
+    (1, 1, 1), (2, 33, 37), (8, 1500, 256), (8, 3001, 250), (8, 8192, 256), (3, 300, 32)])
+def test_nearest_f32_matrix_kernel(device, heads, rows, clusters):
+    print(f"nearest (matrix kernel) H={heads} N={rows} K={clusters}", flush=True)
+    gen = torch.Generator().manual_seed(rows + clusters)
+    x = torch.randn(heads, rows, 128, generator=gen)
+    c = torch.randn(heads, clusters, 128, generator=gen)
+    c[:, clusters // 2] = c[:, 0]           # equal words in different chunks or lanes: the first one is taken
+    x[:, 0] = c[:, 0]
+    got = _ops.nearest_f32(x.to(device), c.to(device)).cpu()
+    assert (got[:, 0] == 0).all() and (got != clusters // 2).all() if clusters > 1 else (got == 0).all()
+    same = total = 0
+    for h in range(heads):
+        dist = (c[h].double().square().sum(-1) - 2.0 * (x[h].double() @ c[h].double().T))
+        order, want = dist.sort(dim=1, stable=True)
+        margin = torch.gather(dist, 1, got[h][:, None])[:, 0] - order[:, 0]
+        assert float(margin.max()) <= 1e-4
+        same += int((got[h] == want[:, 0]).sum())
+        total += rows
+    assert same / total >= 0.9999
+    x[0, 0, 5] = float("nan")
+    assert int(_ops.nearest_f32(x.to(device), c.to(device))[0, 0]) == 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,rows,dim,clusters,m,exclude", [(2, 500, 128, 256, 3, True), (1, 70, 9, 40, 8, False),
                                                                 (2, 64, 128, 64, 1, True)])
