@@ -50,6 +50,39 @@ struct DecodeArgs {
   uint8_t* vc_out;
 };
 
+// A workgroup's split sums: value(h, i) is element i of the kv head's query
+// head h, over waves; (mh, lh) its (max x unit in natural-exponent units,
+// sum).  They go to the combine as partials, or, when the window is one
+// split, become the output at once (the combine's result: its weight is
+// e^0) and no combine runs.  DIRECT: whether that is so, -1 to read it off
+// the splits (decode_g8_kernel has a form of its own: the test alone cost it
+// 0.3 of 36.8 us).
+template <int NQ, int THREADS, int DIRECT, typename Value>
+__device__ __forceinline__ void store_split(const DecodeArgs& a, int64_t b, int64_t kvh, int64_t split, int ntok,
+                                            const float (&mh)[NQ], const float (&lh)[NQ], float unit, Value value) {
+  if (DIRECT < 0 ? a.n_splits == 1 : DIRECT != 0) {
+    for (int idx = threadIdx.x; idx < NQ * kHeadDim; idx += THREADS) {
+      const int h = idx / kHeadDim, i = idx % kHeadDim;
+      float l = 0.f;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) l = h == q ? lh[q] : l;
+      const float v = value(h, i);
+      a.out[(b * a.QH + kvh * NQ + h) * kHeadDim + i] = (_Float16)(ntok > 0 && l > 0.f ? v / l : 0.f);
+    }
+    return;
+  }
+  for (int idx = threadIdx.x; idx < NQ * kHeadDim; idx += THREADS) {
+    const int h = idx / kHeadDim, i = idx % kHeadDim;
+    const float v = value(h, i);
+    const int64_t qh = kvh * NQ + h;
+    a.ws_o[((b * a.QH + qh) * a.n_splits + split) * kHeadDim + i] = v;
+    if (i == 0) {
+      float* ml = a.ws_ml + ((b * a.QH + qh) * a.n_splits + split) * 2;
+      ml[0] = ntok > 0 ? mh[h] * unit : -__builtin_inff();
+      ml[1] = ntok > 0 ? lh[h] : 0.f;
+    }
+  }
+}
 
 // fp16 words of dims [8*c8, 8*c8+8) of one token: fp16(sum_s fp32(word_s)).
 // The sum of two fp16 words is exact in fp32 or too small to move the fp16
@@ -525,17 +558,9 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
     }
   }
   __syncthreads();
-  for (int idx = tid; idx < NQ * kHeadDim; idx += blockDim.x) {
-    const int h = idx / kHeadDim, i = idx % kHeadDim;
-    const float v = o_red[0][h][i] + o_red[1][h][i] + o_red[2][h][i] + o_red[3][h][i];
-    const int64_t qh = kvh * NQ + h;
-    a.ws_o[((b * a.QH + qh) * a.n_splits + split) * kHeadDim + i] = v;
-    if (i == 0) {
-      float* ml = a.ws_ml + ((b * a.QH + qh) * a.n_splits + split) * 2;
-      ml[0] = ntok > 0 ? mh[h] : -__builtin_inff();
-      ml[1] = ntok > 0 ? lh[h] : 0.f;
-    }
-  }
+  store_split<NQ, 256, -1>(a, b, kvh, split, ntok, mh, lh, 1.f, [&](int h, int i) {
+    return o_red[0][h][i] + o_red[1][h][i] + o_red[2][h][i] + o_red[3][h][i];
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -977,20 +1002,12 @@ __global__ __launch_bounds__(kLdsThreads) void decode_lds_kernel(DecodeArgs a) {
       for (int e = 0; e < 4; ++e) o_red[(wave * NQ + ln) * kHeadDim + 16 * dt + 4 * lg + e] = o[dt][e];
   }
   __syncthreads();
-  for (int idx = tid; idx < NQ * kHeadDim; idx += kLdsThreads) {
-    const int h = idx / kHeadDim, i = idx % kHeadDim;
+  store_split<NQ, kLdsThreads, -1>(a, b, kvh, split, ntok, mh, lh, 0.6931471805599453f, [&](int h, int i) {
     float v = 0.f;
 #pragma unroll
     for (int w = 0; w < kLdsWaves; ++w) v += o_red[(w * NQ + h) * kHeadDim + i];
-    const int64_t qh = kvh * NQ + h;
-    a.ws_o[((b * a.QH + qh) * a.n_splits + split) * kHeadDim + i] = v;
-    if (i == 0) {
-      float* ml = a.ws_ml + ((b * a.QH + qh) * a.n_splits + split) * 2;
-      // the combine works in natural-exponent units: m * ln 2
-      ml[0] = ntok > 0 ? mh[h] * 0.6931471805599453f : -__builtin_inff();
-      ml[1] = ntok > 0 ? lh[h] : 0.f;
-    }
-  }
+    return v;
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -1158,7 +1175,7 @@ __device__ __forceinline__ void encode_new_token(const half8 (&xv)[2], const hal
   }
 }
 
-template <int NQ, int S, bool APPEND>
+template <int NQ, int S, bool APPEND, int DIRECT>
 __global__ __launch_bounds__(kG8Threads) void decode_g8_kernel(DecodeArgs a) {
   extern __shared__ __align__(16) unsigned char dyn[];
   constexpr int tab_bytes = 16 * S * kG8Plane;
@@ -1514,62 +1531,84 @@ __global__ __launch_bounds__(kG8Threads) void decode_g8_kernel(DecodeArgs a) {
       for (int e = 0; e < 4; ++e) o_red[(wave * NQ + ln) * kHeadDim + 16 * dt + 4 * lg + e] = o[dt][e];
   }
   __syncthreads();
-  for (int idx = tid; idx < NQ * kHeadDim; idx += kG8Threads) {
-    const int h = idx / kHeadDim, i = idx % kHeadDim;
+  store_split<NQ, kG8Threads, DIRECT>(a, b, kvh, split, ntok, mh, lh, 0.6931471805599453f, [&](int h, int i) {
     float v = 0.f;
 #pragma unroll
     for (int w = 0; w < kG8Waves; ++w) v += o_red[(w * NQ + h) * kHeadDim + i];
-    const int64_t qh = kvh * NQ + h;
-    a.ws_o[((b * a.QH + qh) * a.n_splits + split) * kHeadDim + i] = v;
-    if (i == 0) {
-      float* ml = a.ws_ml + ((b * a.QH + qh) * a.n_splits + split) * 2;
-      ml[0] = ntok > 0 ? mh[h] * 0.6931471805599453f : -__builtin_inff();
-      ml[1] = ntok > 0 ? lh[h] : 0.f;
-    }
-  }
+    return v;
+  });
 }
 
-// out[b,qh,:] = sum_s o_s e^{m_s-M} / sum_s l_s e^{m_s-M}
+// out[b,qh,:] = sum_s o_s e^{m_s-M} / sum_s l_s e^{m_s-M}, summed in split
+// order.  Latency-bound (a few hundred bytes per block): up to N splits have
+// every (max, sum) and output element in flight together; more go 16 at a
+// time after a first pass for the maximum.
+template <int N>
+__device__ __forceinline__ void combine_few(const DecodeArgs& a, int64_t bq, int i) {
+  const float* ml = a.ws_ml + bq * a.n_splits * 2;
+  const float* op = a.ws_o + bq * a.n_splits * kHeadDim + i;
+  float mv[N], lv[N], ov[N];
+#pragma unroll
+  for (int s = 0; s < N; ++s) {
+    if (s < a.n_splits) {
+      mv[s] = ml[2 * s];
+      lv[s] = ml[2 * s + 1];
+      ov[s] = op[s * kHeadDim];
+    }
+  }
+  float M = -__builtin_inff();
+#pragma unroll
+  for (int s = 0; s < N; ++s)
+    if (s < a.n_splits) M = fmaxf(M, mv[s]);
+  float Lsum = 0.f, acc = 0.f;
+#pragma unroll
+  for (int s = 0; s < N; ++s) {
+    if (s >= a.n_splits || mv[s] == -__builtin_inff()) continue;
+    const float w = __expf(mv[s] - M);
+    Lsum += lv[s] * w;
+    acc += ov[s] * w;
+  }
+  a.out[bq * kHeadDim + i] = (_Float16)(Lsum > 0.f ? acc / Lsum : 0.f);
+}
+
+// up to four splits: a kernel of its own (20 registers and a fifth of the
+// code: 0.2 us less per call)
+__global__ __launch_bounds__(128) void decode_combine4_kernel(DecodeArgs a) {
+  combine_few<4>(a, blockIdx.x, threadIdx.x);
+}
+
 __global__ __launch_bounds__(128) void decode_combine_kernel(DecodeArgs a) {
   const int64_t bq = blockIdx.x;  // b*QH + qh
   const int i = threadIdx.x;
+  if (a.n_splits <= 8) return combine_few<8>(a, bq, i);
+  if (a.n_splits <= 16) return combine_few<16>(a, bq, i);
   const float* ml = a.ws_ml + bq * a.n_splits * 2;
-  constexpr int kFew = 4;
-  if (a.n_splits <= kFew) {
-    // every split's (max, sum) and output element in flight together
-    float mv[kFew], lv[kFew], ov[kFew];
-#pragma unroll
-    for (int s = 0; s < kFew; ++s) {
-      if (s < a.n_splits) {
-        mv[s] = ml[2 * s];
-        lv[s] = ml[2 * s + 1];
-        ov[s] = a.ws_o[(bq * a.n_splits + s) * kHeadDim + i];
-      }
-    }
-    float M = -__builtin_inff();
-#pragma unroll
-    for (int s = 0; s < kFew; ++s)
-      if (s < a.n_splits) M = fmaxf(M, mv[s]);
-    float Lsum = 0.f, acc = 0.f;
-#pragma unroll
-    for (int s = 0; s < kFew; ++s) {
-      if (s >= a.n_splits || mv[s] == -__builtin_inff()) continue;
-      const float w = __expf(mv[s] - M);
-      Lsum += lv[s] * w;
-      acc += ov[s] * w;
-    }
-    a.out[bq * kHeadDim + i] = (_Float16)(Lsum > 0.f ? acc / Lsum : 0.f);
-    return;
-  }
+  const float* op = a.ws_o + bq * a.n_splits * kHeadDim + i;
   float M = -__builtin_inff();
-  for (int s = 0; s < a.n_splits; ++s) M = fmaxf(M, ml[2 * s]);
+  for (int s0 = 0; s0 < a.n_splits; s0 += 16) {
+    float mv[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) mv[u] = ml[2 * (s0 + u < a.n_splits ? s0 + u : s0)];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) M = fmaxf(M, mv[u]);
+  }
   float Lsum = 0.f, acc = 0.f;
-  for (int s = 0; s < a.n_splits; ++s) {
-    const float m = ml[2 * s];
-    if (m == -__builtin_inff()) continue;
-    const float w = __expf(m - M);
-    Lsum += ml[2 * s + 1] * w;
-    acc += a.ws_o[(bq * a.n_splits + s) * kHeadDim + i] * w;
+  for (int s0 = 0; s0 < a.n_splits; s0 += 16) {
+    float mv[16], lv[16], ov[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int at = s0 + u < a.n_splits ? s0 + u : s0;
+      mv[u] = ml[2 * at];
+      lv[u] = ml[2 * at + 1];
+      ov[u] = op[(int64_t)at * kHeadDim];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      if (s0 + u >= a.n_splits || mv[u] == -__builtin_inff()) continue;
+      const float w = __expf(mv[u] - M);
+      Lsum += lv[u] * w;
+      acc += ov[u] * w;
+    }
   }
   a.out[bq * kHeadDim + i] = (_Float16)(Lsum > 0.f ? acc / Lsum : 0.f);
 }
@@ -1598,13 +1637,41 @@ static int64_t lds_bytes(int64_t S, int64_t nq) {
          kLdsWaves * kStgRows * kStgStride * 2 + 2 * kLdsWaves * nq * 4;
 }
 
+// Tokens per split of an LDS-table kernel over `window` tokens of n = B * KVH
+// (batch row, kv head) pairs: whole 256-token chunks, up to eight.  A
+// workgroup has a CU to itself, so the splits are those with the least
+// rounds of 256 workgroups x (chunks + 2.5), plus 1 where a combine follows:
+// in units of a chunk's ~2.5 us, what the two table copies, softmax and
+// epilogue take and what the combine's launch takes.  Measured (two stages,
+// 8 kv heads, us per call, longest splits against the chosen ones): 1 row of
+// 1,536 tokens 24.4 -> 14.3, of 4,096 31.8 -> 14.7; 8 rows of 4,096 33.7 ->
+// 24.0; 16 rows of 1,536 25.8 -> 21.1; 20 rows of 4,096 64 -> 55; 16 rows of
+// 4,096 keep two splits each (35.6; four take 44).  Never more than 512
+// workgroups unless the longest splits need them: the partials then stay
+// within those of the longest splits or 2 MB, whatever holds them.
+static int64_t lds_table_split(int64_t n, int64_t window) {
+  const int64_t chunks = ceil_div(window, kLdsChunk);
+  const int64_t longest = chunks < 8 ? chunks : 8;
+  int64_t best = longest;
+  double least = 0.0;
+  for (int64_t c = longest; c >= 1; --c) {
+    const int64_t blocks = n * ceil_div(chunks, c);
+    if (c < longest && blocks > 512) break;
+    const double t = (double)ceil_div(blocks, 256) * ((double)c + 2.5) + (c < chunks ? 1.0 : 0.0);
+    if (c == longest || t < least) {
+      least = t;
+      best = c;
+    }
+  }
+  return best * kLdsChunk;
+}
+
 // Tokens per split of decode_lds_kernel (0: the geometry does not fit).
-static int64_t lds_split_tokens(int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window) {
+static int64_t lds_split_tokens(int64_t n, int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window) {
   if (S > 2 || K != kLdsK || G * S > kLdsCodeBytes || (G * S) % 16 != 0) return 0;
   if (lds_bytes(S, nq) > kMaxLds) return 0;
   if (kLdsWaves * nq * kHeadDim * 4 > kHeadDim * S * K * 2) return 0;  // partials fit the table area
-  const int64_t w = ceil_div(window, kLdsChunk) * kLdsChunk;
-  return w < kLdsMaxSplit ? w : kLdsMaxSplit;
+  return lds_table_split(n, window);
 }
 
 // Dynamic LDS of decode_g8_kernel: tables, one chunk of code records, the
@@ -1614,25 +1681,25 @@ static int64_t g8_lds_bytes(int64_t S, int64_t nq) {
 }
 
 // Tokens per split of decode_g8_kernel (0: the geometry does not fit).
-static int64_t g8_split_tokens(int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window) {
+static int64_t g8_split_tokens(int64_t n, int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window) {
   if (G != 16 || S < 1 || S > 2 || K != kLdsK) return 0;
   if (g8_lds_bytes(S, nq) > kMaxLds) return 0;
   if (kG8Waves * nq * kHeadDim * 4 > 16 * S * kG8Plane) return 0;  // partials fit the table area
-  const int64_t w = ceil_div(window, kG8Chunk) * kG8Chunk;
-  return w < kG8MaxSplit ? w : kG8MaxSplit;
+  return lds_table_split(n, window);
 }
 
 // Tokens per split of the kernel launch_decode picks for a packed-code
-// geometry (the LDS-table kernels take up to 2048-token splits, the L2
-// split kernel kSplitTokens), so callers can size the partials exactly.
-static int64_t packed_split_tokens(int64_t G, int64_t d, int64_t S, int64_t K, int64_t nq, int64_t window,
-                                   bool lds_ok) {
+// geometry and n (batch row, kv head) pairs (the LDS-table kernels take up
+// to 2048-token splits, the L2 split kernel kSplitTokens), so callers can
+// size the partials exactly.
+static int64_t packed_split_tokens(int64_t n, int64_t G, int64_t d, int64_t S, int64_t K, int64_t nq,
+                                   int64_t window, bool lds_ok) {
   if (lds_ok && d == 8) {
-    const int64_t g8 = g8_split_tokens(G, S, K, nq, window);
+    const int64_t g8 = g8_split_tokens(n, G, S, K, nq, window);
     if (g8 > 0) return g8;
   }
   if (lds_ok && (d == 8 || d == 4)) {
-    const int64_t lds = lds_split_tokens(G, S, K, nq, window);
+    const int64_t lds = lds_split_tokens(n, G, S, K, nq, window);
     if (lds > 0) return lds;
   }
   return kSplitTokens;
@@ -1641,7 +1708,7 @@ static int64_t packed_split_tokens(int64_t G, int64_t d, int64_t S, int64_t K, i
 // Bytes of split partials ([B,QH,n_splits] x (128 + 2) fp32) that launch.
 static int64_t packed_partial_bytes(int64_t B, int64_t QH, int64_t G, int64_t d, int64_t S, int64_t K, int64_t nq,
                                     int64_t window, bool lds_ok) {
-  const int64_t ns = ceil_div(window, packed_split_tokens(G, d, S, K, nq, window, lds_ok));
+  const int64_t ns = ceil_div(window, packed_split_tokens(B * (QH / nq), G, d, S, K, nq, window, lds_ok));
   return B * QH * ns * (kHeadDim + 2) * (int64_t)sizeof(float);
 }
 
@@ -1672,8 +1739,8 @@ static void launch_split(const DecodeArgs& a, hipStream_t stream) {
 
 template <int D, int NQ>
 static int launch_decode(DecodeArgs a, bool lds_ok, hipStream_t stream, bool append = false) {
-  const int64_t split = lds_ok && D != 128 && D != 0 ? lds_split_tokens(a.G, a.S, a.K, NQ, a.window) : 0;
-  const int64_t g8_split = lds_ok && D == 8 ? g8_split_tokens(a.G, a.S, a.K, NQ, a.window) : 0;
+  const int64_t split = lds_ok && D != 128 && D != 0 ? lds_split_tokens(a.B * a.KVH, a.G, a.S, a.K, NQ, a.window) : 0;
+  const int64_t g8_split = lds_ok && D == 8 ? g8_split_tokens(a.B * a.KVH, a.G, a.S, a.K, NQ, a.window) : 0;
   if constexpr (D == 128 || D == 0) {
     launch_split<D, NQ>(a, stream);
   } else if (D == 8 && g8_split > 0) {
@@ -1682,19 +1749,22 @@ static int launch_decode(DecodeArgs a, bool lds_ok, hipStream_t stream, bool app
     a.ws_ml = a.ws_o + a.B * a.QH * a.n_splits * kHeadDim;
     const size_t lds = (size_t)g8_lds_bytes(a.S, NQ);
     const dim3 grid((uint32_t)(a.KVH * a.B * a.n_splits));
+    const bool direct = a.n_splits == 1;
+#define JKV_G8(SS, AP, DI) hipLaunchKernelGGL((decode_g8_kernel<NQ, SS, AP, DI>), grid, dim3(kG8Threads), lds, stream, a)
     if (a.S == 2) {
       if (append) {
-        hipLaunchKernelGGL((decode_g8_kernel<NQ, 2, true>), grid, dim3(kG8Threads), lds, stream, a);
+        if (direct) JKV_G8(2, true, 1); else JKV_G8(2, true, 0);
       } else {
-        hipLaunchKernelGGL((decode_g8_kernel<NQ, 2, false>), grid, dim3(kG8Threads), lds, stream, a);
+        if (direct) JKV_G8(2, false, 1); else JKV_G8(2, false, 0);
       }
     } else {
       if (append) {
-        hipLaunchKernelGGL((decode_g8_kernel<NQ, 1, true>), grid, dim3(kG8Threads), lds, stream, a);
+        if (direct) JKV_G8(1, true, 1); else JKV_G8(1, true, 0);
       } else {
-        hipLaunchKernelGGL((decode_g8_kernel<NQ, 1, false>), grid, dim3(kG8Threads), lds, stream, a);
+        if (direct) JKV_G8(1, false, 1); else JKV_G8(1, false, 0);
       }
     }
+#undef JKV_G8
   } else if (append) {
     return set_error(JKV_ENOTSUP, "decode with append needs group dim 8, 16 groups, 1-2 stages, 256 codewords "
                                   "and 16-byte aligned codes and tables");
@@ -1713,8 +1783,13 @@ static int launch_decode(DecodeArgs a, bool lds_ok, hipStream_t stream, bool app
     launch_split<D, NQ>(a, stream);
   }
   JKV_CHECK_LAUNCH();
-  hipLaunchKernelGGL(decode_combine_kernel, dim3((uint32_t)(a.B * a.QH)), dim3(kHeadDim), 0,
-                     stream, a);
+  if (a.n_splits == 1) return JKV_OK;  // written by the split itself
+  const dim3 grid((uint32_t)(a.B * a.QH));
+  if (a.n_splits <= 4) {
+    hipLaunchKernelGGL(decode_combine4_kernel, grid, dim3(kHeadDim), 0, stream, a);
+  } else {
+    hipLaunchKernelGGL(decode_combine_kernel, grid, dim3(kHeadDim), 0, stream, a);
+  }
   JKV_CHECK_LAUNCH();
   return JKV_OK;
 }
@@ -1883,8 +1958,9 @@ int jkv_decode_attention_noalloc(const void* q, int64_t q_stride_b, int64_t q_st
                                  jkv_stream_t stream) {
   using namespace jkv;
   JKV_CHECK_ARG(B >= 0 && QH > 0 && KVH > 0 && QH % KVH == 0 && window > 0, "invalid head geometry");
-  // the partials of the kernel this call will run: 2048-token splits on the
-  // LDS-table kernels (group dims 4 and 8), 256-token splits otherwise
+  // the partials of the kernel this call will run: splits of up to 2048
+  // tokens on the LDS-table kernels (group dims 4 and 8), 256-token ones
+  // otherwise
   const bool lds_ok = packed_lds_ok(k_codes, v_codes, code_stride_b, code_stride_h, k_tables, v_tables);
   const int64_t need = packed_partial_bytes(B, QH, G, d, S, K, QH / KVH, window, lds_ok);
   JKV_CHECK_ARG(need <= kNoAllocScratchBytes,

@@ -63,6 +63,33 @@ def test_decode_matches_oracle(device, batch, qh, kvh, groups, stages, d, length
     assert err <= ATOL, f"max abs error {err}"
 
 
+# the split rule's choices on the table kernels (d = 8 and 4): one split that
+# writes its output itself (one token, whole chunks, a chunk's edge), one- to
+# three-chunk splits, a partial last split, and combines of up to 4, 8, 16 and
+# more splits; rows shorter than the longest leave empty splits
+@pytest.mark.parametrize("batch,qh,kvh,groups,stages,d,lengths,window", [
+    (1, 32, 8, 16, 2, 8, (1,), 4096),
+    (2, 32, 8, 16, 2, 8, (256, 3), 4096),
+    (1, 32, 8, 16, 2, 8, (257,), 4096),
+    (1, 8, 2, 16, 2, 8, (1501,), 4096),
+    (6, 32, 8, 16, 2, 8, (1536, 1, 700, 1280, 1281, 900), 4096),
+    (20, 8, 8, 16, 1, 8, (1400,) * 20, 4096),
+    (1, 32, 8, 16, 1, 8, (8192,), 8192),
+    (1, 16, 8, 32, 1, 4, (1300,), 4096),
+    (1, 32, 8, 32, 1, 4, (90,), 4096),
+])
+def test_decode_split_rule(device, batch, qh, kvh, groups, stages, d, lengths, window):
+    print(f"decode splits B={batch} QH={qh} KVH={kvh} G={groups} S={stages} lengths={lengths[:3]}", flush=True)
+    q, kc, vc, kt, vt = _case(lengths[0] + qh, batch, qh, kvh, groups, stages, d, lengths[0], window)
+    out = jkv.decode_attention(q.to(device), kc.to(device), vc.to(device), kt.half().to(device), vt.half().to(device),
+                               torch.tensor(lengths, dtype=torch.int32, device=device), window=window,
+                               max_length=max(lengths))
+    for b in sorted({0, batch // 2, batch - 1}):
+        e = _expect(q[b : b + 1], kc[b : b + 1], vc[b : b + 1], kt, vt, lengths[b], window, window)
+        err = float((out[b : b + 1].cpu().float() - e.float()).abs().max())
+        assert err <= ATOL, f"row {b} length {lengths[b]}: {err}"
+
+
 @pytest.mark.parametrize("batch,qh,kvh,stages,lengths,window,cap", [
     (2, 32, 8, 2, (4096, 4096), 4096, 4096),    # config 4 geometry: the new token closes split 2
     (3, 8, 2, 2, (1, 257, 5000), 4096, 4096),   # first token; chunk 1's first key; ring wrap
