@@ -130,107 +130,140 @@ __global__ __launch_bounds__(256) void full_tables_many_kernel(FullPrepMany m) {
   full_tables_block(m.masters[job], t.tab16, t.nhalf, t.ncmax, blockIdx.x - job * per);
 }
 
+// The whitener's products run on v_mfma_f32_32x32x2_f32, which adds its two
+// fp32 products one after the other: a chain over e = 0, 1, 2, ... gives the
+// bits of the fma chain acc = fma(a[e], b[e], acc) (lane half h takes e =
+// 2m + h of step m).
+
 // M = W^T W per problem, and M's rows as hi/lo fp16 planes in the order the
 // mat-vec u = M x leaves in the search's B-operand layout: plane row 16c + i
 // holds M row 32(c/2) + 8(i/4) + 4(c%2) + i%4, so output chunk c, lane group
 // lg, element v of the mat-vec is dim 32(c/2) + 8lg + 4(c%2) + v (chunk c/2,
 // word 4(c%2) + v of the lane's B operand).  Hi plane rows 0..127, lo plane
-// rows 128..255.  One 256-thread block per (problem, 8 plane rows), W in LDS;
-// each block writes the M rows its plane rows come from.
-__global__ __launch_bounds__(256) void full_whiten_m_kernel(const float* __restrict__ whiteners,
-                                                            float* __restrict__ m_out,
-                                                            _Float16* __restrict__ perm) {
-  extern __shared__ __align__(16) float wsh[];  // W [e][i]
-  const int64_t p = blockIdx.x >> 4;
-  const int r0 = (blockIdx.x & 15) * 8;
-  const float* w = whiteners + p * kFullD * kFullD;
-  for (int idx = threadIdx.x; idx < kFullD * kFullD / 4; idx += 256)
-    *(float4*)(wsh + 4 * idx) = *(const float4*)(w + 4 * idx);
-  __syncthreads();
+// rows 128..255.  One 256-thread block per (problem, 32 M rows), a 32-column
+// tile per wave.
+__device__ __forceinline__ void full_whiten_m_block(const float* __restrict__ whiteners, float* __restrict__ m_out,
+                                                    _Float16* __restrict__ perm, uint32_t bid) {
+  const int64_t p = bid >> 2;
+  const int lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
+  const int i0 = 32 * (int)(bid & 3), j0 = 32 * (int)(threadIdx.x >> 6);
+  const float* w = whiteners + p * kFullD * kFullD + h * kFullD + j;
+  float16v acc = {};
+#pragma unroll 16
+  for (int m = 0; m < kFullD / 2; ++m)
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w[2 * m * kFullD + i0], w[2 * m * kFullD + j0], acc, 0, 0, 0);
   float* mp = m_out + p * kFullD * kFullD;
   _Float16* hi = perm + p * 2 * kFullD * kFullD;
   _Float16* lo = hi + kFullD * kFullD;
-  for (int idx = threadIdx.x; idx < 8 * kFullD; idx += 256) {
-    const int r = r0 + idx / kFullD, col = idx % kFullD;
-    const int c = r >> 4, i = r & 15;
-    const int src = 32 * (c >> 1) + 8 * (i >> 2) + 4 * (c & 1) + (i & 3);
-    float v = 0.f;
-    for (int e = 0; e < kFullD; ++e) v = fmaf(wsh[e * kFullD + src], wsh[e * kFullD + col], v);
-    mp[src * kFullD + col] = v;
-    const half_t h = (half_t)v;
-    hi[r * kFullD + col] = h;
-    lo[r * kFullD + col] = (half_t)(v - (float)h);
+#pragma unroll
+  for (int el = 0; el < 16; ++el) {
+    const int row = i0 + 8 * (el >> 2) + 4 * h + (el & 3), col = j0 + j;
+    const int r = 16 * (2 * (row >> 5) + ((row >> 2) & 1)) + 4 * ((row >> 3) & 3) + (row & 3);
+    const float v = acc[el];
+    mp[row * kFullD + col] = v;
+    const half_t vh = (half_t)v;
+    hi[r * kFullD + col] = vh;
+    lo[r * kFullD + col] = (half_t)(v - (float)vh);
   }
 }
 
-// M c for every codeword (fp32, tiled like selector_tables128_kernel: one
-// 256-thread block per (problem, stage, 64 codewords), M^T = M in LDS and the
-// fp16 codewords beside it, so two blocks share a CU), the
-// selector norms |W c|^2 = c . M c as the -|c'|^2/2 plane, and four partial
-// maxima of |c'|^2 (the other twelve partial slots are zero).
+// The deployed tables and every problem's M in one launch (neither reads the
+// other): blocks below 4 P form M, the rest the tables.
+__global__ __launch_bounds__(256) void full_whiten_prep_kernel(const float* __restrict__ masters,
+                                                               _Float16* __restrict__ tab16,
+                                                               float* __restrict__ nhalf,
+                                                               float* __restrict__ ncmax_part,
+                                                               const float* __restrict__ whiteners,
+                                                               float* __restrict__ m_out, _Float16* __restrict__ perm,
+                                                               uint32_t m_blocks) {
+  if (blockIdx.x < m_blocks) {
+    full_whiten_m_block(whiteners, m_out, perm, blockIdx.x);
+  } else {
+    full_tables_block(masters, tab16, nhalf, ncmax_part, blockIdx.x - m_blocks);
+  }
+}
+
+// M c for every codeword (fp32), the selector norms |W c|^2 = c . M c as the
+// -|c'|^2/2 plane, and partial maxima of |c'|^2 (eight of the sixteen slots;
+// the others are zero).  One 256-thread block per (problem, stage, 32
+// codewords); wave w forms dims 32w..+31 of all of them, M's columns and the
+// codewords through LDS.  Bound: the fp32 matrix rate (8 us) and the 17 MB
+// of M c.  R16 at 8 heads: 47 us on VALU (a thread per 8 dims x 4 codewords,
+// both operands through LDS), 18 us here; M took 9.7 us in a launch of its
+// own and now rides with the tables (7.5 -> 10.9 us); the same bits.
 __global__ __launch_bounds__(256) void full_whiten_tables_kernel(const _Float16* __restrict__ tab16,
                                                                  const float* __restrict__ m_all,
                                                                  float* __restrict__ mc, float* __restrict__ nhalf,
                                                                  float* __restrict__ ncmax_part, int64_t S) {
-  constexpr int kKTile = 64;
-  extern __shared__ __align__(16) float sm[];
-  float* mt = sm;                                  // [e][i] = M[i][e] = M[e][i]
-  _Float16* ct = (_Float16*)(sm + kFullD * kFullD);  // [e][k], fp16 codewords (exact)
+  constexpr int kCodes = 32, kPitch = kFullD + 4;
+  __shared__ __align__(16) float mcs[kCodes * kPitch];  // M c, one row per codeword
   __shared__ float red[4];
-  const int64_t ps = blockIdx.x >> 2;
-  const int part = blockIdx.x & 3;
-  const int k0 = part * kKTile;
+  const int64_t ps = blockIdx.x >> 3;
+  const int part = blockIdx.x & 7;
+  const int k0 = part * kCodes;
   const int64_t p = ps / S;
-  const int tid = threadIdx.x;
-  const float* msrc = m_all + p * kFullD * kFullD;
-  for (int idx = tid; idx < kFullD * kFullD / 4; idx += 256)
-    *(float4*)(mt + 4 * idx) = *(const float4*)(msrc + 4 * idx);
-  const _Float16* csrc = tab16 + (ps * kFullK + k0) * kFullD;
-  for (int idx = tid; idx < kKTile * kFullD; idx += 256) {
-    const int k = idx / kFullD, e = idx % kFullD;
-    ct[e * kKTile + k] = csrc[k * kFullD + e];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int j = lane & 31, h = lane >> 5;
+  // the block's 8 KiB of codewords, rows 272 bytes apart (straight from L2
+  // each load would touch 32 lines, 19.5 against 17.9 us)
+  __shared__ __align__(16) _Float16 cs[kCodes * (kFullD + 8)];
+  {
+    const uint4* src = (const uint4*)(tab16 + (ps * kFullK + k0) * kFullD);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = tid + 256 * u;  // row i / 16, chunk i % 16
+      *(uint4*)(cs + (i >> 4) * (kFullD + 8) + 8 * (i & 15)) = src[i];
+    }
   }
   __syncthreads();
-  const int tx = tid & 15, ty = tid >> 4;
-  float acc[4][8];
+  const uint4* csrc = (const uint4*)(cs + j * (kFullD + 8));
+  const float* msrc = m_all + p * kFullD * kFullD + h * kFullD + 32 * wave + j;
+  float16v acc = {};
+#pragma unroll 8
+  for (int q = 0; q < kFullD / 8; ++q) {
+    // dims 8q..8q+7 of codeword j, of which this half takes 8q + 2u + h
+    const uint4 c = csrc[q];
+    const uint32_t cv[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
-  for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-    for (int u = 0; u < 8; ++u) acc[jj][u] = 0.f;
-  for (int e = 0; e < kFullD; ++e) {
-    const half4 c4 = *(const half4*)(ct + e * kKTile + 4 * ty);
-    const float4 m0 = *(const float4*)(mt + e * kFullD + 8 * tx);
-    const float4 m1 = *(const float4*)(mt + e * kFullD + 8 * tx + 4);
-    const float cv[4] = {(float)c4[0], (float)c4[1], (float)c4[2], (float)c4[3]};
-    const float mv[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-      for (int u = 0; u < 8; ++u) acc[jj][u] = fmaf(cv[jj], mv[u], acc[jj][u]);
+    for (int u = 0; u < 4; ++u) {
+      const half2v w = __builtin_bit_cast(half2v, cv[u]);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(msrc[(8 * q + 2 * u) * kFullD], (float)(h ? w[1] : w[0]), acc, 0, 0,
+                                                 0);
+    }
   }
-  float mx = 0.f;
+  // element el: dim 32 wave + 8 (el / 4) + 4 h + el % 4 of codeword j
+  float* dst = mc + (ps * kFullK + k0 + j) * kFullD + 32 * wave + 4 * h;
 #pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    const int k = k0 + 4 * ty + jj;
-    float* dst = mc + (ps * kFullK + k) * kFullD + 8 * tx;
-    *(float4*)dst = float4{acc[jj][0], acc[jj][1], acc[jj][2], acc[jj][3]};
-    *(float4*)(dst + 4) = float4{acc[jj][4], acc[jj][5], acc[jj][6], acc[jj][7]};
-    // |c'|^2 = c . (M c) over this thread's 8 dims, summed over the 16 tx lanes
+  for (int q = 0; q < 4; ++q) {
+    const float4 v = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    *(float4*)(dst + 8 * q) = v;
+    *(float4*)(mcs + j * kPitch + 32 * wave + 8 * q + 4 * h) = v;
+  }
+  __syncthreads();
+  // |c'|^2 = c . (M c): 16 lanes of 8 dims per codeword
+  float mx = 0.f;
+  const int tx = tid & 15;
+#pragma unroll
+  for (int r = 0; r < kCodes / 16; ++r) {
+    const int k = 16 * r + (tid >> 4);
+    const half8 c = *(const half8*)(cs + k * (kFullD + 8) + 8 * tx);
+    const float4 v0 = *(const float4*)(mcs + k * kPitch + 8 * tx);
+    const float4 v1 = *(const float4*)(mcs + k * kPitch + 8 * tx + 4);
+    const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
     float nc = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) nc = fmaf((float)ct[(8 * tx + u) * kKTile + 4 * ty + jj], acc[jj][u], nc);
+    for (int u = 0; u < 8; ++u) nc = fmaf((float)c[u], v[u], nc);
 #pragma unroll
     for (int off = 8; off >= 1; off >>= 1) nc += __shfl_xor(nc, off, 16);
-    if (tx == 0) nhalf[ps * kFullK + k] = -0.5f * nc;
+    if (tx == 0) nhalf[ps * kFullK + k0 + k] = -0.5f * nc;
     mx = fmaxf(mx, nc);
   }
 #pragma unroll
   for (int off = 32; off >= 16; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  if (lane == 0) red[wave] = mx;
   __syncthreads();
-  if (tid < 4) {
-    ncmax_part[ps * 16 + 4 * part + tid] = tid == 0 ? fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) : 0.f;
-  }
+  if (tid < 2)
+    ncmax_part[ps * 16 + 2 * part + tid] = tid == 0 ? fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])) : 0.f;
 }
 
 struct FullArgs {
@@ -692,11 +725,7 @@ int launch_full(const EncodeArgs& a, void* workspace, hipStream_t stream) {
   _Float16* tab16 = (_Float16*)ws;
   float* nhalf = (float*)(ws + P * S * (int64_t)kFullTabBytes);
   float* ncmax = (float*)(ws + P * S * ((int64_t)kFullTabBytes + kFullK * 4));
-  JKV_CHECK_ARG(P * S * 16 < ((int64_t)1 << 31), "too many (problem, stage) tables");
-  hipLaunchKernelGGL(full_tables_kernel, dim3((uint32_t)(P * S * 16)), dim3(256), 0, stream, a.tables,
-                     tab16, nhalf, ncmax);
-  JKV_CHECK_LAUNCH();
-
+  JKV_CHECK_ARG(P * S * 16 + P * 4 < ((int64_t)1 << 31), "too many (problem, stage) tables");
   FullArgs f = {};
   f.e = a;
   f.tab16 = tab16;
@@ -707,16 +736,19 @@ int launch_full(const EncodeArgs& a, void* workspace, hipStream_t stream) {
     float* mc = (float*)rest;
     float* m_all = (float*)(rest + P * S * kWhMcBytes);
     _Float16* mperm = (_Float16*)(rest + P * S * kWhMcBytes + P * kWhMBytes);
-    hipLaunchKernelGGL(full_whiten_m_kernel, dim3((uint32_t)(P * 16)), dim3(256), kFullD * kFullD * sizeof(float),
-                       stream, a.whiteners, m_all, mperm);
+    hipLaunchKernelGGL(full_whiten_prep_kernel, dim3((uint32_t)(P * 4 + P * S * 16)), dim3(256), 0, stream, a.tables,
+                       tab16, nhalf, ncmax, a.whiteners, m_all, mperm, (uint32_t)(P * 4));
     JKV_CHECK_LAUNCH();
     // the whitened norms overwrite the raw ones in the plane and the maxima
-    hipLaunchKernelGGL(full_whiten_tables_kernel, dim3((uint32_t)(P * S * 4)), dim3(256),
-                       kFullD * kFullD * sizeof(float) + kFullD * 64 * sizeof(_Float16), stream, tab16, m_all, mc,
+    hipLaunchKernelGGL(full_whiten_tables_kernel, dim3((uint32_t)(P * S * 8)), dim3(256), 0, stream, tab16, m_all, mc,
                        nhalf, ncmax, S);
     JKV_CHECK_LAUNCH();
     f.mc = mc;
     f.mperm = mperm;
+  } else {
+    hipLaunchKernelGGL(full_tables_kernel, dim3((uint32_t)(P * S * 16)), dim3(256), 0, stream, a.tables, tab16, nhalf,
+                       ncmax);
+    JKV_CHECK_LAUNCH();
   }
   // waves per workgroup: 8 (128 rows) unless that leaves the chip short of
   // workgroups; each workgroup holds most of a CU's LDS
