@@ -8,6 +8,7 @@ missing, and every operator checks that its tensors live on a HIP device.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from pathlib import Path
 
@@ -178,38 +179,49 @@ def check(code: int) -> None:
 
 
 def stream_handle(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    """The raw handle of PyTorch's current stream on ``device`` (without the
+    Stream object that ``torch.cuda.current_stream`` builds around it)."""
+
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
     """All tensors must share one HIP device; returns it."""
 
-    device = None
+    index = None
     for tensor in tensors:
         if tensor is None:
             continue
-        if tensor.device.type != "cuda":
+        if not tensor.is_cuda:
             raise ValueError(
                 "jointkv_amd runs on the MI355X (HIP) device only; got a tensor on "
                 f"{tensor.device}"
             )
-        if device is None:
-            device = tensor.device
-        elif tensor.device != device:
+        if index is None:
+            first, index = tensor, tensor.get_device()
+        elif tensor.get_device() != index:
             raise ValueError("tensors live on different devices")
-    if device is None:
+    if index is None:
         raise ValueError("no device tensor given")
-    return device
+    return first.device
+
+
+@functools.lru_cache(maxsize=512)
+def workspace_bytes(query: str, *sizes: int) -> int:
+    """A ``*_workspace_bytes`` query of the library: a function of its sizes
+    alone, so each geometry crosses into C once."""
+
+    return int(getattr(load(), query)(*sizes))
+
+
+_DTYPE_CODES = {torch.float16: JKV_F16, torch.bfloat16: JKV_BF16, torch.float32: JKV_F32}
 
 
 def dtype_code(dtype: torch.dtype) -> int:
-    if dtype == torch.float16:
-        return JKV_F16
-    if dtype == torch.bfloat16:
-        return JKV_BF16
-    if dtype == torch.float32:
-        return JKV_F32
-    raise ValueError(f"unsupported dtype {dtype}")
+    code = _DTYPE_CODES.get(dtype)
+    if code is None:
+        raise ValueError(f"unsupported dtype {dtype}")
+    return code
 
 
 def ptr(tensor: torch.Tensor | None) -> int | None:

@@ -16,9 +16,11 @@ from . import _lib
 
 
 def _encode_states_strides(states: torch.Tensor) -> tuple[torch.Tensor, tuple[int, int, int]]:
-    if states.stride(-1) != 1:
+    strides = states.stride()
+    if strides[-1] != 1:
         states = states.contiguous()
-    return states, (states.stride(0), states.stride(1), states.stride(2))
+        strides = states.stride()
+    return states, strides[:3]
 
 
 def rvq_encode(
@@ -40,8 +42,8 @@ def rvq_encode(
     """
 
     device = _lib.require_device(states, tables, whiteners)
-    batch, heads, tokens, dim = map(int, states.shape)
-    problems, stages, clusters, d = map(int, tables.shape)
+    batch, heads, tokens, dim = states.shape
+    problems, stages, clusters, d = tables.shape
     if dim != groups * group_dim or d != group_dim or problems != heads * groups:
         raise ValueError("state and table geometry differs")
     if tables.dtype != torch.float32 or not tables.is_contiguous():
@@ -51,27 +53,26 @@ def rvq_encode(
     lib = _lib.load()
     states, (sb, sh, st) = _encode_states_strides(states)
     if codes_out is None:
-        codes = torch.empty((batch, heads, tokens, groups, stages), dtype=torch.uint8, device=device)
+        codes = states.new_empty((batch, heads, tokens, groups, stages), dtype=torch.uint8)
     else:
         codes = codes_out
         if (codes.dtype != torch.uint8 or tuple(codes.shape) != (batch, heads, tokens, groups, stages)
                 or codes.stride(-1) != 1 or codes.stride(-2) != stages or codes.device != device):
             raise ValueError("codes_out must be uint8 [B,H,T,G,S] with a contiguous (G,S) block")
-    recon = [torch.empty((batch, heads, tokens, dim), dtype=states.dtype, device=device) for _ in exits]
+    recon = [states.new_empty((batch, heads, tokens, dim)) for _ in exits]
     if whiteners is not None:
         whiteners = whiteners.detach().float().contiguous()
         if tuple(whiteners.shape) != (problems, d, d):
             raise ValueError("assignment whitener has invalid geometry")
-    ws_bytes = int(lib.jkv_rvq_encode_workspace_bytes(heads, groups, stages, clusters, d, int(whiteners is not None)))
-    workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device) if ws_bytes else None
+    ws_bytes = _lib.workspace_bytes("jkv_rvq_encode_workspace_bytes", heads, groups, stages, clusters, d,
+                                    int(whiteners is not None))
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
     depth_arr = _lib.ptr_array(ctypes.c_int32, [int(e) for e in exits])
     recon_arr = _lib.ptr_array(ctypes.c_void_p, [r.data_ptr() for r in recon])
     code = lib.jkv_rvq_encode(
         states.data_ptr(), _lib.dtype_code(states.dtype), batch, heads, tokens, groups, d,
         sb, sh, st, tables.data_ptr(), stages, clusters,
-        _lib.ptr(whiteners), codes.data_ptr(),
-        codes.stride(0), codes.stride(1), codes.stride(2),
-        len(exits), depth_arr, recon_arr,
+        _lib.ptr(whiteners), codes.data_ptr(), *codes.stride()[:3], len(exits), depth_arr, recon_arr,
         _lib.ptr(workspace), ws_bytes, _lib.stream_handle(device),
     )
     _lib.check(code)
@@ -97,8 +98,8 @@ def rvq_encode_kv(
     device = _lib.require_device(key, value, key_tables, value_tables)
     if key.shape != value.shape or key.dtype != value.dtype or key_tables.shape != value_tables.shape:
         raise ValueError("K and V must share their geometry")
-    batch, heads, tokens, dim = map(int, key.shape)
-    problems, stages, clusters, d = map(int, key_tables.shape)
+    batch, heads, tokens, dim = key.shape
+    problems, stages, clusters, d = key_tables.shape
     if dim != groups * group_dim or d != group_dim or problems != heads * groups:
         raise ValueError("state and table geometry differs")
     for t in (key_tables, value_tables):
@@ -112,25 +113,27 @@ def rvq_encode_kv(
         key, strides = _encode_states_strides(key.contiguous())
         value, vstrides = _encode_states_strides(value.contiguous())
     codes = []
+    shape = (batch, heads, tokens, groups, stages)
     for out in (key_codes_out, value_codes_out):
         if out is None:
-            out = torch.empty((batch, heads, tokens, groups, stages), dtype=torch.uint8, device=device)
-        elif (out.dtype != torch.uint8 or tuple(out.shape) != (batch, heads, tokens, groups, stages)
+            out = key.new_empty(shape, dtype=torch.uint8)
+        elif (out.dtype != torch.uint8 or tuple(out.shape) != shape
               or out.stride(-1) != 1 or out.stride(-2) != stages or out.device != device):
             raise ValueError("codes_out must be uint8 [B,H,T,G,S] with a contiguous (G,S) block")
         codes.append(out)
-    if codes[0].stride()[:3] != codes[1].stride()[:3]:
+    code_strides = codes[0].stride()[:3]
+    if code_strides != codes[1].stride()[:3]:
         raise ValueError("K and V code outputs must share their strides")
-    recon_k = [torch.empty((batch, heads, tokens, dim), dtype=key.dtype, device=device) for _ in exits]
-    recon_v = [torch.empty((batch, heads, tokens, dim), dtype=key.dtype, device=device) for _ in exits]
+    recon_k = [key.new_empty((batch, heads, tokens, dim)) for _ in exits]
+    recon_v = [key.new_empty((batch, heads, tokens, dim)) for _ in exits]
     lib = _lib.load()
-    ws_bytes = int(lib.jkv_rvq_encode_workspace_bytes(heads, groups, stages, clusters, d, 0))
+    ws_bytes = _lib.workspace_bytes("jkv_rvq_encode_workspace_bytes", heads, groups, stages, clusters, d, 0)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device) if ws_bytes else None
     depth_arr = _lib.ptr_array(ctypes.c_int32, [int(e) for e in exits])
     code = lib.jkv_rvq_encode_kv(
         key.data_ptr(), value.data_ptr(), _lib.dtype_code(key.dtype), batch, heads, tokens, groups, d,
         *strides, key_tables.data_ptr(), value_tables.data_ptr(), stages, clusters,
-        codes[0].data_ptr(), codes[1].data_ptr(), *codes[0].stride()[:3], len(exits), depth_arr,
+        codes[0].data_ptr(), codes[1].data_ptr(), *code_strides, len(exits), depth_arr,
         _lib.ptr_array(ctypes.c_void_p, [r.data_ptr() for r in recon_k]),
         _lib.ptr_array(ctypes.c_void_p, [r.data_ptr() for r in recon_v]),
         _lib.ptr(workspace), ws_bytes, _lib.stream_handle(device),
@@ -161,8 +164,8 @@ def rvq_encode_many(
     # tensors are enqueued in well under the launch's own GPU time
     first = states[0]
     device = _lib.require_device(first, tables[0])
-    batch, heads, tokens, dim = map(int, first.shape)
-    problems, stages, clusters, d = map(int, tables[0].shape)
+    batch, heads, tokens, dim = first.shape
+    problems, stages, clusters, d = tables[0].shape
     if dim != groups * group_dim or d != group_dim or problems != heads * groups:
         raise ValueError("state and table geometry differs")
     if len(exits) > _lib.MAX_EXITS:
@@ -217,7 +220,7 @@ def nearest_f32(states: torch.Tensor, tables: torch.Tensor) -> torch.Tensor:
     device = _lib.require_device(states, tables)
     if states.ndim != 3 or tables.ndim != 3:
         raise ValueError("nearest-neighbor inputs must have [H,N,D]/[H,K,D]")
-    heads, tokens, dim = map(int, states.shape)
+    heads, tokens, dim = states.shape
     if int(tables.shape[0]) != heads or int(tables.shape[2]) != dim:
         raise ValueError("nearest-neighbor geometry differs")
     states = states.detach().float().contiguous()
@@ -238,7 +241,7 @@ def nearest_topk_f32(states: torch.Tensor, tables: torch.Tensor, candidates: int
     device = _lib.require_device(states, tables, excluded)
     if states.ndim != 3 or tables.ndim != 3:
         raise ValueError("nearest-neighbor inputs must have [H,N,D]/[H,K,D]")
-    heads, tokens, dim = map(int, states.shape)
+    heads, tokens, dim = states.shape
     if int(tables.shape[0]) != heads or int(tables.shape[2]) != dim:
         raise ValueError("nearest-neighbor geometry differs")
     if excluded is not None:
@@ -263,7 +266,7 @@ def gain_shape_sums(rows: torch.Tensor, indices: torch.Tensor, clusters: int, *,
     device = _lib.require_device(rows, indices, weights)
     if rows.ndim != 3 or indices.shape != rows.shape[:2]:
         raise ValueError("gain-shape rows/indices must be [H,N,D]/[H,N]")
-    heads, tokens, dim = map(int, rows.shape)
+    heads, tokens, dim = rows.shape
     rows = rows.detach().float().contiguous()
     indices = indices.to(torch.int64).contiguous()
     if weights is not None:
@@ -292,7 +295,7 @@ def subtract_codewords(residual: torch.Tensor, tables: torch.Tensor, indices: to
             or tables.ndim != 3 or indices.shape != residual.shape[:2]
             or tables.shape[0] != residual.shape[0] or tables.shape[2] != residual.shape[2]):
         raise ValueError("residual must be contiguous fp32 [H,N,D] with tables [H,K,D] and indices [H,N]")
-    heads, tokens, dim = map(int, residual.shape)
+    heads, tokens, dim = residual.shape
     tables = tables.detach().float().contiguous()
     indices = indices.to(torch.int64).contiguous()
     _lib.check(_lib.load().jkv_subtract_codewords(
@@ -312,8 +315,8 @@ def rvq_decode(
     same result, half the table bytes read."""
 
     device = _lib.require_device(codes, tables)
-    batch, heads, tokens, groups, stages = map(int, codes.shape)
-    problems, t_stages, clusters, d = map(int, tables.shape)
+    batch, heads, tokens, groups, stages = codes.shape
+    problems, t_stages, clusters, d = tables.shape
     if problems != heads * groups or t_stages != stages:
         raise ValueError("code and table geometry differs")
     if codes.dtype != torch.uint8 or codes.stride(-1) != 1 or codes.stride(-2) != stages:
@@ -348,8 +351,8 @@ def rvq_scatter_grad(
     """Accumulate the straight-through codebook gradient into ``grad_tables``."""
 
     device = _lib.require_device(codes, grad_tables, *grads)
-    batch, heads, tokens, groups, stages = map(int, codes.shape)
-    problems, t_stages, clusters, d = map(int, grad_tables.shape)
+    batch, heads, tokens, groups, stages = codes.shape
+    problems, t_stages, clusters, d = grad_tables.shape
     if problems != heads * groups or t_stages != stages or d != group_dim:
         raise ValueError("code and gradient-table geometry differs")
     if grad_tables.dtype != torch.float32 or not grad_tables.is_contiguous():
@@ -361,8 +364,8 @@ def rvq_scatter_grad(
     align = (8 if d % 8 == 0 else 4) * grads[0].element_size()
     grads = [g if g.data_ptr() % align == 0 else g.clone() for g in grads]
     lib = _lib.load()
-    ws_bytes = int(lib.jkv_rvq_scatter_workspace_bytes(
-        batch, heads, tokens, groups, d, stages, clusters, _lib.dtype_code(dtype), int(deterministic)))
+    ws_bytes = _lib.workspace_bytes("jkv_rvq_scatter_workspace_bytes", batch, heads, tokens, groups, d, stages,
+                                    clusters, _lib.dtype_code(dtype), int(deterministic))
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
     code = lib.jkv_rvq_scatter_grad(
         len(grads), _lib.ptr_array(ctypes.c_void_p, [g.data_ptr() for g in grads]),
@@ -398,7 +401,7 @@ def rvq_scatter_grad_many(
         return []
     device = _lib.require_device(*codes, *(g for gs in grads for g in gs),
                                  *(grad_tables if grad_tables is not None else ()))
-    batch, heads, tokens, groups, stages = map(int, codes[0].shape)
+    batch, heads, tokens, groups, stages = codes[0].shape
     n_exits = len(exits)
     if any(len(gs) != n_exits for gs in grads):
         raise ValueError("every job needs one gradient per exit")
@@ -439,8 +442,8 @@ def rvq_scatter_grad_many(
                 g = g.to(dtype).contiguous()
             flat.append(g if g.data_ptr() % align == 0 else g.clone())
     lib = _lib.load()
-    ws_bytes = int(lib.jkv_rvq_scatter_workspace_bytes(
-        batch, heads, tokens, groups, d, stages, clusters, _lib.dtype_code(dtype), int(deterministic)))
+    ws_bytes = _lib.workspace_bytes("jkv_rvq_scatter_workspace_bytes", batch, heads, tokens, groups, d, stages,
+                                    clusters, _lib.dtype_code(dtype), int(deterministic))
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
     code = lib.jkv_rvq_scatter_grad_many(
         len(codes), n_exits, _lib.ptr_array(ctypes.c_void_p, [g.data_ptr() for g in flat]),
@@ -529,7 +532,7 @@ def rope_table(device: torch.device, theta: float, n_pos: int) -> torch.Tensor:
     """Cached fp16 rotary table [n_pos', 2, 64] (cos row, sin row per position)
     with n_pos' >= n_pos."""
 
-    key = (str(device), float(theta))
+    key = (device, float(theta))
     table = _ROPE_CACHE.get(key)
     if table is not None and table.shape[0] >= n_pos:
         return table
@@ -570,18 +573,20 @@ def decode_attention(
     device = _lib.require_device(q, key_codes, value_codes, key_tables16, value_tables16, lengths)
     if q.dtype != torch.float16 or q.ndim != 3 or q.stride(-1) != 1:
         raise ValueError("decode queries must be fp16 [B,QH,D] with a contiguous last axis")
-    batch, qheads, dim = map(int, q.shape)
+    batch, qheads, dim = q.shape
     if key_codes.shape != value_codes.shape or key_codes.dtype != torch.uint8:
         raise ValueError("key/value code caches differ")
-    kb, kvheads, cap, groups, stages = map(int, key_codes.shape)
+    kb, kvheads, cap, groups, stages = key_codes.shape
     if kb != batch:
         raise ValueError("query and cache batch differ")
-    for c in (key_codes, value_codes):
-        if c.stride(-1) != 1 or c.stride(-2) != stages or c.stride(-3) != groups * stages:
-            raise ValueError("code caches need contiguous [cap,G,S] blocks")
-    if key_codes.stride() != value_codes.stride():
+    strides = key_codes.stride()
+    value_strides = value_codes.stride()
+    block = (groups * stages, stages, 1)
+    if strides[2:] != block or value_strides[2:] != block:
+        raise ValueError("code caches need contiguous [cap,G,S] blocks")
+    if strides != value_strides:
         raise ValueError("key/value code caches need identical strides")
-    problems, t_stages, clusters, d = map(int, key_tables16.shape)
+    problems, t_stages, clusters, d = key_tables16.shape
     if key_tables16.shape != value_tables16.shape or problems != kvheads * groups or t_stages != stages:
         raise ValueError("code-cache and codebook geometry differs")
     if key_tables16.dtype != torch.float16 or value_tables16.dtype != torch.float16:
@@ -599,13 +604,13 @@ def decode_attention(
     # shorter than the model's window)
     span = max(1, min(int(window), int(max_length)))
     lib = _lib.load()
-    out = torch.empty((batch, qheads, dim), dtype=torch.float16, device=device)
-    ws_bytes = int(lib.jkv_decode_workspace_bytes(batch, qheads, dim, span))
+    out = q.new_empty((batch, qheads, dim))
+    ws_bytes = _lib.workspace_bytes("jkv_decode_workspace_bytes", batch, qheads, dim, span)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     if key_new is None and value_new is None:
         code = lib.jkv_decode_attention(
             q.data_ptr(), q.stride(0), q.stride(1), key_codes.data_ptr(), value_codes.data_ptr(),
-            key_codes.stride(0), key_codes.stride(1), cap, key_tables16.data_ptr(),
+            strides[0], strides[1], cap, key_tables16.data_ptr(),
             value_tables16.data_ptr(), batch, qheads, kvheads, groups, d, stages, clusters,
             lengths.data_ptr(), span, table.data_ptr(), int(table.shape[0]), out.data_ptr(),
             workspace.data_ptr(), ws_bytes, _lib.stream_handle(device),
@@ -622,7 +627,7 @@ def decode_attention(
         code = lib.jkv_decode_attention_append(
             q.data_ptr(), q.stride(0), q.stride(1), key_new.data_ptr(), value_new.data_ptr(),
             key_new.stride(0), key_new.stride(1), key_codes.data_ptr(), value_codes.data_ptr(),
-            key_codes.stride(0), key_codes.stride(1), cap, key_tables16.data_ptr(),
+            strides[0], strides[1], cap, key_tables16.data_ptr(),
             value_tables16.data_ptr(), batch, qheads, kvheads, groups, d, stages, clusters,
             lengths.data_ptr(), span, table.data_ptr(), int(table.shape[0]), out.data_ptr(),
             workspace.data_ptr(), ws_bytes, _lib.stream_handle(device),
@@ -651,10 +656,10 @@ def decode_attention_window(
     device = _lib.require_device(q, key_window, value_window, lengths)
     if q.dtype != torch.float16 or q.ndim != 3 or q.stride(-1) != 1:
         raise ValueError("decode queries must be fp16 [B,QH,D] with a contiguous last axis")
-    batch, qheads, dim = map(int, q.shape)
+    batch, qheads, dim = q.shape
     if key_window.shape != value_window.shape or key_window.dtype != torch.float16 or key_window.ndim != 4:
         raise ValueError("decoded windows must be two fp16 [B,KVH,cap,128] tensors of one shape")
-    wb, kvheads, cap, wd = map(int, key_window.shape)
+    wb, kvheads, cap, wd = key_window.shape
     if wb != batch or wd != dim:
         raise ValueError("query and decoded window geometry differ")
     for w in (key_window, value_window):
@@ -672,8 +677,8 @@ def decode_attention_window(
     table = rope_table(device, rope_theta, int(max_length) + 1)
     span = max(1, min(int(window), int(max_length)))
     lib = _lib.load()
-    out = torch.empty((batch, qheads, dim), dtype=torch.float16, device=device)
-    ws_bytes = int(lib.jkv_decode_workspace_bytes(batch, qheads, dim, span))
+    out = q.new_empty((batch, qheads, dim))
+    ws_bytes = _lib.workspace_bytes("jkv_decode_workspace_bytes", batch, qheads, dim, span)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     code = lib.jkv_decode_attention_window(
         q.data_ptr(), q.stride(0), q.stride(1), key_window.data_ptr(), value_window.data_ptr(),
@@ -690,7 +695,7 @@ def _prefill_operands(q, key, value_or_grad, start_positions, what):
     for name, t in (("query", q), ("key", key), (what, value_or_grad)):
         if t.dtype != torch.float16 or t.ndim != 4 or t.shape[-1] != 128 or t.stride(-1) != 1:
             raise ValueError(f"prefill {name} must be fp16 [B,H,T,128] with a contiguous last axis")
-    batch, qheads, tokens, _dim = map(int, q.shape)
+    batch, qheads, tokens, _dim = q.shape
     if key.shape[0] != batch or key.shape[2] != tokens:
         raise ValueError("prefill query/key/value geometry differs")
     kvheads = int(key.shape[1])
@@ -698,7 +703,8 @@ def _prefill_operands(q, key, value_or_grad, start_positions, what):
         raise ValueError("query heads must be a multiple of kv heads")
     tensors = []
     for t in (q, key, value_or_grad):
-        if any(st % 8 for st in t.stride()[:3]) or t.data_ptr() % 16:
+        b, h, r, _one = t.stride()
+        if b % 8 or h % 8 or r % 8 or t.data_ptr() % 16:
             t = t.contiguous()
         tensors.append(t)
     if start_positions.dtype != torch.int32 or start_positions.shape != (batch,):
@@ -735,7 +741,7 @@ def prefill_attention(
                             or not lse.is_contiguous() or lse.device != q.device):
         raise ValueError("lse must be a contiguous fp32 [B,QH,T] tensor on the query's device")
     table = rope_table(device, rope_theta, int(max_position) + 1)
-    out = torch.empty((batch, qheads, tokens, 128), dtype=torch.float16, device=device)
+    out = q.new_empty((batch, qheads, tokens, 128))
     code = _lib.load().jkv_prefill_attention(
         q.data_ptr(), *q.stride()[:3], key.data_ptr(), *key.stride()[:3], value.data_ptr(),
         *value.stride()[:3], batch, qheads, kvheads, tokens, 128, start_positions.data_ptr(),
@@ -783,8 +789,8 @@ def prefill_attention_codes(
         raise ValueError("prefill from codes needs [B,KVH,T,16,S<=2] codes and [KVH*16,S,256,8] tables")
     if q.dtype != torch.float16 or q.ndim != 4 or q.shape[-1] != 128 or q.stride(-1) != 1:
         raise ValueError("prefill query must be fp16 [B,H,T,128] with a contiguous last axis")
-    batch, qheads, tokens, _dim = map(int, q.shape)
-    _b, kvheads, _t, groups, stages = map(int, key_codes.shape)
+    batch, qheads, tokens, _dim = q.shape
+    _b, kvheads, _t, groups, stages = key_codes.shape
     if (_b, _t) != (batch, tokens) or qheads % kvheads:
         raise ValueError("prefill query/key/value geometry differs")
     if tuple(key_tables16.shape[:2]) != (kvheads * groups, stages):
@@ -856,7 +862,7 @@ def prefill_attention_backward(
              for want, shape in zip(need, ((batch, qheads, tokens, 128), (batch, kvheads, tokens, 128),
                                            (batch, kvheads, tokens, 128)))]
     lib = _lib.load()
-    ws_bytes = int(lib.jkv_prefill_backward_workspace_bytes(batch, qheads, kvheads, tokens, int(window)))
+    ws_bytes = _lib.workspace_bytes("jkv_prefill_backward_workspace_bytes", batch, qheads, kvheads, tokens, int(window))
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     code = lib.jkv_prefill_attention_backward(
         q.data_ptr(), *q.stride()[:3], key.data_ptr(), *key.stride()[:3], value.data_ptr(), *value.stride()[:3],
@@ -893,7 +899,7 @@ def prefill_attention_value_grad(
     table = rope_table(device, rope_theta, int(max_position) + 1)
     d_value = torch.empty((batch, kvheads, tokens, 128), dtype=torch.float32, device=device)
     lib = _lib.load()
-    ws_bytes = int(lib.jkv_prefill_value_grad_workspace_bytes(batch, qheads, kvheads, tokens, int(window)))
+    ws_bytes = _lib.workspace_bytes("jkv_prefill_value_grad_workspace_bytes", batch, qheads, kvheads, tokens, int(window))
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     code = lib.jkv_prefill_attention_value_grad(
         q.data_ptr(), *q.stride()[:3], key.data_ptr(), *key.stride()[:3], d_out.data_ptr(),

@@ -125,8 +125,13 @@ def _start_tensor(start_positions, batch: int, tokens: int, device) -> tuple[tor
         if starts.numel() == 1 and batch != 1:
             starts = starts.expand(batch).contiguous()
         top = int(starts.max().item()) if batch else 0
+    elif isinstance(start_positions, int):
+        # a fill on the stream: a tensor built from host values is a copy that
+        # waits for the device's queued work
+        starts = torch.full((batch,), int(start_positions), dtype=torch.int32, device=device)
+        top = int(start_positions) if batch else 0
     else:
-        values = [int(start_positions)] * batch if isinstance(start_positions, int) else [int(x) for x in start_positions]
+        values = [int(x) for x in start_positions]
         starts = torch.tensor(values, dtype=torch.int32, device=device)
         top = max(values) if values else 0
     if starts.shape != (batch,):
@@ -154,7 +159,7 @@ def prefill_attention(
     Returns ``[B,QH,T,128]`` fp16.
     """
 
-    batch, _qh, tokens, _d = map(int, query.shape)
+    batch, _qh, tokens, _d = query.shape
     starts, top = _start_tensor(start_positions, batch, tokens, query.device)
     if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad):
         return _PrefillAttention.apply(query, key, value, starts, window, rope_theta, top)
@@ -171,7 +176,7 @@ class _PrefillAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, query, key, value, starts, window, rope_theta, top):
-        batch, qheads, tokens, _d = map(int, query.shape)
+        batch, qheads, tokens, _d = query.shape
         lse = torch.empty((batch, qheads, tokens), dtype=torch.float32, device=query.device)
         out = _ops.prefill_attention(query, key, value, starts, window=window, rope_theta=rope_theta,
                                      max_position=top, lse=lse)
@@ -228,7 +233,7 @@ def prefill_attention_from_codes(
     if fused:
         if not _ops.prefill_codes_supported(key_codes, key_tables16):
             raise ValueError("the fused prefill needs [B,KVH,T,16,S<=2] codes and [KVH*16,S,256,8] tables")
-        batch, _qh, tokens, _d = map(int, query.shape)
+        batch, _qh, tokens, _d = query.shape
         starts, top = _start_tensor(start_positions, batch, tokens, query.device)
         return _ops.prefill_attention_codes(query, key_codes, value_codes, key_tables16, value_tables16, starts,
                                             window=window, rope_theta=rope_theta, max_position=top)

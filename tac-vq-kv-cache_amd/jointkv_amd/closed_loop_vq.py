@@ -43,8 +43,8 @@ class _HardResidualVQ(torch.autograd.Function):
     @staticmethod
     def forward(ctx, states, tables, whiteners, groups, group_dim, exits, straight_through, deterministic):
         recon, codes = _ops.rvq_encode(
-            states.detach(),
-            tables.detach(),
+            states,
+            tables,
             groups=groups,
             group_dim=group_dim,
             exits=exits,
@@ -100,10 +100,10 @@ class _HardResidualVQPair(torch.autograd.Function):
     def forward(ctx, key_states, value_states, key_tables, value_tables, groups, group_dim, exits,
                 straight_through, deterministic):
         rk, ck, rv, cv = _ops.rvq_encode_kv(
-            key_states.detach(),
-            value_states.detach(),
-            key_tables.detach(),
-            value_tables.detach(),
+            key_states,
+            value_states,
+            key_tables,
+            value_tables,
             groups=groups,
             group_dim=group_dim,
             exits=exits,
@@ -135,6 +135,12 @@ class _HardResidualVQPair(torch.autograd.Function):
         return gsk, gsv, gtk, gtv, None, None, None, None, None
 
 
+def _flat_masters(tables: torch.Tensor, shape: tuple[int, int, int, int]) -> torch.Tensor:
+    """fp32 masters as the contiguous ``[P,S,K,d]`` the kernels read."""
+
+    return (tables if tables.dtype == torch.float32 else tables.float()).reshape(shape).contiguous()
+
+
 def hard_residual_vq_pair(
     key_states: torch.Tensor,
     value_states: torch.Tensor,
@@ -159,11 +165,11 @@ def hard_residual_vq_pair(
         raise ValueError("K and V states must share their geometry")
     if key_tables.shape != value_tables.shape or key_states.ndim != 4 or key_tables.ndim not in (4, 5):
         raise ValueError("K and V tables must share their geometry")
-    batch, heads, tokens, dimension = map(int, key_states.shape)
+    batch, heads, tokens, dimension = key_states.shape
     if key_tables.ndim == 5:
-        t_heads, groups, stages, clusters, group_dim = map(int, key_tables.shape)
+        t_heads, groups, stages, clusters, group_dim = key_tables.shape
     else:
-        t_heads, stages, clusters, group_dim = map(int, key_tables.shape)
+        t_heads, stages, clusters, group_dim = key_tables.shape
         groups = 1
     if t_heads != heads or groups * group_dim != dimension:
         raise ValueError("state and table geometry differs")
@@ -171,13 +177,10 @@ def hard_residual_vq_pair(
     if not requested or requested[0] <= 0 or requested[-1] > stages:
         raise ValueError("requested prefixes lie outside the VQ ladder")
 
-    def flat(tables):
-        t = tables if tables.dtype == torch.float32 else tables.float()
-        return t.reshape(heads * groups, stages, clusters, group_dim).contiguous()
-
+    shape = (heads * groups, stages, clusters, group_dim)
     outputs = _HardResidualVQPair.apply(
-        key_states, value_states, flat(key_tables), flat(value_tables), groups, group_dim, requested,
-        straight_through_states, deterministic_backward,
+        key_states, value_states, _flat_masters(key_tables, shape), _flat_masters(value_tables, shape), groups,
+        group_dim, requested, straight_through_states, deterministic_backward,
     )
     n = len(requested)
     kc, vc = outputs[2 * n], outputs[2 * n + 1]
@@ -235,7 +238,7 @@ def hard_residual_vq_exits(
 
     if states.ndim != 4 or tables.ndim != 4:
         raise ValueError("states/tables must have [B,H,T,D]/[H,S,K,D]")
-    batch, heads, tokens, dimension = map(int, states.shape)
+    batch, heads, tokens, dimension = states.shape
     if tables.shape[0] != heads or tables.shape[-1] != dimension:
         raise ValueError("state and table geometry differs")
     requested = tuple(sorted(set(int(depth) for depth in prefixes)))
@@ -290,8 +293,8 @@ def hard_grouped_residual_vq(
 
     if states.ndim != 4 or tables.ndim != 5:
         raise ValueError("states/tables must have [B,H,T,G*d]/[H,G,S,K,d]")
-    batch, heads, tokens, dimension = map(int, states.shape)
-    t_heads, groups, stages, clusters, group_dim = map(int, tables.shape)
+    batch, heads, tokens, dimension = states.shape
+    t_heads, groups, stages, clusters, group_dim = tables.shape
     if t_heads != heads or groups * group_dim != dimension:
         raise ValueError("state and table geometry differs")
     requested = tuple(sorted(set(int(depth) for depth in prefixes)))
@@ -333,7 +336,7 @@ def frozen_assignment_reconstruction(
 
     if states.ndim != 4 or tables.ndim != 4 or indices.ndim != 4:
         raise ValueError("frozen assignment geometry must be [B,H,T,D]/[H,S,K,D]/[B,H,T,S]")
-    batch, heads, tokens, dimension = map(int, states.shape)
+    batch, heads, tokens, dimension = states.shape
     stages = int(tables.shape[1])
     if int(tables.shape[0]) != heads or int(tables.shape[-1]) != dimension:
         raise ValueError("frozen assignment table geometry differs")

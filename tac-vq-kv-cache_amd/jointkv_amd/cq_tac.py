@@ -14,7 +14,7 @@ from collections.abc import Sequence
 import torch
 import torch.nn as nn
 
-from .closed_loop_vq import QuantizedKV, _run, hard_residual_vq_pair
+from .closed_loop_vq import QuantizedKV, _flat_masters, _HardResidualVQPair, _run
 
 
 def hard_grouped_cq(
@@ -37,8 +37,8 @@ def hard_grouped_cq(
 
     if states.ndim != 4 or codebooks.ndim != 4:
         raise ValueError("states/codebooks must be [B,H,T,D]/[H,G,K,S]")
-    batch, heads, tokens, dimension = map(int, states.shape)
-    cb_heads, groups, clusters, subdimension = map(int, codebooks.shape)
+    batch, heads, tokens, dimension = states.shape
+    cb_heads, groups, clusters, subdimension = codebooks.shape
     if cb_heads != heads or groups * subdimension != dimension:
         raise ValueError("CQ codebook geometry differs from states")
     if token_chunk_size <= 0:
@@ -140,13 +140,14 @@ class ClosedLoopGroupedCQ(nn.Module):
             raise ValueError("grouped CQ supports one fixed-rate uniform mode")
         whitener = None if self._identity_selector[layer] else self.key_whitener(layer)
         kt, vt = self.key_tables[layer], self.value_tables[layer]
-        heads, groups, _k, sub = map(int, kt.shape)
+        heads, groups, clusters, sub = kt.shape
         if (whitener is None and raw_key.shape == raw_value.shape and raw_key.dtype == raw_value.dtype
                 and raw_key.ndim == 4 and raw_key.shape[1] == heads and raw_key.shape[3] == groups * sub):
             # one launch for the layer's K and V (same bits as two encodes)
-            kx, kc, vx, vc = hard_residual_vq_pair(raw_key, raw_value, kt.unsqueeze(2), vt.unsqueeze(2),
-                                                   prefixes=(1,))
-            key, key_indices, value, value_indices = kx[1], kc[..., 0], vx[1], vc[..., 0]
+            shape = (heads * groups, 1, clusters, sub)
+            key, value, kc, vc = _HardResidualVQPair.apply(
+                raw_key, raw_value, _flat_masters(kt, shape), _flat_masters(vt, shape), groups, sub, (1,), True, False)
+            key_indices, value_indices = kc.select(-1, 0), vc.select(-1, 0)
         else:
             key, key_indices = hard_grouped_cq(
                 raw_key,
