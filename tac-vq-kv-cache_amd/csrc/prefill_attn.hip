@@ -2,8 +2,8 @@
 // fp16 K̂/V̂ (pre-RoPE), with the reference model's fp16 rotary applied to
 // q and K̂ at absolute positions start[b] + t.
 //
-// One workgroup of 8 waves per (batch, kv head, head group, block of query
-// rows).  Each wave owns one query head and 32 query rows (two 16-row
+// One workgroup of 8 waves (4 for small grids) per (batch, kv head, head
+// group, block of query rows).  Each wave owns one query head and 32 query rows (two 16-row
 // groups); the workgroup
 // shares 64-key tiles of rotated K̂ ([key][dim]) and V̂ᵀ ([dim][key]) in LDS,
 // double-buffered: the next tile's global loads are issued before the
@@ -17,6 +17,7 @@
 // with an online softmax in fp32 (base-2 exponent, scale folded in).
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "jkv_common.h"
@@ -26,7 +27,6 @@ namespace jkv {
 
 static const int kPD = 128;            // head dim
 static const int kPKT = 64;            // keys per tile
-static const int kPThreads = 512;      // 8 waves
 static const int kKStride = kPD + 8;   // K̂ tile row stride (halves): 272 B spreads keys over banks
 static const int kVStride = kPKT + 4;  // V̂ᵀ tile row stride (halves): 136 B, conflict-free b64 reads and pair writes
 static const int kKTile = kPKT * kKStride;
@@ -47,8 +47,10 @@ struct PrefillArgs {
   _Float16* out;  // [B,QH,T,D] contiguous
   float* lse;     // [B,QH,T] natural-log row normaliser, or null
   int32_t heads_per_wg;  // HW: query heads per workgroup (min(NQ, 4))
-  int32_t row_sets;      // 8 / HW: 32-row sets per head in a workgroup
+  int32_t row_sets;      // waves / HW: 32-row sets per head in a workgroup
   int32_t head_groups;   // NQ / HW
+  int32_t group;         // slices per run of the block order (divides an XCD's slices)
+  int32_t fold;          // blocks per XCD after which the order runs backwards (0: nowhere)
   // codes instead of K̂/V̂ rows (prefill_attn_kernel<CS>, CS = stages): uint8
   // records [B,KVH,T,16,CS] with byte strides and the fp16 deployed tables
   // [KVH*16][CS][256][8]
@@ -101,8 +103,10 @@ __device__ __forceinline__ half4 lds_read_tr16(uint32_t addr) {
 // codes while each tile loads (codes -> 16-byte codeword gathers from the
 // L2-resident fp16 tables -> fp16 stage sum, the codec's reconstruction), so
 // K̂ and V̂ are never written to memory.
-template <int CS>
-__global__ __launch_bounds__(kPThreads) void prefill_attn_kernel(PrefillArgs a) {
+template <int CS, int NWV>
+__global__ __launch_bounds__(64 * NWV) void prefill_attn_kernel(PrefillArgs a) {
+  static_assert(NWV == 8 || (NWV == 4 && CS == 0), "eight waves, or four from fp16 rows");
+  constexpr int NK = 8 / NWV;  // K̂ rows a thread stages per tile
   __shared__ __align__(16) _Float16 k_lds[2][kKTile];
   __shared__ __align__(16) _Float16 v_lds[2][kVTile];
 
@@ -112,14 +116,21 @@ __global__ __launch_bounds__(kPThreads) void prefill_attn_kernel(PrefillArgs a) 
   const int HW = a.heads_per_wg, RS = a.row_sets;
   const int64_t block_rows = 32 * (int64_t)RS;
   const int64_t nqb = ceil_div(a.T, block_rows);
-  // logical block: query blocks fastest, then (kv head, head group), then
-  // batch row.  xcd_remap keeps the query blocks of one (batch, kv head) on
-  // one XCD, so its K/V tiles are fetched into one L2; longest key ranges go
-  // first within each.
-  const uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
+  // logical block: an XCD's blocks are runs of `group` (batch row, kv head,
+  // head group) slices, each run longest key ranges first over all its
+  // slices.  xcd_remap keeps the query blocks of one slice on one XCD, so its
+  // K/V tiles are fetched into one L2.  Where every block is resident at
+  // once, two per CU, the second half runs backwards: a CU's first block is
+  // long where its second is short.
+  uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
+  if (a.fold > 0) {
+    const uint32_t per = gridDim.x >> 3, at = bid % per, first = (uint32_t)a.fold;
+    if (at >= first) bid += per - 1 - at + first - at;  // at -> first + (per - 1 - at)
+  }
   const int64_t gy = a.KVH * a.head_groups;
-  const int64_t qblk = nqb - 1 - (int64_t)(bid % (uint32_t)nqb);
-  const int64_t yz = bid / (uint32_t)nqb;
+  const uint32_t run = (uint32_t)a.group * (uint32_t)nqb, in_run = bid % run;
+  const int64_t qblk = nqb - 1 - (int64_t)(in_run / (uint32_t)a.group);
+  const int64_t yz = (int64_t)(bid / run) * a.group + in_run % (uint32_t)a.group;
   const int64_t kvh = (yz % gy) / a.head_groups;
   const int64_t hg = (yz % gy) % a.head_groups;
   const int64_t b = yz / gy;
@@ -188,7 +199,7 @@ __global__ __launch_bounds__(kPThreads) void prefill_attn_kernel(PrefillArgs a) 
   // same dims (groups p and p + 8 for K̂, group tid/32 of both keys for V̂)
   constexpr int NW = CS > 0 ? CS : 1;
   struct TileRegs {
-    half8 k[2][NW], v[2][NW], cs, sn;
+    half8 k[NK][2][NW], v[2][NW], cs[NK], sn[NK];
   };
   // the code bytes of one tile's K̂ pair and V̂ keys (CS > 0): dword 0 holds
   // groups p and p + 8 of key tid/8 (CS bytes each, at bytes 0 and 2), dword 1
@@ -261,41 +272,48 @@ __global__ __launch_bounds__(kPThreads) void prefill_attn_kernel(PrefillArgs a) 
   auto fetch = [&](int64_t tile, const CodeRegs& c, TileRegs& r) {
     if constexpr (CS == 0) {
       const int32_t first = (int32_t)(tile * kPKT);
-      const uint32_t kr = first + kk < T32 ? (uint32_t)kk : 0u;
-      int32_t pos = p32 >= rlast32 ? rlast32 : p32 + first + (int32_t)kr;  // (no int32 overflow)
-      pos = pos < 0 ? 0 : (pos < rlast32 ? pos : rlast32);
-      const uint32_t ko = kr * (uint32_t)a.kst * 2u + 16u * kpart, to = (uint32_t)pos * (2u * kRopeRow) + 16u * kpart;
       const int ks = (int)((uint32_t)first * (uint32_t)a.kst * 2u);
-      r.k[0][0] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, (int)ko, ks, 0));
-      r.k[1][0] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, (int)(ko + 128u), ks, 0));
-      r.cs = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(t_rsrc, (int)to, 0, 0));
-      r.sn = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(t_rsrc, (int)(to + 128u), 0, 0));
+#pragma unroll
+      for (int n = 0; n < NK; ++n) {
+        const int row = kk + 8 * NWV * n;
+        const uint32_t kr = first + row < T32 ? (uint32_t)row : 0u;
+        int32_t pos = p32 >= rlast32 ? rlast32 : p32 + first + (int32_t)kr;  // (no int32 overflow)
+        pos = pos < 0 ? 0 : (pos < rlast32 ? pos : rlast32);
+        const uint32_t ko = kr * (uint32_t)a.kst * 2u + 16u * kpart, to = (uint32_t)pos * (2u * kRopeRow) + 16u * kpart;
+        r.k[n][0][0] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, (int)ko, ks, 0));
+        r.k[n][1][0] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, (int)(ko + 128u), ks, 0));
+        r.cs[n] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(t_rsrc, (int)to, 0, 0));
+        r.sn[n] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(t_rsrc, (int)(to + 128u), 0, 0));
+      }
     } else {
       const TileBase t = tile_base(tile);
-      r.cs = *(const half8*)(t.tt + t.to);
-      r.sn = *(const half8*)(t.tt + t.to + 64);
+      r.cs[0] = *(const half8*)(t.tt + t.to);
+      r.sn[0] = *(const half8*)(t.tt + t.to + 64);
 #pragma unroll
       for (int st = 0; st < CS; ++st) {
-        r.k[0][st] = word(ktab, kpart, st, (c.kw >> (8 * st)) & 0xffu);
-        r.k[1][st] = word(ktab, kpart + 8, st, (c.kw >> (16 + 8 * st)) & 0xffu);
+        r.k[0][0][st] = word(ktab, kpart, st, (c.kw >> (8 * st)) & 0xffu);
+        r.k[0][1][st] = word(ktab, kpart + 8, st, (c.kw >> (16 + 8 * st)) & 0xffu);
         r.v[0][st] = word(vtab, vdb, st, (c.vw >> (8 * st)) & 0xffu);
         r.v[1][st] = word(vtab, vdb, st, (c.vw >> (16 + 8 * st)) & 0xffu);
       }
     }
   };
   auto store = [&](const TileRegs& r, int buf) {
-    // the codec's reconstruction: fp16 of the fp32 stage sum, which one fp16
-    // add gives for two stages
-    half8 k0 = r.k[0][0], k1 = r.k[1][0];
-    if constexpr (CS == 2) {
-      k0 = k0 + r.k[0][1];
-      k1 = k1 + r.k[1][1];
+#pragma unroll
+    for (int n = 0; n < NK; ++n) {
+      // the codec's reconstruction: fp16 of the fp32 stage sum, which one fp16
+      // add gives for two stages
+      half8 k0 = r.k[n][0][0], k1 = r.k[n][1][0];
+      if constexpr (CS == 2) {
+        k0 = k0 + r.k[n][0][1];
+        k1 = k1 + r.k[n][1][1];
+      }
+      half8 r0, r1;
+      rope16(k0, k1, r.cs[n], r.sn[n], &r0, &r1);
+      _Float16* kd = k_lds[buf] + (kk + 8 * NWV * n) * kKStride + 8 * kpart;
+      *(half8*)kd = r0;
+      *(half8*)(kd + 64) = r1;
     }
-    half8 r0, r1;
-    rope16(k0, k1, r.cs, r.sn, &r0, &r1);
-    _Float16* kd = k_lds[buf] + kk * kKStride + 8 * kpart;
-    *(half8*)kd = r0;
-    *(half8*)(kd + 64) = r1;
     if constexpr (CS > 0) {
       half8 v0 = r.v[0][0], v1 = r.v[1][0];
       if constexpr (CS == 2) {
@@ -311,8 +329,8 @@ __global__ __launch_bounds__(kPThreads) void prefill_attn_kernel(PrefillArgs a) 
   // ... lds: lane i of an instruction lands at its LDS base + 16 i), row-major
   // [key][dim] with 16-byte chunk j of key r in slot j ^ 2 (r & 7), so that
   // the transposing reads of the product below (32 bytes of 8 keys) hit
-  // distinct banks.  Wave w fills keys 8w..8w+7 with two instructions; keys
-  // past T read the tile's first key (their weights are 0).  Offsets fit 32
+  // distinct banks.  Wave w fills keys 8w..8w+7 (of each 8 NWV) with two
+  // instructions each; keys past T read the tile's first key (their weights are 0).  Offsets fit 32
   // bits (host-checked).
   const int vrow = 8 * wave + (lane >> 4), vslot = lane & 15;
   const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -322,11 +340,11 @@ __global__ __launch_bounds__(kPThreads) void prefill_attn_kernel(PrefillArgs a) 
       const int32_t first = (int32_t)(tile * kPKT), T32 = (int32_t)a.T;
       char* vd = (char*)v_lds[buf] + 2048 * wave;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int r = vrow + 4 * i;
+      for (int i = 0; i < 2 * NK; ++i) {
+        const int r = vrow + 4 * (i & 1) + 8 * NWV * (i >> 1);
         const uint32_t rr = first + r < T32 ? (uint32_t)r : 0u;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            v_rsrc, (void __attribute__((address_space(3)))*)(vd + 1024 * i), 16,
+            v_rsrc, (void __attribute__((address_space(3)))*)(vd + 1024 * (i & 1) + 2048 * NWV * (i >> 1)), 16,
             rr * (uint32_t)a.vst * 2u + 16u * (uint32_t)(vslot ^ (2 * (r & 7))), (uint32_t)first * (uint32_t)a.vst * 2u,
             0, 0);
       }
@@ -519,18 +537,42 @@ static int launch_prefill(PrefillArgs& a, int cs, const void* q, int64_t q_sb, i
   a.lse = lse;
   const int64_t NQ = QH / KVH;
   a.heads_per_wg = (int32_t)(NQ < 4 ? NQ : 4);
-  a.row_sets = 8 / a.heads_per_wg;
+  // From fp16 rows, four-wave workgroups (half the query rows, two per CU)
+  // where eight-wave ones would not go round the CUs twice: a tile then takes
+  // 2.4 us instead of 3.1 with a wave to itself on each SIMD, and both halves
+  // of the order pair up (below).  [1,32/8,T]: T = 333 23.2 -> 17.7 us, 777
+  // 40.0 -> 32.2, 2,048 91 -> 81; [2,1024] 52.9 -> 46.0; larger grids take
+  // the same time or (2 x 2,048: 121 against 133) longer in four-wave form.
+  const int64_t n8 = ceil_div(T, 32 * (int64_t)(8 / a.heads_per_wg)) * KVH * (NQ / a.heads_per_wg) * B;
+  const int waves = cs == 0 && n8 <= 256 ? 4 : 8;
+  a.row_sets = waves / a.heads_per_wg;
   a.head_groups = (int32_t)(NQ / a.heads_per_wg);
   const int64_t nqb = ceil_div(T, 32 * (int64_t)a.row_sets);
   const int64_t blocks = nqb * KVH * a.head_groups * B;
   JKV_CHECK_ARG(blocks < ((int64_t)1 << 31), "prefill grid too large");
-  const dim3 grid((uint32_t)blocks), block(kPThreads);
+  const int64_t slices = KVH * a.head_groups * B;
+  a.group = 1;
+  a.fold = 0;
+  if (slices % 8 == 0) {
+    // as many of an XCD's slices as leave their K/V (512 bytes per token) in
+    // half of its 4 MiB L2 (slice by slice, each began with long blocks while
+    // the one before ended: [4,32/8,1024] 94 -> 72 us, [16,2048] 922 -> 883,
+    // [64,512] 438 -> 390); four-wave blocks that all reside at once fold
+    // ([2,1024] 56.6 -> 46.0, [4,512] 35.0 -> 29.1)
+    const int64_t per = slices / 8, cap = std::max<int64_t>(1, (2 << 20) / (T * 512));
+    for (int64_t g = 1; g <= per && g <= cap; ++g)
+      if (per % g == 0) a.group = (int32_t)g;
+    if (waves == 4 && blocks > 256 && blocks <= 512) a.fold = 32;
+  }
+  const dim3 grid((uint32_t)blocks), block((uint32_t)(64 * waves));
   if (cs == 2) {
-    hipLaunchKernelGGL(prefill_attn_kernel<2>, grid, block, 0, stream, a);
+    hipLaunchKernelGGL((prefill_attn_kernel<2, 8>), grid, block, 0, stream, a);
   } else if (cs == 1) {
-    hipLaunchKernelGGL(prefill_attn_kernel<1>, grid, block, 0, stream, a);
+    hipLaunchKernelGGL((prefill_attn_kernel<1, 8>), grid, block, 0, stream, a);
+  } else if (waves == 4) {
+    hipLaunchKernelGGL((prefill_attn_kernel<0, 4>), grid, block, 0, stream, a);
   } else {
-    hipLaunchKernelGGL(prefill_attn_kernel<0>, grid, block, 0, stream, a);
+    hipLaunchKernelGGL((prefill_attn_kernel<0, 8>), grid, block, 0, stream, a);
   }
   JKV_CHECK_LAUNCH();
   return JKV_OK;

@@ -41,6 +41,27 @@ def test_prefill_matches_oracle(device, batch, qh, kvh, tokens, starts, window):
         assert torch.equal(out.cpu()[0, :, 0], v[0, 0, 0].expand(qh, 128))
 
 
+# the forms a grid's size picks: four-wave blocks (one, or two per CU with the
+# order folded) and eight-wave ones, runs of one and of several slices, slices
+# that do not spread over the XCDs, every heads-per-block layout
+@pytest.mark.parametrize("batch,qh,kvh,tokens,starts,window", [
+    (1, 32, 8, 333, (0,), 100),           # four waves, ragged last block
+    (4, 32, 8, 512, (0, 3, 9, 700), 4096),  # four waves, 512 blocks: folded
+    (2, 32, 8, 1000, (0, 50), 300),       # folded with a ragged half
+    (3, 8, 1, 300, (0, 1, 2), 4096),      # six slices (GQA 8): no runs
+    (8, 8, 8, 300, (5,) * 8, 4096),       # one head per block, runs of eight slices
+    (6, 32, 8, 770, (0,) * 6, 4096),      # eight waves, runs of several slices
+])
+def test_prefill_grid_forms(device, batch, qh, kvh, tokens, starts, window):
+    print(f"prefill forms B={batch} QH={qh} KVH={kvh} T={tokens} win={window}", flush=True)
+    q, k, v = _case(303 + tokens, batch, qh, kvh, tokens)
+    out = jkv.prefill_attention(q.to(device), k.to(device), v.to(device), list(starts), window=window).cpu()
+    for b in sorted({0, batch - 1}):
+        expect = ref.prefill_attention(q[b : b + 1], k[b : b + 1], v[b : b + 1], starts[b : b + 1], window=window)
+        err = float((out[b : b + 1].float() - expect.float()).abs().max())
+        assert err <= ATOL, f"row {b}: max abs error {err}"
+
+
 def test_prefill_from_codes_and_strided_inputs(device):
     # K/V as G2 codes rebuilt by the codec's decode, query as a strided view
     gen = torch.Generator().manual_seed(8601)
