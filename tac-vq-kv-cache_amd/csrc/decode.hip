@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256) void rvq_decode_kernel(RvqDecodeArgs a) {
 // i / G, i / G + 512 / G, ...: the 16 or 32 threads of a token write its row
 // in one contiguous run.  The same sums in the same order as
 // rvq_decode_kernel.
-static const int kLdsDecodeTokens = 512;  // shortest run
+static const int kLdsDecodeTokens = 128;  // shortest run
 template <int DT, bool F16>
 __global__ __launch_bounds__(512) void rvq_decode_lds_kernel(RvqDecodeArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -205,8 +205,10 @@ static int rvq_decode_impl(const uint8_t* codes, int64_t code_stride_b, int64_t 
     return d % cw == 0 && (uintptr_t)tables % tab_align == 0 && (uintptr_t)out % (cw * esize) == 0;
   };
   const int cw = aligned(8) ? 8 : aligned(4) ? 4 : 1;
-  // 8-dim groups whose head tables fit 128 KiB of LDS: gathers from LDS
-  const bool lds = d == 8 && K == 256 && G * S <= 32 && 512 % G == 0 && cw == 8 && depth <= 2 &&
+  // 8-dim groups whose head tables fit 128 KiB of LDS: gathers from LDS, once
+  // the rows pay for staging the tables (S = 2, 8 heads: 6.2 us against 3.4
+  // from L2 at 777 tokens, 7.2 both at 32,768 rows, 19 against 36 at 262,144)
+  const bool lds = B * H * T >= 32768 && d == 8 && K == 256 && G * S <= 32 && 512 % G == 0 && cw == 8 && depth <= 2 &&
                    (uintptr_t)tables % 16 == 0 && B * H * ceil_div(T, kLdsDecodeTokens) < ((int64_t)1 << 31);
   if (lds) {
     // runs long enough for one round of workgroups over 256 CUs (each holds

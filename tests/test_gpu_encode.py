@@ -441,6 +441,18 @@ def test_rvq_decode_lds_runs_match_oracle(device, groups, stages, depth, tables_
     assert torch.equal(got.cpu(), want)
 
 
+# either side of the row count from which the tables are staged in LDS
+@pytest.mark.parametrize("tokens,tables_f16", [(4095, True), (4096, True), (4500, False)])
+def test_rvq_decode_staging_rule(device, tokens, tables_f16):
+    gen = _gen(6262 + tokens)
+    tables = ref.synthetic_tables(gen, (8 * 16, 2, 256, 8), (1.0, 0.5), stage_axis=1)
+    tables = tables + 1e-3 * torch.randn(tables.shape, generator=gen)
+    codes = torch.randint(0, 256, (1, 8, tokens, 16, 2), generator=gen, dtype=torch.uint8)
+    given = tables.half() if tables_f16 else tables
+    got = jkv.closed_loop_vq._ops.rvq_decode(codes.to(device), given.to(device), depth=2, dtype=torch.float16)
+    assert torch.equal(got.cpu(), ref.frozen_decode(codes, tables, 2, torch.float16))
+
+
 # bf16 states on the grouped MFMA kernel: slabs of 64 rows, 256 per workgroup
 # pass; one row, tile and slab edges, rows that straddle batch entries, strided
 # [B,T,H,D] views, both group widths, codebooks far from unit scale
