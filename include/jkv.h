@@ -441,6 +441,16 @@ int jkv_prefill_attention_value_grad(const void* q, int64_t q_stride_b, int64_t 
                                      const void* rope_table, int64_t rope_len, float* d_value,
                                      void* workspace, int64_t workspace_bytes, jkv_stream_t stream);
 
+/* The same, with the sums rounded once to fp16 d_value [B,KVH,T,128]. */
+int jkv_prefill_attention_value_grad_f16(const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                                     int64_t q_stride_t, const void* k, int64_t k_stride_b,
+                                     int64_t k_stride_h, int64_t k_stride_t, const void* d_out,
+                                     int64_t d_stride_b, int64_t d_stride_h, int64_t d_stride_t,
+                                     const float* lse, int64_t B, int64_t QH, int64_t KVH, int64_t T,
+                                     int64_t D, const int32_t* start_positions, int64_t window,
+                                     const void* rope_table, int64_t rope_len, void* d_value,
+                                     void* workspace, int64_t workspace_bytes, jkv_stream_t stream_);
+
 /* Workspace of jkv_prefill_attention_value_grad for this geometry (bytes):
  * the runs' partial slots when there are several, then the rotated queries. */
 int64_t jkv_prefill_value_grad_workspace_bytes(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window);
@@ -471,6 +481,18 @@ int jkv_prefill_attention_backward(const void* q, int64_t q_stride_b, int64_t q_
                                    const void* rope_table, int64_t rope_len, float* d_query, float* d_key,
                                    float* d_value, void* workspace, int64_t workspace_bytes,
                                    jkv_stream_t stream);
+
+/* The same, with the fp32 sums rounded once to fp16 gradients. */
+int jkv_prefill_attention_backward_f16(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+                                   const void* k, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_t,
+                                   const void* v, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_t,
+                                   const void* out, int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_t,
+                                   const void* d_out, int64_t d_stride_b, int64_t d_stride_h,
+                                   int64_t d_stride_t, const float* lse, int64_t B, int64_t QH, int64_t KVH,
+                                   int64_t T, int64_t D, const int32_t* start_positions, int64_t window,
+                                   const void* rope_table, int64_t rope_len, void* d_query, void* d_key,
+                                   void* d_value, void* workspace, int64_t workspace_bytes,
+                                   jkv_stream_t stream_);
 
 /* Workspace of jkv_prefill_attention_backward (bytes). */
 int64_t jkv_prefill_backward_workspace_bytes(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window);

@@ -31,6 +31,7 @@
 // registers: three workgroups per CU.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "jkv_common.h"
@@ -66,6 +67,19 @@ struct ValueGradArgs {
   int64_t slot_stride;  // elements between the chunks' partial slots (0: one chunk)
   int32_t slots;        // partial slots (grid rows) of the key-block kernels
 };
+
+// element i of a result: fp32, or its fp16 rounding (the empty asm keeps the
+// fp32 rounding: the compiler would fuse the last multiply-add into the
+// conversion)
+template <bool HALF>
+__device__ __forceinline__ void put_grad(float* out, int64_t i, float v) {
+  if constexpr (HALF) {
+    asm volatile("" : "+v"(v));
+    ((_Float16*)out)[i] = (_Float16)v;
+  } else {
+    out[i] = v;
+  }
+}
 
 // The 32-row query tiles (absolute: tile t holds rows 32t..32t+31) that the
 // workgroup of key block key0 in grid row y walks, top tile first.  The rows
@@ -161,9 +175,11 @@ __device__ __forceinline__ uint32_t row_slot(int r, int j) {
 // rows with the same transposing reads that give dOᵀ to the value gradient.
 // Each wave owns KT 16-key tiles (a workgroup 64 KT keys): KT = 2 for one
 // gradient, KT = 1 for both, which keeps both sets of accumulators within
-// three waves per SIMD.
+// three waves per SIMD.  HALF: the walk's sums are the results, in fp16 (a
+// form of its own: as a run-time choice it cost the KV walk registers, 425 ->
+// 522 us at [4,32/8,2048]).
 enum WalkMode { kWalkV, kWalkK, kWalkKV };
-template <int MODE, int KT>
+template <int MODE, int KT, bool HALF>
 __device__ __forceinline__ void kv_grad_walk(const ValueGradArgs& a) {
   constexpr bool kV = MODE != kWalkK, DK = MODE != kWalkV;  // forms dV̂ / dK̂
   constexpr int kKeys = 64 * KT;                           // keys per workgroup
@@ -516,12 +532,12 @@ __device__ __forceinline__ void kv_grad_walk(const ValueGradArgs& a) {
       const int64_t key = kw0 + 16 * kt + 4 * lg + e;
       if (key >= a.T) continue;
       if constexpr (kV) {
-        float* out = a.dv + orow;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) out[key * kBD + 16 * dt + ln] = acc[iV][kt][dt][e];
+        for (int dt = 0; dt < 8; ++dt) put_grad<HALF>(a.dv, orow + key * kBD + 16 * dt + ln, acc[iV][kt][dt][e]);
       }
       if constexpr (DK) {
-        float* out = (kV ? a.dk : a.dv) + orow;
+        float* out = kV ? a.dk : a.dv;
+        const int64_t at = orow + key * kBD;
         const _Float16* tr = rope_row(p0 + key);
         const float inv = 1.0f / sqrtf((float)kBD);
 #pragma unroll
@@ -529,25 +545,28 @@ __device__ __forceinline__ void kv_grad_walk(const ValueGradArgs& a) {
           const int f = 16 * dt + ln;
           const float c = (float)tr[f], sn = (float)tr[64 + f];
           const float lo = acc[iK][kt][dt][e] * inv, hi = acc[iK][kt][dt + 4][e] * inv;
-          out[key * kBD + f] = lo * c + hi * sn;
-          out[key * kBD + 64 + f] = hi * c - lo * sn;
+          put_grad<HALF>(out, at + f, lo * c + hi * sn);
+          put_grad<HALF>(out, at + 64 + f, hi * c - lo * sn);
         }
       }
     }
 }
 
 // 168 registers: three workgroups per CU
+template <bool HALF>
 __global__ __launch_bounds__(kBThreads) __attribute__((amdgpu_waves_per_eu(3)))
 void prefill_value_grad_kernel(ValueGradArgs a) {
-  kv_grad_walk<kWalkV, 2>(a);
+  kv_grad_walk<kWalkV, 2, HALF>(a);
 }
+template <bool HALF>
 __global__ __launch_bounds__(kBThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_key_grad_kernel(ValueGradArgs a) {
-  kv_grad_walk<kWalkK, 2>(a);
+  kv_grad_walk<kWalkK, 2, HALF>(a);
 }
+template <bool HALF>
 __global__ __launch_bounds__(kBThreads) __attribute__((amdgpu_waves_per_eu(3)))
 void prefill_kv_grad_kernel(ValueGradArgs a) {
-  kv_grad_walk<kWalkKV, 1>(a);
+  kv_grad_walk<kWalkKV, 1, HALF>(a);
 }
 
 // Query gradient of the same attention, and delta = rowsum(dO * O) that the
@@ -575,8 +594,11 @@ struct QGradArgs {
   float* dq;          // [B,QH,T,D] fp32, or the run's partial slot
   _Float16* q_rot;    // [B,QH,T,D] fp16 contiguous: the rotated queries, written for the key and value legs (or null)
   int32_t heads_per_wg, row_sets, head_groups;
+  int32_t group;  // slices per run of the block order (divides an XCD's slices)
+  int32_t fold;   // blocks per XCD after which the order runs backwards (0: nowhere)
 };
 
+template <bool HALF>
 __global__ __launch_bounds__(kBThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void prefill_q_grad_kernel(QGradArgs qa_) {
   const ValueGradArgs& a = qa_.g;  // a.k: the rotated K̂_rot, contiguous [B,KVH,T,128]
@@ -589,11 +611,19 @@ void prefill_q_grad_kernel(QGradArgs qa_) {
   const int NQ = a.nq;
   const int64_t block_rows = 32 * (int64_t)RS;
   const int64_t nqb = ceil_div(a.T, block_rows);
-  const uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
+  // the forward's block order: runs of `group` (batch row, kv head, head
+  // group) slices on one XCD, longest key ranges first over the run's slices
+  // (later row blocks see more keys); where all blocks reside at once, two
+  // per CU, the second half runs backwards
+  uint32_t bid = xcd_remap(blockIdx.x, gridDim.x);
+  if (qa_.fold > 0) {
+    const uint32_t per = gridDim.x >> 3, at = bid % per, first = (uint32_t)qa_.fold;
+    if (at >= first) bid += per - 1 - at + first - at;
+  }
   const int chunk = blockIdx.y;
-  // longest key ranges first (later row blocks see more keys)
-  const int64_t qblk = nqb - 1 - (int64_t)(bid % (uint32_t)nqb);
-  const int64_t yz = bid / (uint32_t)nqb;
+  const uint32_t slices_run = (uint32_t)qa_.group * (uint32_t)nqb, in_run = bid % slices_run;
+  const int64_t qblk = nqb - 1 - (int64_t)(in_run / (uint32_t)qa_.group);
+  const int64_t yz = (int64_t)(bid / slices_run) * qa_.group + in_run % (uint32_t)qa_.group;
   const int64_t gy = a.KVH * qa_.head_groups;
   const int64_t kvh = (yz % gy) / qa_.head_groups;
   const int64_t hg = (yz % gy) % qa_.head_groups;
@@ -816,7 +846,7 @@ void prefill_q_grad_kernel(QGradArgs qa_) {
 
   // ---- 1/sqrt(D), the rotary's transpose at the row's position, store:
   // lane holds dims 16dt + ln of rows row0 + 16rg + 4lg + e ----
-  float* out = qa_.dq + (int64_t)chunk * a.slot_stride + ((b * a.QH + head) * a.T) * kBD;
+  const int64_t orow = (int64_t)chunk * a.slot_stride + ((b * a.QH + head) * a.T) * kBD;
   const float inv = 1.0f / sqrtf((float)kBD);
 #pragma unroll
   for (int rg = 0; rg < 2; ++rg)
@@ -830,16 +860,18 @@ void prefill_q_grad_kernel(QGradArgs qa_) {
         const int f = 16 * dt + ln;
         const float c = (float)tr[f], sn = (float)tr[64 + f];
         const float lo = acc[rg][dt][e] * inv, hi = acc[rg][dt + 4][e] * inv;
-        out[row * kBD + f] = lo * c + hi * sn;
-        out[row * kBD + 64 + f] = hi * c - lo * sn;
+        put_grad<HALF>(qa_.dq, orow + row * kBD + f, lo * c + hi * sn);
+        put_grad<HALF>(qa_.dq, orow + row * kBD + 64 + f, hi * c - lo * sn);
       }
     }
 }
 
 // dV̂ (or dK̂) = the sum of the partial slots of the chunks that the key's
-// block meets, in chunk order.  Rows [*, T, 128] fp32, as float4.
+// block meets, in chunk order.  Rows [*, T, 128] fp32, as float4; F16 rounds
+// the sums to fp16.
+template <bool F16>
 __global__ __launch_bounds__(256) void value_grad_reduce_kernel(const float* __restrict__ part,
-                                                                float* __restrict__ dv, int64_t n4,
+                                                                void* __restrict__ dv, int64_t n4,
                                                                 int64_t slot4, int slots, int64_t T,
                                                                 int64_t window, int keys, int64_t per) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -856,34 +888,54 @@ __global__ __launch_bounds__(256) void value_grad_reduce_kernel(const float* __r
     acc.z += v.z;
     acc.w += v.w;
   }
-  ((float4*)dv)[i] = acc;
+  if constexpr (F16) {
+    ((half4*)dv)[i] = half4{(_Float16)acc.x, (_Float16)acc.y, (_Float16)acc.z, (_Float16)acc.w};
+  } else {
+    ((float4*)dv)[i] = acc;
+  }
 }
 
 // Tiles per chunk and partial slots of the key-block kernels (blocks of
-// `keys` keys): chunks of 16 tiles, or of an eighth of the longest block's
-// rows when that is more; the slots are the most chunks one block meets.
-static void value_grad_chunks(int64_t T, int64_t window, int keys, int* chunk_tiles, int* slots);
+// `keys` keys, n = B KVH slices): chunks of 16 tiles, of an eighth of the
+// longest block's rows when that is more, or shorter where the grid is small;
+// the slots are the most chunks one block meets.
+static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, int* chunk_tiles, int* slots);
 
 // bytes of the value gradient's workspace: the chunks' partial slots (when
 // there are several), then the rotated queries [B,QH,T,128] fp16 at a
 // 256-byte boundary
 static int64_t value_grad_workspace(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window) {
   int chunk_tiles, chunks;
-  value_grad_chunks(T, window, kBKeys, &chunk_tiles, &chunks);
+  value_grad_chunks(B * KVH, T, window, kBKeys, &chunk_tiles, &chunks);
   const int64_t slots = chunks > 1 ? (int64_t)chunks * B * KVH * T * kBD * (int64_t)sizeof(float) : 0;
   return ceil_div(slots, 256) * 256 + B * QH * T * kBD * 2;
 }
 
-static void value_grad_chunks(int64_t T, int64_t window, int keys, int* chunk_tiles, int* slots) {
+static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, int* chunk_tiles, int* slots) {
   int64_t rows = (int64_t)keys - 1 + window;
   if (rows > T || rows < 0) rows = T;
   const int64_t span = ceil_div(rows, kBRows);  // tiles of the longest block (blocks start on a tile)
   int64_t per = 16;
   if (ceil_div(span, per) > 8) per = ceil_div(span, 8);
-  const int64_t all = ceil_div(ceil_div(T, kBRows), per);
-  const int64_t most = ceil_div(span - 1, per) + 1;
+  auto slots_of = [&](int64_t p) {
+    const int64_t all = ceil_div(ceil_div(T, kBRows), p);
+    const int64_t most = ceil_div(span - 1, p) + 1;
+    return all < most ? all : most;
+  };
+  // shorter chunks while a launch has fewer walks than these (a block meets
+  // about half of the slots): the longest walk is the launch's time there,
+  // against partial slots to write and sum.  us per call, 16 tiles against
+  // the chosen ones: full backward [1,32/8,777] 142 -> 94, [2,512] 127 -> 80,
+  // [2,1024] 186 -> 158; value gradient alone [1,777] 76 -> 36, [2,1024]
+  // 83 -> 57, [1,2048] 101 -> 82; [2,2048] (1,280 and 640 walks) keeps 16
+  // (442; shorter ones 450)
+  while (per > 2) {
+    const int64_t walks = n * ceil_div(T, (int64_t)keys) * (slots_of(per) + 1) / 2;
+    if (walks >= (per >= 16 ? 640 : per >= 8 ? 400 : 250)) break;
+    per = std::max<int64_t>(per / 2, 2);
+  }
   *chunk_tiles = (int)per;
-  *slots = (int)(all < most ? all : most);
+  *slots = (int)slots_of(per);
 }
 
 }  // namespace jkv
@@ -907,7 +959,8 @@ namespace jkv {
 template <int MODE>
 static int launch_kv_grad(ValueGradArgs a, int64_t D, const int64_t (&strides)[12], int nstrides,
                           const void* rope_table, float* d_out_buf, void* workspace, int64_t workspace_bytes,
-                          hipStream_t stream, const _Float16* q_rot_given = nullptr, float* d_key_buf = nullptr) {
+                          hipStream_t stream, bool half_out, const _Float16* q_rot_given = nullptr,
+                          float* d_key_buf = nullptr) {
   constexpr bool DK = MODE != kWalkV;
   constexpr int keys = MODE == kWalkKV ? 64 : kBKeys;
   constexpr int nout = MODE == kWalkKV ? 2 : 1;
@@ -943,7 +996,7 @@ static int launch_kv_grad(ValueGradArgs a, int64_t D, const int64_t (&strides)[1
   a.rope = (const _Float16*)rope_table;
   a.nq = (int32_t)NQ;
   int chunk_tiles, chunks;
-  value_grad_chunks(T, a.window, keys, &chunk_tiles, &chunks);
+  value_grad_chunks(B * KVH, T, a.window, keys, &chunk_tiles, &chunks);
   a.chunk_tiles = chunk_tiles;
   a.slots = chunks;
   const int64_t n = B * KVH * T * kBD;
@@ -978,27 +1031,70 @@ static int launch_kv_grad(ValueGradArgs a, int64_t D, const int64_t (&strides)[1
     q_rot = qr;
   }
   a.q = q_rot;  // contiguous [B,QH,T,128]
+  const dim3 walks((uint32_t)blocks, (uint32_t)chunks), threads(kBThreads);
+  // several chunks: fp32 slots, whose sum is rounded
+  const bool half_walk = half_out && chunks == 1;
+#define JKV_WALK(kernel)                                                  \
+  do {                                                                    \
+    if (half_walk) {                                                      \
+      hipLaunchKernelGGL(kernel<true>, walks, threads, 0, stream, a);     \
+    } else {                                                              \
+      hipLaunchKernelGGL(kernel<false>, walks, threads, 0, stream, a);    \
+    }                                                                     \
+  } while (0)
   if constexpr (MODE == kWalkK) {
-    hipLaunchKernelGGL(prefill_key_grad_kernel, dim3((uint32_t)blocks, (uint32_t)chunks), dim3(kBThreads), 0,
-                       stream, a);
+    JKV_WALK(prefill_key_grad_kernel);
   } else if constexpr (MODE == kWalkKV) {
-    hipLaunchKernelGGL(prefill_kv_grad_kernel, dim3((uint32_t)blocks, (uint32_t)chunks), dim3(kBThreads), 0,
-                       stream, a);
+    JKV_WALK(prefill_kv_grad_kernel);
   } else {
-    hipLaunchKernelGGL(prefill_value_grad_kernel, dim3((uint32_t)blocks, (uint32_t)chunks), dim3(kBThreads), 0,
-                       stream, a);
+    JKV_WALK(prefill_value_grad_kernel);
   }
+#undef JKV_WALK
   JKV_CHECK_LAUNCH();
   if (chunks > 1) {
     const int64_t n4 = n / 4;
     for (int o = 0; o < nout; ++o) {
-      hipLaunchKernelGGL(value_grad_reduce_kernel, dim3((uint32_t)ceil_div(n4, 256)), dim3(256), 0, stream,
-                         (const float*)((unsigned char*)workspace + o * slot_bytes), o == 0 ? d_out_buf : d_key_buf,
-                         n4, n4, chunks, T, a.window, keys, (int64_t)chunk_tiles);
+      const float* part = (const float*)((unsigned char*)workspace + o * slot_bytes);
+      void* to = o == 0 ? d_out_buf : d_key_buf;
+      const dim3 grid((uint32_t)ceil_div(n4, 256));
+      if (half_out) {
+        hipLaunchKernelGGL(value_grad_reduce_kernel<true>, grid, dim3(256), 0, stream, part, to, n4, n4, chunks, T,
+                           a.window, keys, (int64_t)chunk_tiles);
+      } else {
+        hipLaunchKernelGGL(value_grad_reduce_kernel<false>, grid, dim3(256), 0, stream, part, to, n4, n4, chunks, T,
+                           a.window, keys, (int64_t)chunk_tiles);
+      }
       JKV_CHECK_LAUNCH();
     }
   }
   return JKV_OK;
+}
+
+}  // namespace jkv
+
+namespace jkv {
+
+static int value_grad(bool half_out, const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                                     int64_t q_stride_t, const void* k, int64_t k_stride_b,
+                                     int64_t k_stride_h, int64_t k_stride_t, const void* d_out,
+                                     int64_t d_stride_b, int64_t d_stride_h, int64_t d_stride_t,
+                                     const float* lse, int64_t B, int64_t QH, int64_t KVH, int64_t T,
+                                     int64_t D, const int32_t* start_positions, int64_t window,
+                                     const void* rope_table, int64_t rope_len, void* d_value,
+                                     void* workspace, int64_t workspace_bytes, jkv_stream_t stream_) {
+  ValueGradArgs a = {};
+  a.q = (const _Float16*)q; a.qsb = q_stride_b; a.qsh = q_stride_h; a.qst = q_stride_t;
+  a.k = (const _Float16*)k; a.ksb = k_stride_b; a.ksh = k_stride_h; a.kst = k_stride_t;
+  a.dout = (const _Float16*)d_out; a.dsb = d_stride_b; a.dsh = d_stride_h; a.dst = d_stride_t;
+  a.lse = lse;
+  a.B = B; a.QH = QH; a.KVH = KVH; a.T = T;
+  a.start = start_positions;
+  a.window = window;
+  a.rope_len = rope_len;
+  const int64_t strides[12] = {q_stride_b, q_stride_h, q_stride_t, k_stride_b, k_stride_h, k_stride_t,
+                               d_stride_b, d_stride_h, d_stride_t, 0, 0, 0};
+  return launch_kv_grad<kWalkV>(a, D, strides, 9, rope_table, (float*)d_value, workspace, workspace_bytes,
+                                (hipStream_t)stream_, half_out);
 }
 
 }  // namespace jkv
@@ -1013,20 +1109,18 @@ int jkv_prefill_attention_value_grad(const void* q, int64_t q_stride_b, int64_t 
                                      int64_t D, const int32_t* start_positions, int64_t window,
                                      const void* rope_table, int64_t rope_len, float* d_value,
                                      void* workspace, int64_t workspace_bytes, jkv_stream_t stream_) {
-  using namespace jkv;
-  ValueGradArgs a = {};
-  a.q = (const _Float16*)q; a.qsb = q_stride_b; a.qsh = q_stride_h; a.qst = q_stride_t;
-  a.k = (const _Float16*)k; a.ksb = k_stride_b; a.ksh = k_stride_h; a.kst = k_stride_t;
-  a.dout = (const _Float16*)d_out; a.dsb = d_stride_b; a.dsh = d_stride_h; a.dst = d_stride_t;
-  a.lse = lse;
-  a.B = B; a.QH = QH; a.KVH = KVH; a.T = T;
-  a.start = start_positions;
-  a.window = window;
-  a.rope_len = rope_len;
-  const int64_t strides[12] = {q_stride_b, q_stride_h, q_stride_t, k_stride_b, k_stride_h, k_stride_t,
-                               d_stride_b, d_stride_h, d_stride_t, 0, 0, 0};
-  return launch_kv_grad<kWalkV>(a, D, strides, 9, rope_table, d_value, workspace, workspace_bytes,
-                                (hipStream_t)stream_);
+  return jkv::value_grad(false, q, q_stride_b, q_stride_h, q_stride_t, k, k_stride_b, k_stride_h, k_stride_t, d_out, d_stride_b, d_stride_h, d_stride_t, lse, B, QH, KVH, T, D, start_positions, window, rope_table, rope_len, d_value, workspace, workspace_bytes, stream_);
+}
+
+int jkv_prefill_attention_value_grad_f16(const void* q, int64_t q_stride_b, int64_t q_stride_h,
+                                     int64_t q_stride_t, const void* k, int64_t k_stride_b,
+                                     int64_t k_stride_h, int64_t k_stride_t, const void* d_out,
+                                     int64_t d_stride_b, int64_t d_stride_h, int64_t d_stride_t,
+                                     const float* lse, int64_t B, int64_t QH, int64_t KVH, int64_t T,
+                                     int64_t D, const int32_t* start_positions, int64_t window,
+                                     const void* rope_table, int64_t rope_len, void* d_value,
+                                     void* workspace, int64_t workspace_bytes, jkv_stream_t stream_) {
+  return jkv::value_grad(true, q, q_stride_b, q_stride_h, q_stride_t, k, k_stride_b, k_stride_h, k_stride_t, d_out, d_stride_b, d_stride_h, d_stride_t, lse, B, QH, KVH, T, D, start_positions, window, rope_table, rope_len, d_value, workspace, workspace_bytes, stream_);
 }
 
 int jkv_prefill_attention_key_grad(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
@@ -1053,15 +1147,15 @@ int jkv_prefill_attention_key_grad(const void* q, int64_t q_stride_b, int64_t q_
   const int64_t strides[12] = {q_stride_b, q_stride_h, q_stride_t, k_stride_b, k_stride_h, k_stride_t,
                                v_stride_b, v_stride_h, v_stride_t, d_stride_b, d_stride_h, d_stride_t};
   return launch_kv_grad<kWalkK>(a, D, strides, 12, rope_table, d_key, workspace, workspace_bytes,
-                                (hipStream_t)stream_);
+                                (hipStream_t)stream_, false);
 }
 
 int64_t jkv_prefill_backward_workspace_bytes(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window) {
   using namespace jkv;
   if (B <= 0 || QH <= 0 || KVH <= 0 || T <= 0 || window < 1) return 0;
   int chunk_tiles, chunks, chunks64;
-  value_grad_chunks(T, window, kBKeys, &chunk_tiles, &chunks);
-  value_grad_chunks(T, window, 64, &chunk_tiles, &chunks64);
+  value_grad_chunks(B * KVH, T, window, kBKeys, &chunk_tiles, &chunks);
+  value_grad_chunks(B * KVH, T, window, 64, &chunk_tiles, &chunks64);
   const int64_t delta = ceil_div(B * QH * T * (int64_t)sizeof(float), 256) * 256;
   const int64_t k_rot = ceil_div(B * KVH * T * kBD * 2, 256) * 256;
   const int64_t q_rot = ceil_div(B * QH * T * kBD * 2, 256) * 256;
@@ -1075,18 +1169,22 @@ int64_t jkv_prefill_backward_workspace_bytes(int64_t B, int64_t QH, int64_t KVH,
   return delta + k_rot + q_rot + area;
 }
 
-int jkv_prefill_attention_backward(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+}  // extern "C"
+
+namespace jkv {
+
+static int backward(bool half_out, const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
                                    const void* k, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_t,
                                    const void* v, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_t,
                                    const void* out, int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_t,
                                    const void* d_out, int64_t d_stride_b, int64_t d_stride_h,
                                    int64_t d_stride_t, const float* lse, int64_t B, int64_t QH, int64_t KVH,
                                    int64_t T, int64_t D, const int32_t* start_positions, int64_t window,
-                                   const void* rope_table, int64_t rope_len, float* d_query, float* d_key,
-                                   float* d_value, void* workspace, int64_t workspace_bytes,
+                                   const void* rope_table, int64_t rope_len, void* d_query_, void* d_key_,
+                                   void* d_value_, void* workspace, int64_t workspace_bytes,
                                    jkv_stream_t stream_) {
-  using namespace jkv;
   hipStream_t stream = (hipStream_t)stream_;
+  float *d_query = (float*)d_query_, *d_key = (float*)d_key_, *d_value = (float*)d_value_;
   JKV_CHECK_ARG(D == kBD, "prefill gradients support head_dim 128, got %lld", (long long)D);
   JKV_CHECK_ARG(B >= 0 && QH > 0 && KVH > 0 && T >= 0 && QH % KVH == 0, "invalid prefill geometry");
   JKV_CHECK_ARG(window >= 1, "window must be positive");
@@ -1160,7 +1258,22 @@ int jkv_prefill_attention_backward(const void* q, int64_t q_stride_b, int64_t q_
     const int64_t nqb = ceil_div(T, 32 * (int64_t)qa.row_sets);
     const int64_t blocks = nqb * KVH * qa.head_groups * B;
     JKV_CHECK_ARG(blocks < ((int64_t)1 << 31), "prefill grid too large");
-    hipLaunchKernelGGL(prefill_q_grad_kernel, dim3((uint32_t)blocks), dim3(kBThreads), 0, stream, qa);
+    const int64_t slices = KVH * qa.head_groups * B;
+    qa.group = 1;
+    qa.fold = 0;
+    if (slices % 8 == 0) {
+      // as many of an XCD's slices as leave their K/V (512 bytes per token)
+      // in half of its 4 MiB L2, as in the forward
+      const int64_t per = slices / 8, cap = std::max<int64_t>(1, (2 << 20) / (T * 512));
+      for (int64_t i = 1; i <= per && i <= cap; ++i)
+        if (per % i == 0) qa.group = (int32_t)i;
+      if (blocks > 256 && blocks <= 512) qa.fold = 32;
+    }
+    if (d_query != nullptr && half_out) {
+      hipLaunchKernelGGL(prefill_q_grad_kernel<true>, dim3((uint32_t)blocks), dim3(kBThreads), 0, stream, qa);
+    } else {
+      hipLaunchKernelGGL(prefill_q_grad_kernel<false>, dim3((uint32_t)blocks), dim3(kBThreads), 0, stream, qa);
+    }
     JKV_CHECK_LAUNCH();
   }
   // the key and value legs read the rotated queries the query leg wrote;
@@ -1169,17 +1282,48 @@ int jkv_prefill_attention_backward(const void* q, int64_t q_stride_b, int64_t q_
   const bool q_leg = d_query || d_key;
   if (d_key && d_value) {
     const int rc = launch_kv_grad<kWalkKV>(g, D, strides, 12, rope_table, d_value, slots, slot_bytes, stream,
-                                           q_rot, d_key);
+                                           half_out, q_rot, d_key);
     if (rc != JKV_OK) return rc;
   } else if (d_key) {
-    const int rc = launch_kv_grad<kWalkK>(g, D, strides, 12, rope_table, d_key, slots, slot_bytes, stream, q_rot);
+    const int rc = launch_kv_grad<kWalkK>(g, D, strides, 12, rope_table, d_key, slots, slot_bytes, stream,
+                                          half_out, q_rot);
     if (rc != JKV_OK) return rc;
   } else if (d_value) {
     const int rc = launch_kv_grad<kWalkV>(g, D, strides, 12, rope_table, d_value, slots, slot_bytes, stream,
-                                          q_leg ? q_rot : nullptr);
+                                          half_out, q_leg ? q_rot : nullptr);
     if (rc != JKV_OK) return rc;
   }
   return JKV_OK;
+}
+
+}  // namespace jkv
+
+extern "C" {
+
+int jkv_prefill_attention_backward(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+                                   const void* k, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_t,
+                                   const void* v, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_t,
+                                   const void* out, int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_t,
+                                   const void* d_out, int64_t d_stride_b, int64_t d_stride_h,
+                                   int64_t d_stride_t, const float* lse, int64_t B, int64_t QH, int64_t KVH,
+                                   int64_t T, int64_t D, const int32_t* start_positions, int64_t window,
+                                   const void* rope_table, int64_t rope_len, float* d_query, float* d_key,
+                                   float* d_value, void* workspace, int64_t workspace_bytes,
+                                   jkv_stream_t stream_) {
+  return jkv::backward(false, q, q_stride_b, q_stride_h, q_stride_t, k, k_stride_b, k_stride_h, k_stride_t, v, v_stride_b, v_stride_h, v_stride_t, out, o_stride_b, o_stride_h, o_stride_t, d_out, d_stride_b, d_stride_h, d_stride_t, lse, B, QH, KVH, T, D, start_positions, window, rope_table, rope_len, d_query, d_key, d_value, workspace, workspace_bytes, stream_);
+}
+
+int jkv_prefill_attention_backward_f16(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_t,
+                                   const void* k, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_t,
+                                   const void* v, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_t,
+                                   const void* out, int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_t,
+                                   const void* d_out, int64_t d_stride_b, int64_t d_stride_h,
+                                   int64_t d_stride_t, const float* lse, int64_t B, int64_t QH, int64_t KVH,
+                                   int64_t T, int64_t D, const int32_t* start_positions, int64_t window,
+                                   const void* rope_table, int64_t rope_len, void* d_query, void* d_key,
+                                   void* d_value, void* workspace, int64_t workspace_bytes,
+                                   jkv_stream_t stream_) {
+  return jkv::backward(true, q, q_stride_b, q_stride_h, q_stride_t, k, k_stride_b, k_stride_h, k_stride_t, v, v_stride_b, v_stride_h, v_stride_t, out, o_stride_b, o_stride_h, o_stride_t, d_out, d_stride_b, d_stride_h, d_stride_t, lse, B, QH, KVH, T, D, start_positions, window, rope_table, rope_len, d_query, d_key, d_value, workspace, workspace_bytes, stream_);
 }
 
 }  // extern "C"

@@ -138,6 +138,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "jkv_f32_to_f16": (ctypes.c_int, [_vp, _vp, _i64, _vp]),
 }
 
+# the fp16-output forms take the same arguments
+for _name in ("jkv_prefill_attention_value_grad", "jkv_prefill_attention_backward"):
+    SIGNATURES[_name + "_f16"] = SIGNATURES[_name]
+
 _lib: ctypes.CDLL | None = None
 
 

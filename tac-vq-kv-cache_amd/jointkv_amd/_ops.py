@@ -830,6 +830,14 @@ def prefill_attention_codes(
     return out
 
 
+def _grad_entry(lib, name: str, dtype: torch.dtype):
+    if dtype == torch.float32:
+        return getattr(lib, name)
+    if dtype == torch.float16:
+        return getattr(lib, name + "_f16")
+    raise ValueError("prefill gradients are fp32 or fp16")
+
+
 def prefill_attention_backward(
     q: torch.Tensor,
     key: torch.Tensor,
@@ -843,10 +851,12 @@ def prefill_attention_backward(
     rope_theta: float,
     max_position: int,
     need: tuple[bool, bool, bool] = (True, True, True),
+    dtype: torch.dtype = torch.float32,
 ):
     """Gradients of :func:`prefill_attention` with respect to the pre-RoPE
-    ``q``, ``key`` and ``value`` (fp32; ``None`` where ``need`` is False),
-    from the forward's ``out`` and ``lse`` and the output gradient."""
+    ``q``, ``key`` and ``value`` (``None`` where ``need`` is False), from the
+    forward's ``out`` and ``lse`` and the output gradient: the fp32 sums, or
+    with ``dtype=torch.float16`` their rounding."""
 
     if key.shape != value.shape:
         raise ValueError("prefill query/key/value geometry differs")
@@ -858,13 +868,13 @@ def prefill_attention_backward(
     if lse.dtype != torch.float32 or lse.shape != (batch, qheads, tokens) or not lse.is_contiguous():
         raise ValueError("lse must be a contiguous fp32 [B,QH,T] tensor")
     table = rope_table(device, rope_theta, int(max_position) + 1)
-    grads = [torch.empty(shape, dtype=torch.float32, device=device) if want else None
+    grads = [torch.empty(shape, dtype=dtype, device=device) if want else None
              for want, shape in zip(need, ((batch, qheads, tokens, 128), (batch, kvheads, tokens, 128),
                                            (batch, kvheads, tokens, 128)))]
     lib = _lib.load()
     ws_bytes = _lib.workspace_bytes("jkv_prefill_backward_workspace_bytes", batch, qheads, kvheads, tokens, int(window))
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
-    code = lib.jkv_prefill_attention_backward(
+    code = _grad_entry(lib, "jkv_prefill_attention_backward", dtype)(
         q.data_ptr(), *q.stride()[:3], key.data_ptr(), *key.stride()[:3], value.data_ptr(), *value.stride()[:3],
         out.data_ptr(), *out.stride()[:3], d_out.data_ptr(), *d_out.stride()[:3], lse.data_ptr(),
         batch, qheads, kvheads, tokens, 128, start_positions.data_ptr(), int(window), table.data_ptr(),
@@ -885,10 +895,11 @@ def prefill_attention_value_grad(
     window: int,
     rope_theta: float,
     max_position: int,
+    dtype: torch.dtype = torch.float32,
 ) -> torch.Tensor:
     """Gradient of :func:`prefill_attention` with respect to ``value``:
-    fp32 ``[B,KVH,T,128]`` from ``d_out`` (fp16 ``[B,QH,T,128]``) and the
-    forward's ``lse``."""
+    ``[B,KVH,T,128]`` fp32 (or its fp16 rounding, ``dtype``) from ``d_out``
+    (fp16 ``[B,QH,T,128]``) and the forward's ``lse``."""
 
     device, (q, key, d_out), start_positions, (batch, qheads, kvheads, tokens) = _prefill_operands(
         q, key, d_out, start_positions, "output gradient")
@@ -897,11 +908,11 @@ def prefill_attention_value_grad(
     if lse.dtype != torch.float32 or lse.shape != (batch, qheads, tokens) or not lse.is_contiguous():
         raise ValueError("lse must be a contiguous fp32 [B,QH,T] tensor")
     table = rope_table(device, rope_theta, int(max_position) + 1)
-    d_value = torch.empty((batch, kvheads, tokens, 128), dtype=torch.float32, device=device)
+    d_value = torch.empty((batch, kvheads, tokens, 128), dtype=dtype, device=device)
     lib = _lib.load()
     ws_bytes = _lib.workspace_bytes("jkv_prefill_value_grad_workspace_bytes", batch, qheads, kvheads, tokens, int(window))
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
-    code = lib.jkv_prefill_attention_value_grad(
+    code = _grad_entry(lib, "jkv_prefill_attention_value_grad", dtype)(
         q.data_ptr(), *q.stride()[:3], key.data_ptr(), *key.stride()[:3], d_out.data_ptr(),
         *d_out.stride()[:3], lse.data_ptr(), batch, qheads, kvheads, tokens, 128,
         start_positions.data_ptr(), int(window), table.data_ptr(), int(table.shape[0]),

@@ -193,16 +193,13 @@ class _PrefillAttention(torch.autograd.Function):
         if need_q or need_k:
             dq, dk, dv = _ops.prefill_attention_backward(
                 query, key, value, out, d_out, lse, starts, window=window, rope_theta=rope_theta,
-                max_position=top, need=(need_q, need_k, need_v))
+                max_position=top, need=(need_q, need_k, need_v), dtype=query.dtype)
         else:
             dq = dk = None
             dv = _ops.prefill_attention_value_grad(query, key, d_out, lse, starts, window=window,
-                                                   rope_theta=rope_theta, max_position=top)
-        # each input's dtype, as SDPA's backward returns it (fp32 sums, one rounding)
-        return (dq.to(query.dtype) if dq is not None else None,
-                dk.to(key.dtype) if dk is not None else None,
-                dv.to(value.dtype) if (dv is not None and need_v) else None,
-                None, None, None, None)
+                                                   rope_theta=rope_theta, max_position=top, dtype=value.dtype)
+        # in the inputs' fp16, as SDPA's backward returns them (fp32 sums, one rounding)
+        return dq, dk, dv if need_v else None, None, None, None, None
 
 
 def prefill_attention_from_codes(

@@ -141,6 +141,43 @@ def test_key_grad_entry_matches_backward_key_leg(device, batch, qh, kvh, tokens,
     assert err <= 1e-4 * scale + 1e-6
 
 
+# chunks of 2, 4, 8 and 16 query tiles (by the grid's size), one chunk written
+# without slots, folded query blocks; the fp16 forms are the fp32 sums rounded
+# once, so they must equal them cast
+@pytest.mark.parametrize("batch,qh,kvh,tokens,window", [
+    (1, 8, 2, 40, 4096),       # one chunk of two tiles
+    (2, 8, 2, 331, 100),       # chunks of two tiles, window binds
+    (4, 32, 8, 512, 4096),     # four tiles; 512 query blocks, folded
+    (2, 32, 8, 1000, 4096),    # eight tiles, ragged
+    (32, 8, 8, 200, 4096),     # sixteen tiles: one chunk, no slots
+])
+def test_backward_chunk_rule_and_fp16_outputs(device, batch, qh, kvh, tokens, window):
+    print(f"backward chunks B={batch} QH={qh} KVH={kvh} T={tokens} win={window}", flush=True)
+    q, k, v, d = _case(2100 + tokens, batch, qh, kvh, tokens)
+    qd, kd, vd, dd = (t.to(device) for t in (q, k, v, d))
+    st = torch.zeros(batch, dtype=torch.int32, device=device)
+    kw = dict(window=window, rope_theta=10000.0, max_position=tokens - 1)
+    lse = torch.empty(batch, qh, tokens, dtype=torch.float32, device=device)
+    out = _ops.prefill_attention(qd, kd, vd, st, lse=lse, **kw)
+    wide = _ops.prefill_attention_backward(qd, kd, vd, out, dd, lse, st, **kw)
+    for need in ((True, True, True), (True, False, False), (False, True, False), (True, False, True)):
+        half = _ops.prefill_attention_backward(qd, kd, vd, out, dd, lse, st, need=need, dtype=torch.float16, **kw)
+        full = _ops.prefill_attention_backward(qd, kd, vd, out, dd, lse, st, need=need, **kw)
+        for a, b in zip(half, full):
+            assert (a is None) == (b is None) and (a is None or torch.equal(a, b.half()))
+    dv16 = _ops.prefill_attention_value_grad(qd, kd, dd, lse, st, dtype=torch.float16, **kw)
+    dv32 = _ops.prefill_attention_value_grad(qd, kd, dd, lse, st, **kw)
+    assert torch.equal(dv16, dv32.half())
+    for b in sorted({0, batch - 1}):
+        one = slice(b, b + 1)
+        dq_ref, dk_ref = ref.prefill_qk_grad(q[one], k[one], v[one], d[one], (0,), window=window)
+        dv_ref = ref.prefill_value_grad(q[one], k[one], v[one], d[one], (0,), window=window)
+        for name, got, want in zip(("dq", "dk", "dv", "dv alone"), (*wide, dv32), (dq_ref, dk_ref, dv_ref, dv_ref)):
+            scale = float(want.abs().max())
+            err = float((got[one].cpu().float() - want).abs().max())
+            assert err <= DV_RTOL * scale + 1e-3, f"{name} row {b}: max abs error {err} (scale {scale})"
+
+
 @pytest.mark.parametrize("batch,qh,kvh,tokens,starts,window", [
     (2, 8, 2, 300, (0, 40), 4096),      # GQA 4, ragged tiles, two start positions
     (1, 32, 8, 200, (0,), 64),          # Mistral heads, window binds
