@@ -200,7 +200,7 @@ __device__ __forceinline__ uint32_t stage_code(const uint32_t (&cw)[SS / 4], int
   return __builtin_amdgcn_ubfe(cw[s >> 2], 8u * (uint32_t)(s & 3), 8u);
 }
 
-// SS: the stage count of full-vector codebooks (D = 128) when it is 16 or
+// SS: the stage count of full-vector codebooks (D = 128) when it is 8, 16 or
 // 32, else 0 (a.S at run time).
 template <int D, int NQ, int SS>
 __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
@@ -263,9 +263,17 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
     }
   }
   // ---- the split's code records into LDS, 16-byte chunks, one pass ----
-  const bool codes_in_lds = D != 0 && code_bytes <= kMaxCodeBytes && (code_bytes % 16) == 0 &&
-                            code_bytes * kTok <= kRecLds;
-  if (codes_in_lds) {
+  const bool codes_in_lds = SS == 8 || (D != 0 && code_bytes <= kMaxCodeBytes && (code_bytes % 16) == 0 &&
+                                        code_bytes * kTok <= kRecLds);
+  if constexpr (SS == 8) {
+    // eight-byte records: one piece each
+    const int64_t kbase = b * a.csb + kvh * a.csh;
+    for (int j = tid; j < ntok; j += 256) {
+      const int64_t off = kbase + ((t0 + j) % a.cap) * 8;
+      *(uint2*)(kc_lds + j * 8) = *(const uint2*)(a.kc + off);
+      *(uint2*)(vc_lds + j * 8) = *(const uint2*)(a.vc + off);
+    }
+  } else if (codes_in_lds) {
     const int per_tok = (int)(code_bytes / 16);
     const int64_t kbase = b * a.csb + kvh * a.csh;
     for (int idx = tid; idx < ntok * per_tok; idx += blockDim.x) {
@@ -389,7 +397,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
           tile_scores(tile, cur);
         }
       } else {
-        // full-vector codebooks with 16 or 32 stages: each chunk is the fp32
+        // full-vector codebooks with 8, 16 or 32 stages: each chunk is the fp32
         // stage sum in stage order rounded to fp16; no tile runs ahead (the
         // slice loads in flight fill the register budget)
         const __amdgpu_buffer_rsrc_t krsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -491,7 +499,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
       }
     };
     if constexpr (SS != 0) {
-      // full-vector codebooks with 16 or 32 stages: two tokens per gather_sum
+      // full-vector codebooks with 8, 16 or 32 stages: two tokens per gather_sum
       // (the slice loads in flight fill the register budget), the products in
       // token order as below
       const __amdgpu_buffer_rsrc_t vrsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -1720,11 +1728,18 @@ static bool packed_lds_ok(const void* k_codes, const void* v_codes, int64_t code
 }
 
 // The L2 split kernel, with the full-vector stage count as a template
-// argument where it is 16 or 32 (R16 / R32 codecs).
+// argument where it is 8, 16 or 32 (R8 / R16 / R32 codecs): eight stages at
+// batch 8, 32 query and 8 KV heads, 3,000 tokens took 114 us per call at run
+// time (one slice in flight per add, half lines in K) and take 40; batch 1,
+// 1,000 tokens 82 -> 22.
 template <int D, int NQ>
 static void launch_split(const DecodeArgs& a, hipStream_t stream) {
   const dim3 grid((uint32_t)(a.B * a.KVH * a.n_splits));
   if constexpr (D == 128) {
+    if (a.S == 8) {
+      hipLaunchKernelGGL((decode_split_kernel<D, NQ, 8>), grid, dim3(256), 0, stream, a);
+      return;
+    }
     if (a.S == 16) {
       hipLaunchKernelGGL((decode_split_kernel<D, NQ, 16>), grid, dim3(256), 0, stream, a);
       return;

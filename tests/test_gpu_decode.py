@@ -90,6 +90,22 @@ def test_decode_split_rule(device, batch, qh, kvh, groups, stages, d, lengths, w
         assert err <= ATOL, f"row {b} length {lengths[b]}: {err}"
 
 
+# eight full-vector stages (eight-byte records): ragged tiles, a ring that
+# wraps, one query head per kv head and GQA 8
+@pytest.mark.parametrize("batch,qh,kvh,length,window,cap", [
+    (1, 8, 2, 333, 4096, 4096), (2, 32, 8, 700, 256, 301), (1, 2, 2, 1, 64, 64), (1, 16, 2, 257, 512, 512)])
+def test_decode_eight_full_vector_stages(device, batch, qh, kvh, length, window, cap):
+    print(f"decode R8 B={batch} QH={qh} KVH={kvh} len={length} win={window} cap={cap}", flush=True)
+    q, kc, vc, kt, vt = _case(length + qh, batch, qh, kvh, 1, 8, 128, length, cap)
+    out = jkv.decode_attention(
+        q.to(device), kc.to(device), vc.to(device), kt.half().to(device), vt.half().to(device),
+        torch.full((batch,), length, dtype=torch.int32, device=device), window=window,
+    )
+    expect = _expect(q, kc, vc, kt, vt, length, window, cap)
+    err = float((out.cpu().float() - expect.float()).abs().max())
+    assert err <= ATOL, f"max abs error {err}"
+
+
 @pytest.mark.parametrize("batch,qh,kvh,stages,lengths,window,cap", [
     (2, 32, 8, 2, (4096, 4096), 4096, 4096),    # config 4 geometry: the new token closes split 2
     (3, 8, 2, 2, (1, 257, 5000), 4096, 4096),   # first token; chunk 1's first key; ring wrap
