@@ -163,7 +163,8 @@ __global__ __launch_bounds__(256) void nearest_f32_kernel(NearestArgs a) {
 // Bound: the fp32 matrix rate (64 cycles per product, 2 waves per SIMD); LDS
 // reads are 4 bytes per cycle and SIMD.  [8,8192,128] against 256 codewords:
 // 186 us on nearest_f32_kernel (23 TFLOP/s, bound by its LDS reads),
-// 43 us here (27 us of products; the rows' load and the table's staging lead).
+// 41 us here (27 us of products; the rows' load leads, and the distances fold
+// while both waves of a SIMD wait).
 // Pitch 132 floats puts eight consecutive codewords' 16-byte pieces in
 // distinct banks.
 static const int kNmThreads = 512;
@@ -191,20 +192,61 @@ __global__ __launch_bounds__(kNmThreads) void nearest_mfma_kernel(NearestArgs a)
   const int64_t row = ((int64_t)blockIdx.x * kTiles + tile) * 32 + j;
   const int64_t at = row < a.N ? row : a.N - 1;  // rows past N repeat the last
 
+  // the table in halves of four chunks (zero rows past K), 16 bytes per thread
+  // and load, eight in flight: the first ahead of the rows, the second behind
+  // them
+  const float4* csrc = (const float4*)(a.tables + h * a.K * 128);
+  float4 piece[8];
+  auto fetch = [&](int part_of) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int i = 4096 * part_of + kNmThreads * q + tid;
+      piece[q] = (float4){0.f, 0.f, 0.f, 0.f};
+      if ((i >> 5) < K) piece[q] = csrc[i];
+    }
+  };
+  auto put = [&](int part_of) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int i = 4096 * part_of + kNmThreads * q + tid;
+      *(float4*)(cs + (i >> 5) * kNmPitch + 4 * (i & 31)) = piece[q];
+    }
+  };
+  // |c|^2 of codewords from .. from + n (+inf past K)
+  auto norms = [&](int from, int n) {
+    if (tid >= n) return;
+    float acc = __builtin_inff();
+    if (from + tid < K) {
+      acc = 0.f;
+      const float* c = cs + (from + tid) * kNmPitch;
+#pragma unroll 8
+      for (int q = 0; q < 128; q += 4) {
+        const float4 v = *(const float4*)(c + q);
+        acc = fmaf(v.x, v.x, acc);
+        acc = fmaf(v.y, v.y, acc);
+        acc = fmaf(v.z, v.z, acc);
+        acc = fmaf(v.w, v.w, acc);
+      }
+    }
+    s_cc[from + tid] = acc;
+  };
+  fetch(0);
   // this lane's half of its row: dims 8m + 4 hf .. +3
   const float4* xsrc = (const float4*)(a.states + (h * a.N + at) * 128) + hf;
   float4 x[16];
 #pragma unroll
   for (int m = 0; m < 16; ++m) x[m] = xsrc[2 * m];
-
-  // the table, zero rows past K (up to a whole chunk), 16 bytes per thread
-  const float4* csrc = (const float4*)(a.tables + h * a.K * 128);
-  for (int i = tid; i < chunks * 32 * 32; i += kNmThreads) {
-    const int r = i >> 5, q = i & 31;
-    float4 v = {0.f, 0.f, 0.f, 0.f};
-    if (r < K) v = csrc[i];
-    *(float4*)(cs + r * kNmPitch + 4 * q) = v;
-  }
+  put(0);
+  // up to two waves to a row tile, each wave's pairs of chunks lie within the
+  // halves: the second half's loads fly during the first half's products
+  // ([8,8192] 47.2 -> 45.5 us per launch, [8,1500] 17.5 -> 16.2 against one
+  // staging loop, 16 loads one after the other, ahead of everything)
+  constexpr bool kHalves = SPLIT <= 2;
+  const bool second = chunks > 4;
+  if (second) fetch(1);
+  if (!kHalves && second) put(1);
+  __syncthreads();
+  norms(0, kHalves ? 128 : 256);
   float xx = 0.f;
 #pragma unroll
   for (int m = 0; m < 16; ++m) {
@@ -215,66 +257,64 @@ __global__ __launch_bounds__(kNmThreads) void nearest_mfma_kernel(NearestArgs a)
   }
   xx += __shfl_xor(xx, 32, 64);
   __syncthreads();
-  if (tid < chunks * 32) {
-    float acc = __builtin_inff();
-    if (tid < K) {
-      acc = 0.f;
-      const float* c = cs + tid * kNmPitch;
-      for (int q = 0; q < 128; q += 4) {
-        const float4 v = *(const float4*)(c + q);
-        acc = fmaf(v.x, v.x, acc);
-        acc = fmaf(v.y, v.y, acc);
-        acc = fmaf(v.z, v.z, acc);
-        acc = fmaf(v.w, v.w, acc);
-      }
-    }
-    s_cc[tid] = acc;
-  }
-  __syncthreads();
 
   float best = __builtin_inff();
   int bidx = 0;
-  // chunks part, part + SPLIT, ...: two at a time
-  for (int c0 = part; c0 < chunks; c0 += 2 * SPLIT) {
-    const int c1 = c0 + SPLIT;
-    const bool two = c1 < chunks;
-    const float* ap0 = cs + (32 * c0 + j) * kNmPitch + 4 * hf;
-    const float* ap1 = two ? cs + (32 * c1 + j) * kNmPitch + 4 * hf : ap0;
-    float16v acc0 = {}, acc1 = {};
+  // chunks c0, c0 + SPLIT, ... below end: two at a time
+  auto search = [&](int c0, int end) {
+    for (; c0 < end; c0 += 2 * SPLIT) {
+      const int c1 = c0 + SPLIT;
+      const bool two = c1 < chunks;
+      const float* ap0 = cs + (32 * c0 + j) * kNmPitch + 4 * hf;
+      const float* ap1 = two ? cs + (32 * c1 + j) * kNmPitch + 4 * hf : ap0;
+      float16v acc0 = {}, acc1 = {};
 #pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      const float4 a0 = *(const float4*)(ap0 + 8 * m);
-      const float4 a1 = *(const float4*)(ap1 + 8 * m);
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, x[m].x, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, x[m].x, acc1, 0, 0, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, x[m].y, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, x[m].y, acc1, 0, 0, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, x[m].z, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, x[m].z, acc1, 0, 0, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, x[m].w, acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, x[m].w, acc1, 0, 0, 0);
-    }
-    // element el of lane (hf, j) is codeword 8 (el / 4) + 4 hf + el % 4 of the
-    // chunk: indices rise within the lane, so strict < keeps the first of
-    // equal distances
-    auto fold = [&](int c, const float16v& acc) {
+      for (int m = 0; m < 16; ++m) {
+        const float4 a0 = *(const float4*)(ap0 + 8 * m);
+        const float4 a1 = *(const float4*)(ap1 + 8 * m);
+        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.x, x[m].x, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.x, x[m].x, acc1, 0, 0, 0);
+        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.y, x[m].y, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.y, x[m].y, acc1, 0, 0, 0);
+        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.z, x[m].z, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.z, x[m].z, acc1, 0, 0, 0);
+        acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.w, x[m].w, acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.w, x[m].w, acc1, 0, 0, 0);
+      }
+      // element el of lane (hf, j) is codeword 8 (el / 4) + 4 hf + el % 4 of the
+      // chunk: indices rise within the lane, so strict < keeps the first of
+      // equal distances
+      auto fold = [&](int c, const float16v& acc) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k0 = 32 * c + 8 * q + 4 * hf;
-        const float4 cc = *(const float4*)(s_cc + k0);
-        const float cv[4] = {cc.x, cc.y, cc.z, cc.w};
+        for (int q = 0; q < 4; ++q) {
+          const int k0 = 32 * c + 8 * q + 4 * hf;
+          const float4 cc = *(const float4*)(s_cc + k0);
+          const float cv[4] = {cc.x, cc.y, cc.z, cc.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float dist = (xx + cv[e]) - 2.f * acc[4 * q + e];
-          if (dist < best) {
-            best = dist;
-            bidx = k0 + e;
+          for (int e = 0; e < 4; ++e) {
+            const float dist = (xx + cv[e]) - 2.f * acc[4 * q + e];
+            if (dist < best) {
+              best = dist;
+              bidx = k0 + e;
+            }
           }
         }
-      }
-    };
-    fold(c0, acc0);
-    if (two) fold(c1, acc1);
+      };
+      fold(c0, acc0);
+      if (two) fold(c1, acc1);
+    }
+  };
+  if constexpr (kHalves) {
+    search(part, min(chunks, 4));
+    if (second) {
+      put(1);
+      __syncthreads();
+      norms(128, 128);
+      __syncthreads();
+      search(4 + part, chunks);
+    }
+  } else {
+    search(part, chunks);
   }
   // the other lane half holds the row's other codewords; the lower index wins ties
   {

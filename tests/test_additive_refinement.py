@@ -209,7 +209,8 @@ def test_block_refinement_argument_errors(kwargs, match):
 # near-tie (the 1e-4 that the difference of two 128-term fp32 sums allows)
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,rows,clusters", [
-    (1, 1, 1), (2, 33, 37), (8, 1500, 256), (8, 3001, 250), (8, 8192, 256), (3, 300, 32)])
+    (1, 1, 1), (2, 33, 37), (8, 1500, 256), (8, 3001, 250), (8, 8192, 256), (3, 300, 32),
+    (8, 8192, 140), (8, 4000, 150), (8, 4000, 100)])
 def test_nearest_f32_matrix_kernel(device, heads, rows, clusters):
     print(f"nearest (matrix kernel) H={heads} N={rows} K={clusters}", flush=True)
     gen = torch.Generator().manual_seed(rows + clusters)
