@@ -144,6 +144,8 @@ class ClosedLoopGroupedCQ(nn.Module):
         if (whitener is None and raw_key.shape == raw_value.shape and raw_key.dtype == raw_value.dtype
                 and raw_key.ndim == 4 and raw_key.shape[1] == heads and raw_key.shape[3] == groups * sub):
             # one launch for the layer's K and V (same bits as two encodes)
+            if vt.shape != kt.shape:  # a table replaced since the constructor's check
+                raise ValueError("K and V tables must share their geometry")
             shape = (heads * groups, 1, clusters, sub)
             key, value, kc, vc = _HardResidualVQPair.apply(
                 raw_key, raw_value, _flat_masters(kt, shape), _flat_masters(vt, shape), groups, sub, (1,), True, False)

@@ -212,3 +212,14 @@ def test_pack_rejects_bad_widths_and_ranges():
         unpack_fixed_width(torch.zeros(3, dtype=torch.uint8), 3, 4)
     with pytest.raises(ValueError, match="count must be non-negative"):
         unpack_fixed_width(torch.zeros(0, dtype=torch.uint8), 3, -1)
+
+
+def test_grouped_cq_refuses_a_replaced_value_table():
+    gen = torch.Generator().manual_seed(3)
+    books = [torch.randn(2, 4, 256, 8, generator=gen)]
+    eye = [torch.eye(8).expand(2, 4, 8, 8).contiguous()]
+    codec = ClosedLoopGroupedCQ(books, books, eye, dynamic_bpa=1.0)
+    codec.value_tables[0] = torch.nn.Parameter(torch.randn(2, 8, 256, 4, generator=gen))  # as many elements
+    states = torch.randn(1, 2, 5, 32, generator=gen).half()
+    with pytest.raises(ValueError, match="share their geometry"):
+        codec(0, states, states)
