@@ -42,8 +42,8 @@ def rvq_encode(
     """
 
     device = _lib.require_device(states, tables, whiteners)
-    batch, heads, tokens, dim = states.shape
-    problems, stages, clusters, d = tables.shape
+    batch, heads, tokens, dim = map(int, states.shape)
+    problems, stages, clusters, d = map(int, tables.shape)
     if dim != groups * group_dim or d != group_dim or problems != heads * groups:
         raise ValueError("state and table geometry differs")
     if tables.dtype != torch.float32 or not tables.is_contiguous():
@@ -98,8 +98,8 @@ def rvq_encode_kv(
     device = _lib.require_device(key, value, key_tables, value_tables)
     if key.shape != value.shape or key.dtype != value.dtype or key_tables.shape != value_tables.shape:
         raise ValueError("K and V must share their geometry")
-    batch, heads, tokens, dim = key.shape
-    problems, stages, clusters, d = key_tables.shape
+    batch, heads, tokens, dim = map(int, key.shape)
+    problems, stages, clusters, d = map(int, key_tables.shape)
     if dim != groups * group_dim or d != group_dim or problems != heads * groups:
         raise ValueError("state and table geometry differs")
     for t in (key_tables, value_tables):
@@ -164,8 +164,8 @@ def rvq_encode_many(
     # tensors are enqueued in well under the launch's own GPU time
     first = states[0]
     device = _lib.require_device(first, tables[0])
-    batch, heads, tokens, dim = first.shape
-    problems, stages, clusters, d = tables[0].shape
+    batch, heads, tokens, dim = map(int, first.shape)
+    problems, stages, clusters, d = map(int, tables[0].shape)
     if dim != groups * group_dim or d != group_dim or problems != heads * groups:
         raise ValueError("state and table geometry differs")
     if len(exits) > _lib.MAX_EXITS:
@@ -220,7 +220,7 @@ def nearest_f32(states: torch.Tensor, tables: torch.Tensor) -> torch.Tensor:
     device = _lib.require_device(states, tables)
     if states.ndim != 3 or tables.ndim != 3:
         raise ValueError("nearest-neighbor inputs must have [H,N,D]/[H,K,D]")
-    heads, tokens, dim = states.shape
+    heads, tokens, dim = map(int, states.shape)
     if int(tables.shape[0]) != heads or int(tables.shape[2]) != dim:
         raise ValueError("nearest-neighbor geometry differs")
     states = states.detach().float().contiguous()
@@ -241,7 +241,7 @@ def nearest_topk_f32(states: torch.Tensor, tables: torch.Tensor, candidates: int
     device = _lib.require_device(states, tables, excluded)
     if states.ndim != 3 or tables.ndim != 3:
         raise ValueError("nearest-neighbor inputs must have [H,N,D]/[H,K,D]")
-    heads, tokens, dim = states.shape
+    heads, tokens, dim = map(int, states.shape)
     if int(tables.shape[0]) != heads or int(tables.shape[2]) != dim:
         raise ValueError("nearest-neighbor geometry differs")
     if excluded is not None:
@@ -266,7 +266,7 @@ def gain_shape_sums(rows: torch.Tensor, indices: torch.Tensor, clusters: int, *,
     device = _lib.require_device(rows, indices, weights)
     if rows.ndim != 3 or indices.shape != rows.shape[:2]:
         raise ValueError("gain-shape rows/indices must be [H,N,D]/[H,N]")
-    heads, tokens, dim = rows.shape
+    heads, tokens, dim = map(int, rows.shape)
     rows = rows.detach().float().contiguous()
     indices = indices.to(torch.int64).contiguous()
     if weights is not None:
@@ -295,7 +295,7 @@ def subtract_codewords(residual: torch.Tensor, tables: torch.Tensor, indices: to
             or tables.ndim != 3 or indices.shape != residual.shape[:2]
             or tables.shape[0] != residual.shape[0] or tables.shape[2] != residual.shape[2]):
         raise ValueError("residual must be contiguous fp32 [H,N,D] with tables [H,K,D] and indices [H,N]")
-    heads, tokens, dim = residual.shape
+    heads, tokens, dim = map(int, residual.shape)
     tables = tables.detach().float().contiguous()
     indices = indices.to(torch.int64).contiguous()
     _lib.check(_lib.load().jkv_subtract_codewords(
@@ -315,8 +315,8 @@ def rvq_decode(
     same result, half the table bytes read."""
 
     device = _lib.require_device(codes, tables)
-    batch, heads, tokens, groups, stages = codes.shape
-    problems, t_stages, clusters, d = tables.shape
+    batch, heads, tokens, groups, stages = map(int, codes.shape)
+    problems, t_stages, clusters, d = map(int, tables.shape)
     if problems != heads * groups or t_stages != stages:
         raise ValueError("code and table geometry differs")
     if codes.dtype != torch.uint8 or codes.stride(-1) != 1 or codes.stride(-2) != stages:
@@ -351,8 +351,8 @@ def rvq_scatter_grad(
     """Accumulate the straight-through codebook gradient into ``grad_tables``."""
 
     device = _lib.require_device(codes, grad_tables, *grads)
-    batch, heads, tokens, groups, stages = codes.shape
-    problems, t_stages, clusters, d = grad_tables.shape
+    batch, heads, tokens, groups, stages = map(int, codes.shape)
+    problems, t_stages, clusters, d = map(int, grad_tables.shape)
     if problems != heads * groups or t_stages != stages or d != group_dim:
         raise ValueError("code and gradient-table geometry differs")
     if grad_tables.dtype != torch.float32 or not grad_tables.is_contiguous():
@@ -401,7 +401,7 @@ def rvq_scatter_grad_many(
         return []
     device = _lib.require_device(*codes, *(g for gs in grads for g in gs),
                                  *(grad_tables if grad_tables is not None else ()))
-    batch, heads, tokens, groups, stages = codes[0].shape
+    batch, heads, tokens, groups, stages = map(int, codes[0].shape)
     n_exits = len(exits)
     if any(len(gs) != n_exits for gs in grads):
         raise ValueError("every job needs one gradient per exit")
@@ -573,10 +573,10 @@ def decode_attention(
     device = _lib.require_device(q, key_codes, value_codes, key_tables16, value_tables16, lengths)
     if q.dtype != torch.float16 or q.ndim != 3 or q.stride(-1) != 1:
         raise ValueError("decode queries must be fp16 [B,QH,D] with a contiguous last axis")
-    batch, qheads, dim = q.shape
+    batch, qheads, dim = map(int, q.shape)
     if key_codes.shape != value_codes.shape or key_codes.dtype != torch.uint8:
         raise ValueError("key/value code caches differ")
-    kb, kvheads, cap, groups, stages = key_codes.shape
+    kb, kvheads, cap, groups, stages = map(int, key_codes.shape)
     if kb != batch:
         raise ValueError("query and cache batch differ")
     strides = key_codes.stride()
@@ -586,7 +586,7 @@ def decode_attention(
         raise ValueError("code caches need contiguous [cap,G,S] blocks")
     if strides != value_strides:
         raise ValueError("key/value code caches need identical strides")
-    problems, t_stages, clusters, d = key_tables16.shape
+    problems, t_stages, clusters, d = map(int, key_tables16.shape)
     if key_tables16.shape != value_tables16.shape or problems != kvheads * groups or t_stages != stages:
         raise ValueError("code-cache and codebook geometry differs")
     if key_tables16.dtype != torch.float16 or value_tables16.dtype != torch.float16:
@@ -656,10 +656,10 @@ def decode_attention_window(
     device = _lib.require_device(q, key_window, value_window, lengths)
     if q.dtype != torch.float16 or q.ndim != 3 or q.stride(-1) != 1:
         raise ValueError("decode queries must be fp16 [B,QH,D] with a contiguous last axis")
-    batch, qheads, dim = q.shape
+    batch, qheads, dim = map(int, q.shape)
     if key_window.shape != value_window.shape or key_window.dtype != torch.float16 or key_window.ndim != 4:
         raise ValueError("decoded windows must be two fp16 [B,KVH,cap,128] tensors of one shape")
-    wb, kvheads, cap, wd = key_window.shape
+    wb, kvheads, cap, wd = map(int, key_window.shape)
     if wb != batch or wd != dim:
         raise ValueError("query and decoded window geometry differ")
     for w in (key_window, value_window):
@@ -695,7 +695,7 @@ def _prefill_operands(q, key, value_or_grad, start_positions, what):
     for name, t in (("query", q), ("key", key), (what, value_or_grad)):
         if t.dtype != torch.float16 or t.ndim != 4 or t.shape[-1] != 128 or t.stride(-1) != 1:
             raise ValueError(f"prefill {name} must be fp16 [B,H,T,128] with a contiguous last axis")
-    batch, qheads, tokens, _dim = q.shape
+    batch, qheads, tokens, _dim = map(int, q.shape)
     if key.shape[0] != batch or key.shape[2] != tokens:
         raise ValueError("prefill query/key/value geometry differs")
     kvheads = int(key.shape[1])
@@ -789,8 +789,8 @@ def prefill_attention_codes(
         raise ValueError("prefill from codes needs [B,KVH,T,16,S<=2] codes and [KVH*16,S,256,8] tables")
     if q.dtype != torch.float16 or q.ndim != 4 or q.shape[-1] != 128 or q.stride(-1) != 1:
         raise ValueError("prefill query must be fp16 [B,H,T,128] with a contiguous last axis")
-    batch, qheads, tokens, _dim = q.shape
-    _b, kvheads, _t, groups, stages = key_codes.shape
+    batch, qheads, tokens, _dim = map(int, q.shape)
+    _b, kvheads, _t, groups, stages = map(int, key_codes.shape)
     if (_b, _t) != (batch, tokens) or qheads % kvheads:
         raise ValueError("prefill query/key/value geometry differs")
     if tuple(key_tables16.shape[:2]) != (kvheads * groups, stages):

@@ -159,7 +159,7 @@ def prefill_attention(
     Returns ``[B,QH,T,128]`` fp16.
     """
 
-    batch, _qh, tokens, _d = query.shape
+    batch, _qh, tokens, _d = map(int, query.shape)
     starts, top = _start_tensor(start_positions, batch, tokens, query.device)
     if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad):
         return _PrefillAttention.apply(query, key, value, starts, window, rope_theta, top)
@@ -176,7 +176,7 @@ class _PrefillAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, query, key, value, starts, window, rope_theta, top):
-        batch, qheads, tokens, _d = query.shape
+        batch, qheads, tokens, _d = map(int, query.shape)
         lse = torch.empty((batch, qheads, tokens), dtype=torch.float32, device=query.device)
         out = _ops.prefill_attention(query, key, value, starts, window=window, rope_theta=rope_theta,
                                      max_position=top, lse=lse)
@@ -230,7 +230,7 @@ def prefill_attention_from_codes(
     if fused:
         if not _ops.prefill_codes_supported(key_codes, key_tables16):
             raise ValueError("the fused prefill needs [B,KVH,T,16,S<=2] codes and [KVH*16,S,256,8] tables")
-        batch, _qh, tokens, _d = query.shape
+        batch, _qh, tokens, _d = map(int, query.shape)
         starts, top = _start_tensor(start_positions, batch, tokens, query.device)
         return _ops.prefill_attention_codes(query, key_codes, value_codes, key_tables16, value_tables16, starts,
                                             window=window, rope_theta=rope_theta, max_position=top)

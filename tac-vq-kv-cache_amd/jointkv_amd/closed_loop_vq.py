@@ -165,11 +165,11 @@ def hard_residual_vq_pair(
         raise ValueError("K and V states must share their geometry")
     if key_tables.shape != value_tables.shape or key_states.ndim != 4 or key_tables.ndim not in (4, 5):
         raise ValueError("K and V tables must share their geometry")
-    batch, heads, tokens, dimension = key_states.shape
+    batch, heads, tokens, dimension = map(int, key_states.shape)
     if key_tables.ndim == 5:
-        t_heads, groups, stages, clusters, group_dim = key_tables.shape
+        t_heads, groups, stages, clusters, group_dim = map(int, key_tables.shape)
     else:
-        t_heads, stages, clusters, group_dim = key_tables.shape
+        t_heads, stages, clusters, group_dim = map(int, key_tables.shape)
         groups = 1
     if t_heads != heads or groups * group_dim != dimension:
         raise ValueError("state and table geometry differs")
@@ -238,7 +238,7 @@ def hard_residual_vq_exits(
 
     if states.ndim != 4 or tables.ndim != 4:
         raise ValueError("states/tables must have [B,H,T,D]/[H,S,K,D]")
-    batch, heads, tokens, dimension = states.shape
+    batch, heads, tokens, dimension = map(int, states.shape)
     if tables.shape[0] != heads or tables.shape[-1] != dimension:
         raise ValueError("state and table geometry differs")
     requested = tuple(sorted(set(int(depth) for depth in prefixes)))
@@ -293,8 +293,8 @@ def hard_grouped_residual_vq(
 
     if states.ndim != 4 or tables.ndim != 5:
         raise ValueError("states/tables must have [B,H,T,G*d]/[H,G,S,K,d]")
-    batch, heads, tokens, dimension = states.shape
-    t_heads, groups, stages, clusters, group_dim = tables.shape
+    batch, heads, tokens, dimension = map(int, states.shape)
+    t_heads, groups, stages, clusters, group_dim = map(int, tables.shape)
     if t_heads != heads or groups * group_dim != dimension:
         raise ValueError("state and table geometry differs")
     requested = tuple(sorted(set(int(depth) for depth in prefixes)))
@@ -336,7 +336,7 @@ def frozen_assignment_reconstruction(
 
     if states.ndim != 4 or tables.ndim != 4 or indices.ndim != 4:
         raise ValueError("frozen assignment geometry must be [B,H,T,D]/[H,S,K,D]/[B,H,T,S]")
-    batch, heads, tokens, dimension = states.shape
+    batch, heads, tokens, dimension = map(int, states.shape)
     stages = int(tables.shape[1])
     if int(tables.shape[0]) != heads or int(tables.shape[-1]) != dimension:
         raise ValueError("frozen assignment table geometry differs")

@@ -37,8 +37,8 @@ def hard_grouped_cq(
 
     if states.ndim != 4 or codebooks.ndim != 4:
         raise ValueError("states/codebooks must be [B,H,T,D]/[H,G,K,S]")
-    batch, heads, tokens, dimension = states.shape
-    cb_heads, groups, clusters, subdimension = codebooks.shape
+    batch, heads, tokens, dimension = map(int, states.shape)
+    cb_heads, groups, clusters, subdimension = map(int, codebooks.shape)
     if cb_heads != heads or groups * subdimension != dimension:
         raise ValueError("CQ codebook geometry differs from states")
     if token_chunk_size <= 0:
@@ -140,7 +140,7 @@ class ClosedLoopGroupedCQ(nn.Module):
             raise ValueError("grouped CQ supports one fixed-rate uniform mode")
         whitener = None if self._identity_selector[layer] else self.key_whitener(layer)
         kt, vt = self.key_tables[layer], self.value_tables[layer]
-        heads, groups, clusters, sub = kt.shape
+        heads, groups, clusters, sub = map(int, kt.shape)
         if (whitener is None and raw_key.shape == raw_value.shape and raw_key.dtype == raw_value.dtype
                 and raw_key.ndim == 4 and raw_key.shape[1] == heads and raw_key.shape[3] == groups * sub):
             # one launch for the layer's K and V (same bits as two encodes)
