@@ -53,13 +53,13 @@ def rvq_encode(
     lib = _lib.load()
     states, (sb, sh, st) = _encode_states_strides(states)
     if codes_out is None:
-        codes = states.new_empty((batch, heads, tokens, groups, stages), dtype=torch.uint8)
+        codes = torch.empty((batch, heads, tokens, groups, stages), dtype=torch.uint8, device=device)
     else:
         codes = codes_out
         if (codes.dtype != torch.uint8 or tuple(codes.shape) != (batch, heads, tokens, groups, stages)
                 or codes.stride(-1) != 1 or codes.stride(-2) != stages or codes.device != device):
             raise ValueError("codes_out must be uint8 [B,H,T,G,S] with a contiguous (G,S) block")
-    recon = [states.new_empty((batch, heads, tokens, dim)) for _ in exits]
+    recon = [torch.empty((batch, heads, tokens, dim), dtype=states.dtype, device=device) for _ in exits]
     if whiteners is not None:
         whiteners = whiteners.detach().float().contiguous()
         if tuple(whiteners.shape) != (problems, d, d):
@@ -116,7 +116,7 @@ def rvq_encode_kv(
     shape = (batch, heads, tokens, groups, stages)
     for out in (key_codes_out, value_codes_out):
         if out is None:
-            out = key.new_empty(shape, dtype=torch.uint8)
+            out = torch.empty(shape, dtype=torch.uint8, device=device)
         elif (out.dtype != torch.uint8 or tuple(out.shape) != shape
               or out.stride(-1) != 1 or out.stride(-2) != stages or out.device != device):
             raise ValueError("codes_out must be uint8 [B,H,T,G,S] with a contiguous (G,S) block")
@@ -124,8 +124,8 @@ def rvq_encode_kv(
     code_strides = codes[0].stride()[:3]
     if code_strides != codes[1].stride()[:3]:
         raise ValueError("K and V code outputs must share their strides")
-    recon_k = [key.new_empty((batch, heads, tokens, dim)) for _ in exits]
-    recon_v = [key.new_empty((batch, heads, tokens, dim)) for _ in exits]
+    recon_k = [torch.empty((batch, heads, tokens, dim), dtype=key.dtype, device=device) for _ in exits]
+    recon_v = [torch.empty((batch, heads, tokens, dim), dtype=key.dtype, device=device) for _ in exits]
     lib = _lib.load()
     ws_bytes = _lib.workspace_bytes("jkv_rvq_encode_workspace_bytes", heads, groups, stages, clusters, d, 0)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device) if ws_bytes else None
@@ -604,7 +604,7 @@ def decode_attention(
     # shorter than the model's window)
     span = max(1, min(int(window), int(max_length)))
     lib = _lib.load()
-    out = q.new_empty((batch, qheads, dim))
+    out = torch.empty((batch, qheads, dim), dtype=torch.float16, device=device)
     ws_bytes = _lib.workspace_bytes("jkv_decode_workspace_bytes", batch, qheads, dim, span)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     if key_new is None and value_new is None:
@@ -677,7 +677,7 @@ def decode_attention_window(
     table = rope_table(device, rope_theta, int(max_length) + 1)
     span = max(1, min(int(window), int(max_length)))
     lib = _lib.load()
-    out = q.new_empty((batch, qheads, dim))
+    out = torch.empty((batch, qheads, dim), dtype=torch.float16, device=device)
     ws_bytes = _lib.workspace_bytes("jkv_decode_workspace_bytes", batch, qheads, dim, span)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     code = lib.jkv_decode_attention_window(
@@ -741,7 +741,7 @@ def prefill_attention(
                             or not lse.is_contiguous() or lse.device != q.device):
         raise ValueError("lse must be a contiguous fp32 [B,QH,T] tensor on the query's device")
     table = rope_table(device, rope_theta, int(max_position) + 1)
-    out = q.new_empty((batch, qheads, tokens, 128))
+    out = torch.empty((batch, qheads, tokens, 128), dtype=torch.float16, device=device)
     code = _lib.load().jkv_prefill_attention(
         q.data_ptr(), *q.stride()[:3], key.data_ptr(), *key.stride()[:3], value.data_ptr(),
         *value.stride()[:3], batch, qheads, kvheads, tokens, 128, start_positions.data_ptr(),

@@ -1,4 +1,5 @@
-"""The operators' Python side without a device: what ``torch.jit.trace`` records.
+"""The operators' Python side without a device: what ``torch.jit.trace``
+records, and results of tensor subclasses.
 
 The library's entry points are replaced by ones that check their arguments
 against the ctypes signatures (a traced shape entry is a tensor, which they
@@ -120,3 +121,15 @@ def test_traces(recorder, name):
     assert replayed is None or (recorder.calls and set(recorder.calls) == {replayed})
     eager, again = (r if isinstance(r, tuple) else (r,) for r in (eager, again))
     assert [(r.shape, r.dtype) for r in again] == [(r.shape, r.dtype) for r in eager]
+
+
+class _Tagged(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("name", list(_calls()))
+def test_results_are_plain_tensors(recorder, name):
+    # a state's subclass is the caller's own: results do not take it on
+    call, inputs, _ = _calls()[name]
+    out = call(*(t.detach().as_subclass(_Tagged) for t in inputs))
+    assert all(type(r) is torch.Tensor for r in (out if isinstance(out, tuple) else (out,)))
