@@ -425,9 +425,15 @@ int jkv_prefill_attention_codes(const void* q, int64_t q_stride_b, int64_t q_str
  *   workspace  jkv_prefill_value_grad_workspace_bytes() bytes, 16-byte
  *            aligned: the rotated queries [B,QH,T,128] fp16, and when a key
  *            block's query rows are split into runs that fill the device
- *            evenly, the runs' partial slots that a second kernel adds up
+ *            evenly, the runs' partial slots that a second kernel adds up.
+ *            Small grids take more and shorter runs than large ones, so the
+ *            query is no monotone function of B.  Any workspace that holds
+ *            the slots of 512-row runs is enough (the query of a larger B or
+ *            T among them): less than the query makes the runs longer.
  * Deterministic: each key's sum runs over the heads, rows and runs in one
- * fixed order.  Limits (JKV_EINVAL past them): B and QH < 65536, T < 2^30,
+ * fixed order, which the geometry (B*KVH, T, window) and a workspace below
+ * the query choose: the same rows in a batch of another size may round
+ * otherwise (fp32 sums).  Limits (JKV_EINVAL past them): B and QH < 65536, T < 2^30,
  * rope_len < 2^23, and for the query heads of one kv head under 2^31 bytes
  * of rotated queries (QH/KVH * T * 256), of d_out ((QH/KVH - 1) * stride_h
  * + (T - 1) * stride_t + 128 elements) and of lse.
@@ -468,6 +474,8 @@ int64_t jkv_prefill_value_grad_workspace_bytes(int64_t B, int64_t QH, int64_t KV
  * sqrt(128), dV = Pᵀ dO, with P recomputed from the forward's lse.
  *   out      the forward output [B,QH,T,128] fp16 (for rowsum(dO * O))
  *   workspace  jkv_prefill_backward_workspace_bytes() bytes, 16-byte aligned
+ *            (less, down to that of 512-row runs, and determinism: as for
+ *            jkv_prefill_attention_value_grad)
  * Query heads per kv head: 1, 2 or a multiple of 4.  Deterministic.  The
  * value leg has the limits of jkv_prefill_attention_value_grad.
  */

@@ -897,21 +897,11 @@ __global__ __launch_bounds__(256) void value_grad_reduce_kernel(const float* __r
 
 // Tiles per chunk and partial slots of the key-block kernels (blocks of
 // `keys` keys, n = B KVH slices): chunks of 16 tiles, of an eighth of the
-// longest block's rows when that is more, or shorter where the grid is small;
-// the slots are the most chunks one block meets.
-static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, int* chunk_tiles, int* slots);
-
-// bytes of the value gradient's workspace: the chunks' partial slots (when
-// there are several), then the rotated queries [B,QH,T,128] fp16 at a
-// 256-byte boundary
-static int64_t value_grad_workspace(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window) {
-  int chunk_tiles, chunks;
-  value_grad_chunks(B * KVH, T, window, kBKeys, &chunk_tiles, &chunks);
-  const int64_t slots = chunks > 1 ? (int64_t)chunks * B * KVH * T * kBD * (int64_t)sizeof(float) : 0;
-  return ceil_div(slots, 256) * 256 + B * QH * T * kBD * 2;
-}
-
-static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, int* chunk_tiles, int* slots) {
+// longest block's rows when that is more, or shorter where the grid is small
+// and the workspace holds their slots (up to max_slots); the slots are the
+// most chunks one block meets.
+static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, int64_t max_slots, int* chunk_tiles,
+                              int* slots) {
   int64_t rows = (int64_t)keys - 1 + window;
   if (rows > T || rows < 0) rows = T;
   const int64_t span = ceil_div(rows, kBRows);  // tiles of the longest block (blocks start on a tile)
@@ -932,10 +922,46 @@ static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, in
   while (per > 2) {
     const int64_t walks = n * ceil_div(T, (int64_t)keys) * (slots_of(per) + 1) / 2;
     if (walks >= (per >= 16 ? 640 : per >= 8 ? 400 : 250)) break;
-    per = std::max<int64_t>(per / 2, 2);
+    const int64_t next = std::max<int64_t>(per / 2, 2);
+    if (slots_of(next) > 1 && slots_of(next) > max_slots) break;
+    per = next;
   }
   *chunk_tiles = (int)per;
   *slots = (int)slots_of(per);
+}
+
+static const int64_t kAnySlots = (int64_t)1 << 62;
+
+// bytes of the partial slots of a walk over blocks of `keys` keys with nout
+// outputs (none where one chunk writes the results): of the chunks that the
+// rule wants, or with max_slots = 0 of the 16-tile ones, the least that a call
+// takes
+static int64_t slot_area(int64_t n, int64_t T, int64_t window, int keys, int nout, int64_t max_slots) {
+  int chunk_tiles, chunks;
+  value_grad_chunks(n, T, window, keys, max_slots, &chunk_tiles, &chunks);
+  return chunks > 1 ? (int64_t)nout * chunks * n * T * kBD * (int64_t)sizeof(float) : 0;
+}
+
+// bytes of the value gradient's workspace: the chunks' partial slots (when
+// there are several), then the rotated queries [B,QH,T,128] fp16 (both whole
+// multiples of 256 bytes)
+static int64_t value_grad_workspace(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window,
+                                    int64_t max_slots) {
+  return slot_area(B * KVH, T, window, kBKeys, 1, max_slots) + B * QH * T * kBD * 2;
+}
+
+// bytes of the full backward's workspace: delta, the rotated keys and queries,
+// and one area that serves the query leg (one query gradient, where only delta
+// is wanted), then the key leg's slots, the value leg's slots (and rotated
+// queries, when it runs alone) or the slots of both from the walk that forms
+// both
+static int64_t backward_workspace(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window, int64_t max_slots) {
+  const int64_t delta = ceil_div(B * QH * T * (int64_t)sizeof(float), 256) * 256;
+  const int64_t rot = B * (KVH + QH) * T * kBD * 2;
+  const int64_t q = B * QH * T * kBD * (int64_t)sizeof(float);
+  const int64_t v = value_grad_workspace(B, QH, KVH, T, window, max_slots);
+  const int64_t kv = slot_area(B * KVH, T, window, 64, 2, max_slots);
+  return delta + rot + std::max(q, std::max(v, kv));
 }
 
 }  // namespace jkv
@@ -944,7 +970,7 @@ extern "C" {
 
 int64_t jkv_prefill_value_grad_workspace_bytes(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window) {
   if (B <= 0 || QH <= 0 || KVH <= 0 || T <= 0 || window < 1) return 0;
-  return jkv::value_grad_workspace(B, QH, KVH, T, window);
+  return jkv::value_grad_workspace(B, QH, KVH, T, window, jkv::kAnySlots);
 }
 
 }  // extern "C"
@@ -995,22 +1021,24 @@ static int launch_kv_grad(ValueGradArgs a, int64_t D, const int64_t (&strides)[1
                 "prefill buffers must be 16-byte aligned");
   a.rope = (const _Float16*)rope_table;
   a.nq = (int32_t)NQ;
-  int chunk_tiles, chunks;
-  value_grad_chunks(B * KVH, T, a.window, keys, &chunk_tiles, &chunks);
-  a.chunk_tiles = chunk_tiles;
-  a.slots = chunks;
-  const int64_t n = B * KVH * T * kBD;
   // workspace: the chunks' partial slots (of each output), then the rotated
-  // queries (unless the caller hands them in)
-  const int64_t slot_bytes = chunks > 1 ? (int64_t)chunks * n * (int64_t)sizeof(float) : 0;
-  const int64_t need =
-      q_rot_given != nullptr ? nout * slot_bytes : value_grad_workspace(B, QH, KVH, T, a.window);
+  // queries (unless the caller hands them in); the chunks are the shortest
+  // that the rule wants and whose slots fit
+  const int64_t n = B * KVH * T * kBD;
+  const int64_t q_rot_bytes = q_rot_given != nullptr ? 0 : B * QH * T * kBD * 2;
+  const int64_t need = slot_area(B * KVH, T, a.window, keys, nout, 0) + q_rot_bytes;
   if (need > 0) {
     JKV_CHECK_ARG(workspace != nullptr && workspace_bytes >= need,
                   "prefill gradient workspace too small: %lld bytes, need %lld", (long long)workspace_bytes,
                   (long long)need);
     JKV_CHECK_ARG(((uintptr_t)workspace) % 16 == 0, "workspace must be 16-byte aligned");
   }
+  int chunk_tiles, chunks;
+  const int64_t held = workspace != nullptr ? workspace_bytes - q_rot_bytes : 0;
+  value_grad_chunks(B * KVH, T, a.window, keys, held / (nout * n * (int64_t)sizeof(float)), &chunk_tiles, &chunks);
+  a.chunk_tiles = chunk_tiles;
+  a.slots = chunks;
+  const int64_t slot_bytes = chunks > 1 ? (int64_t)chunks * n * (int64_t)sizeof(float) : 0;
   if (chunks > 1) {
     a.dv = (float*)workspace;
     a.dk = (float*)((unsigned char*)workspace + slot_bytes);
@@ -1024,7 +1052,7 @@ static int launch_kv_grad(ValueGradArgs a, int64_t D, const int64_t (&strides)[1
   JKV_CHECK_ARG(blocks < ((int64_t)1 << 31), "prefill grid too large");
   const _Float16* q_rot = q_rot_given;
   if (q_rot == nullptr) {
-    _Float16* qr = (_Float16*)((unsigned char*)workspace + ceil_div(slot_bytes, 256) * 256);
+    _Float16* qr = (_Float16*)((unsigned char*)workspace + slot_bytes);
     hipLaunchKernelGGL(rotate_rows_kernel, dim3((uint32_t)ceil_div(8 * T, 256), (uint32_t)QH, (uint32_t)B),
                        dim3(256), 0, stream, a.q, a.qsb, a.qsh, a.qst, T, a.start, a.rope, a.rope_len, qr);
     JKV_CHECK_LAUNCH();
@@ -1151,22 +1179,8 @@ int jkv_prefill_attention_key_grad(const void* q, int64_t q_stride_b, int64_t q_
 }
 
 int64_t jkv_prefill_backward_workspace_bytes(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window) {
-  using namespace jkv;
   if (B <= 0 || QH <= 0 || KVH <= 0 || T <= 0 || window < 1) return 0;
-  int chunk_tiles, chunks, chunks64;
-  value_grad_chunks(B * KVH, T, window, kBKeys, &chunk_tiles, &chunks);
-  value_grad_chunks(B * KVH, T, window, 64, &chunk_tiles, &chunks64);
-  const int64_t delta = ceil_div(B * QH * T * (int64_t)sizeof(float), 256) * 256;
-  const int64_t k_rot = ceil_div(B * KVH * T * kBD * 2, 256) * 256;
-  const int64_t q_rot = ceil_div(B * QH * T * kBD * 2, 256) * 256;
-  // the slot area serves the query leg (delta only), then the key leg's
-  // slots, the value leg's slots (and rotated queries, when it runs alone) or
-  // the slots of both from the walk that forms both
-  const int64_t qk = (int64_t)chunks * B * QH * T * kBD * (int64_t)sizeof(float);
-  const int64_t v = value_grad_workspace(B, QH, KVH, T, window);
-  const int64_t kv = chunks64 > 1 ? 2 * (int64_t)chunks64 * B * KVH * T * kBD * (int64_t)sizeof(float) : 0;
-  const int64_t area = qk > v ? (qk > kv ? qk : kv) : (v > kv ? v : kv);
-  return delta + k_rot + q_rot + area;
+  return jkv::backward_workspace(B, QH, KVH, T, window, jkv::kAnySlots);
 }
 
 }  // extern "C"
@@ -1189,7 +1203,7 @@ static int backward(bool half_out, const void* q, int64_t q_stride_b, int64_t q_
   JKV_CHECK_ARG(B >= 0 && QH > 0 && KVH > 0 && T >= 0 && QH % KVH == 0, "invalid prefill geometry");
   JKV_CHECK_ARG(window >= 1, "window must be positive");
   if (B == 0 || T == 0 || (!d_query && !d_key && !d_value)) return JKV_OK;
-  const int64_t need = jkv_prefill_backward_workspace_bytes(B, QH, KVH, T, window);
+  const int64_t need = backward_workspace(B, QH, KVH, T, window, 0);
   JKV_CHECK_ARG(workspace != nullptr && workspace_bytes >= need && ((uintptr_t)workspace) % 16 == 0,
                 "prefill backward needs %lld bytes of 16-byte aligned workspace", (long long)need);
   const int64_t NQ = QH / KVH;

@@ -220,3 +220,58 @@ def test_many_job_wrappers_reject_host_tensors_and_accept_empty_lists():
         _ops.rvq_scatter_grad_many([[torch.randn(1, 2, 4, 8).half()]], (1,),
                                    [torch.zeros(1, 2, 4, 1, 1, dtype=torch.uint8)], group_dim=8,
                                    table_shape=(2, 1, 256, 8))
+
+
+def _gradient_workspace_floor(name, batch, qh, kvh, tokens, window):
+    """The least workspace a gradient entry takes, from its refusal of none."""
+    lib = _lib.load()
+    strides = (tokens * 128, tokens * 128, 128)
+    rows = 4 if name == "jkv_prefill_attention_backward" else 2
+    args = [x for _ in range(rows) for x in (16, *strides)]
+    outs = (16, 16, 16) if rows == 4 else (16,)
+    rc = getattr(lib, name)(*args, 16, *strides, 16, batch, qh, kvh, tokens, 128, 16, window, 16, 8192, *outs, 16, 0,
+                            None)
+    text = lib.jkv_last_error().decode()
+    assert rc == _lib.JKV_EINVAL and "workspace" in text
+    return int(re.findall(r"needs? (\d+)", text)[-1])
+
+
+@pytest.mark.parametrize("entry,query", [
+    ("jkv_prefill_attention_value_grad", "jkv_prefill_value_grad_workspace_bytes"),
+    ("jkv_prefill_attention_backward", "jkv_prefill_backward_workspace_bytes")])
+def test_a_gradient_workspace_serves_every_smaller_batch_and_length(entry, query):
+    # shorter runs on small grids ask for more than a larger batch does; a
+    # caller who sized its workspace once is served all the same
+    size = getattr(_lib.load(), query)
+    tokens_of = (1, 33, 192, 512, 777, 1024, 2048, 5000)
+    for window in (4096, 300):
+        below = [0] * len(tokens_of)
+        for batch in (1, 2, 3, 8, 11, 12, 16, 40):
+            floors = [_gradient_workspace_floor(entry, batch, 32, 8, t, window) for t in tokens_of]
+            assert all(f <= size(batch, 32, 8, t, window) for f, t in zip(floors, tokens_of))
+            assert floors == sorted(floors) and all(f >= b for f, b in zip(floors, below))
+            below = floors
+    # what a larger batch asks for is enough for a smaller one
+    for small, large in ((1, 2), (2, 3), (11, 12), (3, 40)):
+        for tokens in (192, 777, 2048):
+            assert _gradient_workspace_floor(entry, small, 32, 8, tokens, 4096) <= size(large, 32, 8, tokens, 4096)
+
+
+@pytest.mark.parametrize("batch,qh,kvh,tokens", [
+    (1, 32, 8, 777), (1, 32, 8, 1024), (2, 32, 8, 512), (2, 32, 8, 1024), (12, 32, 8, 192), (1, 32, 4, 2048),
+    (1, 32, 1, 4096), (1, 4, 4, 100)])
+def test_backward_workspace_is_what_its_legs_use(batch, qh, kvh, tokens):
+    lib = _lib.load()
+    row = tokens * 128
+    size = lib.jkv_prefill_backward_workspace_bytes(batch, qh, kvh, tokens, 4096)
+    rotated = batch * (qh + kvh) * row * 2
+    delta = -(-batch * qh * tokens * 4 // 256) * 256
+    query_leg = batch * qh * row * 4
+    value_leg = lib.jkv_prefill_value_grad_workspace_bytes(batch, qh, kvh, tokens, 4096)
+    # the walk that forms both gradients: two outputs, runs of 64 rows at least
+    both_legs = 2 * batch * kvh * row * 4 * -(-tokens // 64)
+    area = size - delta - rotated
+    assert max(query_leg, value_leg) <= area <= max(query_leg, value_leg, both_legs)
+    # no factor of the key blocks' runs on the queries (it made these 2 to 5
+    # times as large)
+    assert size <= 150e6

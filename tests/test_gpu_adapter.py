@@ -3,6 +3,8 @@ its HIP value gradient, and one layer's V-only step against the oracle."""
 
 from __future__ import annotations
 
+import re
+
 import pytest
 import torch
 
@@ -101,6 +103,47 @@ def test_full_backward_matches_oracle(device, batch, qh, kvh, tokens, starts, wi
         err = float((got.cpu().float() - want).abs().max())
         print(f"  {name} err {err:.2e} of {scale:.2e}", flush=True)
         assert err <= DV_RTOL * scale + 1e-3, f"{name} max abs error {err} (scale {scale})"
+
+
+# a workspace below the query, down to the least that the entries take: longer
+# runs of query rows, the same fp32 sums in another order
+@pytest.mark.parametrize("batch,qh,kvh,tokens,window", [(1, 8, 2, 777, 4096), (2, 32, 8, 331, 100), (1, 8, 2, 40, 4096)])
+def test_gradients_in_less_workspace(device, batch, qh, kvh, tokens, window):
+    print(f"less workspace B={batch} QH={qh} KVH={kvh} T={tokens} win={window}", flush=True)
+    q, k, v, d = (t.to(device) for t in _case(2700 + tokens, batch, qh, kvh, tokens))
+    st = torch.zeros(batch, dtype=torch.int32, device=device)
+    kw = dict(window=window, rope_theta=10000.0, max_position=tokens - 1)
+    lse = torch.empty(batch, qh, tokens, dtype=torch.float32, device=device)
+    out = _ops.prefill_attention(q, k, v, st, lse=lse, **kw)
+    table = _ops.rope_table(device, 10000.0, tokens)
+    lib = _ops._lib.load()
+
+    def call(entry, rows, outs, work):
+        return getattr(lib, entry)(
+            *(x for t in rows for x in (t.data_ptr(), *t.stride()[:3])), lse.data_ptr(), batch, qh, kvh, tokens, 128,
+            st.data_ptr(), window, table.data_ptr(), int(table.shape[0]), *(t.data_ptr() for t in outs),
+            work.data_ptr(), work.numel(), _ops._lib.stream_handle(device))
+
+    def empty(like):
+        return torch.empty(like.shape, dtype=torch.float32, device=device)
+
+    for entry, query, rows, like, want in (
+            ("jkv_prefill_attention_value_grad", "jkv_prefill_value_grad_workspace_bytes", (q, k, d), (v,),
+             (_ops.prefill_attention_value_grad(q, k, d, lse, st, **kw),)),
+            ("jkv_prefill_attention_backward", "jkv_prefill_backward_workspace_bytes", (q, k, v, out, d), (q, k, v),
+             _ops.prefill_attention_backward(q, k, v, out, d, lse, st, **kw))):
+        full = int(getattr(lib, query)(batch, qh, kvh, tokens, window))
+        # a refusal names the least
+        assert call(entry, rows, [empty(t) for t in like], torch.empty(16, dtype=torch.uint8, device=device)) != 0
+        least = int(re.findall(r"needs? (\d+)", lib.jkv_last_error().decode())[-1])
+        assert least <= full
+        for size in sorted({least, (least + full) // 2, full}):
+            outs = [empty(t) for t in like]
+            _ops._lib.check(call(entry, rows, outs, torch.empty(size, dtype=torch.uint8, device=device)))
+            for got, ref_ in zip(outs, want):
+                assert size < full or torch.equal(got, ref_)
+                # two orders of at most 777 x 16 products' fp32 sums
+                assert float((got - ref_).abs().max()) <= 1e-5 * float(ref_.abs().max())
 
 
 @pytest.mark.parametrize("batch,qh,kvh,tokens,starts,window", [
