@@ -37,6 +37,7 @@ struct DecodeArgs {
   int64_t rope_len;
   int32_t n_splits;
   int32_t split_tokens;  // tokens per split
+  int32_t records_aligned;  // code records may be read in 16-byte pieces (8 where they are 8 bytes)
   float* ws_o;   // [B,QH,n_splits,D]
   float* ws_ml;  // [B,QH,n_splits,2]
   _Float16* out;
@@ -262,11 +263,21 @@ __global__ __launch_bounds__(256) void decode_split_kernel(DecodeArgs a) {
       }
     }
   }
-  // ---- the split's code records into LDS, 16-byte chunks, one pass ----
+  // ---- the split's code records into LDS, one pass: 16-byte pieces (a
+  // record of eight stages is one of 8), or bytes where the caller's cache is
+  // not aligned to them ----
   const bool codes_in_lds = SS == 8 || (D != 0 && code_bytes <= kMaxCodeBytes && (code_bytes % 16) == 0 &&
                                         code_bytes * kTok <= kRecLds);
-  if constexpr (SS == 8) {
-    // eight-byte records: one piece each
+  if (codes_in_lds && !a.records_aligned) {
+    const int64_t kbase = b * a.csb + kvh * a.csh;
+    const int bytes = (int)code_bytes;
+    for (int idx = tid; idx < ntok * bytes; idx += 256) {
+      const int j = idx / bytes;
+      const int64_t off = kbase + ((t0 + j) % a.cap) * bytes + (idx - j * bytes);
+      kc_lds[idx] = a.kc[off];
+      vc_lds[idx] = a.vc[off];
+    }
+  } else if constexpr (SS == 8) {
     const int64_t kbase = b * a.csb + kvh * a.csh;
     for (int j = tid; j < ntok; j += 256) {
       const int64_t off = kbase + ((t0 + j) % a.cap) * 8;
@@ -1872,6 +1883,9 @@ static int decode_packed(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   a.qsb = q_stride_b; a.qsh = q_stride_h;
   a.kc = k_codes; a.vc = v_codes;
   a.csb = code_stride_b; a.csh = code_stride_h; a.cap = cap;
+  const int64_t piece = G * S == 8 ? 8 : 16;
+  a.records_aligned = (uintptr_t)k_codes % piece == 0 && (uintptr_t)v_codes % piece == 0 &&
+                      code_stride_b % piece == 0 && code_stride_h % piece == 0;
   a.kt = (const _Float16*)k_tables; a.vt = (const _Float16*)v_tables;
   a.B = B; a.QH = QH; a.KVH = KVH; a.G = G; a.d = d; a.S = S; a.K = K;
   a.lengths = lengths;

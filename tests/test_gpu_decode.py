@@ -106,6 +106,37 @@ def test_decode_eight_full_vector_stages(device, batch, qh, kvh, length, window,
     assert err <= ATOL, f"max abs error {err}"
 
 
+# records anywhere in memory: a cache sliced out of a larger one at a byte
+# offset, its heads and batch rows apart by any number of bytes, gives the bits
+# of an aligned copy (16 groups of 8 dims at four stages and 32 of 4 at two:
+# the kernel that reads tables from L2, which staged 64-byte records)
+@pytest.mark.parametrize("groups,stages,d", [(1, 8, 128), (1, 16, 128), (1, 32, 128), (1, 3, 128), (16, 4, 8), (32, 2, 4),
+                                             (16, 2, 8)])
+@pytest.mark.parametrize("offset,pad", [(1, 0), (0, 1), (4, 4), (8, 8)])
+def test_decode_from_unaligned_records(device, groups, stages, d, offset, pad):
+    batch, qh, kvh, length, cap = 2, 8, 2, 333, 400
+    print(f"unaligned records G={groups} S={stages} d={d} offset={offset} pad={pad}", flush=True)
+    q, kc, vc, kt, vt = (t.to(device) for t in _case(stages + offset, batch, qh, kvh, groups, stages, d, length, cap))
+    kt, vt = kt.half(), vt.half()
+    lengths = torch.tensor([length, length - 90], dtype=torch.int32, device=device)
+    rec = groups * stages
+
+    def apart(codes):
+        head = cap * rec + pad
+        flat = torch.zeros(batch * (kvh * head + pad) + offset, dtype=torch.uint8, device=device)
+        view = flat[offset:].as_strided((batch, kvh, cap, groups, stages), (kvh * head + pad, head, rec, stages, 1))
+        view.copy_(codes)
+        return view
+
+    want = jkv.decode_attention(q, kc, vc, kt, vt, lengths, window=cap)
+    got = jkv.decode_attention(q, apart(kc), apart(vc), kt, vt, lengths, window=cap)
+    if d != 128 and stages * groups <= 32:
+        # unaligned caches leave the LDS-table kernel for another one
+        assert float((got.float() - want.float()).abs().max()) <= ATOL
+    else:
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("batch,qh,kvh,stages,lengths,window,cap", [
     (2, 32, 8, 2, (4096, 4096), 4096, 4096),    # config 4 geometry: the new token closes split 2
     (3, 8, 2, 2, (1, 257, 5000), 4096, 4096),   # first token; chunk 1's first key; ring wrap
