@@ -254,7 +254,15 @@ int jkv_scale_sgd(int32_t n, float* const* params, float* const* grads,
  *   rope_table  jkv_rope_table() output covering positions [0, rope_len),
  *            rope_len > max(lengths) - 1
  *   out      [B,QH,D] fp16 contiguous
- *   workspace  jkv_decode_workspace_bytes() bytes (split-KV partials)
+ *   workspace  jkv_decode_workspace_bytes() bytes (split-KV partials).  The
+ *            kernels that hold the tables in LDS (group dims 4 and 8, 16-byte
+ *            aligned codes and tables) split a window into runs of 256 to
+ *            2048 tokens, chosen from B*KVH and window, and take any
+ *            workspace that holds the partials of 2048-token splits
+ * A call repeats bit for bit.  The splits, and with them the rounding of the
+ * probabilities (fp16, under the split's own maximum) and the order of the
+ * fp32 sums, follow from B*KVH, window and the workspace: the same row in a
+ * batch of another size may differ in its last fp16 bits.
  */
 int64_t jkv_decode_workspace_bytes(int64_t B, int64_t QH, int64_t D,
                                    int64_t window);
@@ -312,7 +320,8 @@ int jkv_decode_attention_append(const void* q, int64_t q_stride_b,
  * space than that return JKV_EINVAL: B*QH*n_splits*(128+2)*4 bytes, with
  * n_splits = ceil(window/2048) for group dims 4 and 8 on 16-byte aligned
  * codes and tables (e.g. config 4 up to B*QH = 16,131 at a 4096-token
- * window) and ceil(window/256) otherwise (the bound that
+ * window; small grids take shorter splits, of at most 512*(QH/KVH)*520
+ * bytes) and ceil(window/256) otherwise (the bound that
  * jkv_decode_workspace_bytes reports).  The array is looked up on the first call on each
  * device (the current HIP device); no call allocates or frees memory.  Every
  * call on a device shares that device's array: calls that overlap on one

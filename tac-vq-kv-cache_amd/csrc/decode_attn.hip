@@ -1665,17 +1665,20 @@ static int64_t lds_bytes(int64_t S, int64_t nq) {
 // 8 kv heads, us per call, longest splits against the chosen ones): 1 row of
 // 1,536 tokens 24.4 -> 14.3, of 4,096 31.8 -> 14.7; 8 rows of 4,096 33.7 ->
 // 24.0; 16 rows of 1,536 25.8 -> 21.1; 20 rows of 4,096 64 -> 55; 16 rows of
-// 4,096 keep two splits each (35.6; four take 44).  Never more than 512
-// workgroups unless the longest splits need them: the partials then stay
-// within those of the longest splits or 2 MB, whatever holds them.
-static int64_t lds_table_split(int64_t n, int64_t window) {
+// 4,096 keep two splits each (35.6; four take 44).  Splits shorter than the
+// longest are at most 512 workgroups (partials of 512 x QH/KVH x 520 bytes,
+// 2.13 MB at eight query heads per kv head) and `room`, the workgroups whose
+// partials the caller's workspace holds.
+constexpr int64_t kMaxChunks = kLdsMaxSplit / kLdsChunk;  // a register slot each in both kernels
+static_assert(kG8Chunk == kLdsChunk && kG8MaxSplit == kLdsMaxSplit, "one split rule for both table kernels");
+static int64_t lds_table_split(int64_t n, int64_t window, int64_t room) {
   const int64_t chunks = ceil_div(window, kLdsChunk);
-  const int64_t longest = chunks < 8 ? chunks : 8;
+  const int64_t longest = chunks < kMaxChunks ? chunks : kMaxChunks;
   int64_t best = longest;
   double least = 0.0;
   for (int64_t c = longest; c >= 1; --c) {
     const int64_t blocks = n * ceil_div(chunks, c);
-    if (c < longest && blocks > 512) break;
+    if (c < longest && (blocks > 512 || blocks > room)) break;
     const double t = (double)ceil_div(blocks, 256) * ((double)c + 2.5) + (c < chunks ? 1.0 : 0.0);
     if (c == longest || t < least) {
       least = t;
@@ -1686,11 +1689,12 @@ static int64_t lds_table_split(int64_t n, int64_t window) {
 }
 
 // Tokens per split of decode_lds_kernel (0: the geometry does not fit).
-static int64_t lds_split_tokens(int64_t n, int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window) {
+static int64_t lds_split_tokens(int64_t n, int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window,
+                                int64_t room) {
   if (S > 2 || K != kLdsK || G * S > kLdsCodeBytes || (G * S) % 16 != 0) return 0;
   if (lds_bytes(S, nq) > kMaxLds) return 0;
   if (kLdsWaves * nq * kHeadDim * 4 > kHeadDim * S * K * 2) return 0;  // partials fit the table area
-  return lds_table_split(n, window);
+  return lds_table_split(n, window, room);
 }
 
 // Dynamic LDS of decode_g8_kernel: tables, one chunk of code records, the
@@ -1700,35 +1704,25 @@ static int64_t g8_lds_bytes(int64_t S, int64_t nq) {
 }
 
 // Tokens per split of decode_g8_kernel (0: the geometry does not fit).
-static int64_t g8_split_tokens(int64_t n, int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window) {
+static int64_t g8_split_tokens(int64_t n, int64_t G, int64_t S, int64_t K, int64_t nq, int64_t window,
+                               int64_t room) {
   if (G != 16 || S < 1 || S > 2 || K != kLdsK) return 0;
   if (g8_lds_bytes(S, nq) > kMaxLds) return 0;
   if (kG8Waves * nq * kHeadDim * 4 > 16 * S * kG8Plane) return 0;  // partials fit the table area
-  return lds_table_split(n, window);
+  return lds_table_split(n, window, room);
 }
 
-// Tokens per split of the kernel launch_decode picks for a packed-code
-// geometry and n (batch row, kv head) pairs (the LDS-table kernels take up
-// to 2048-token splits, the L2 split kernel kSplitTokens), so callers can
-// size the partials exactly.
-static int64_t packed_split_tokens(int64_t n, int64_t G, int64_t d, int64_t S, int64_t K, int64_t nq,
-                                   int64_t window, bool lds_ok) {
-  if (lds_ok && d == 8) {
-    const int64_t g8 = g8_split_tokens(n, G, S, K, nq, window);
-    if (g8 > 0) return g8;
-  }
-  if (lds_ok && (d == 8 || d == 4)) {
-    const int64_t lds = lds_split_tokens(n, G, S, K, nq, window);
-    if (lds > 0) return lds;
-  }
-  return kSplitTokens;
-}
-
-// Bytes of split partials ([B,QH,n_splits] x (128 + 2) fp32) that launch.
+// Bytes of split partials ([B,QH,n_splits] x (128 + 2) fp32) that a
+// packed-code call needs at least: 2048-token splits on the LDS-table kernels
+// (shorter ones only as the workspace holds them), kSplitTokens on the L2
+// split kernel.
 static int64_t packed_partial_bytes(int64_t B, int64_t QH, int64_t G, int64_t d, int64_t S, int64_t K, int64_t nq,
                                     int64_t window, bool lds_ok) {
-  const int64_t ns = ceil_div(window, packed_split_tokens(B * (QH / nq), G, d, S, K, nq, window, lds_ok));
-  return B * QH * ns * (kHeadDim + 2) * (int64_t)sizeof(float);
+  const int64_t n = B * (QH / nq);
+  int64_t split = 0;
+  if (lds_ok && d == 8) split = g8_split_tokens(n, G, S, K, nq, window, 0);
+  if (lds_ok && split == 0 && (d == 8 || d == 4)) split = lds_split_tokens(n, G, S, K, nq, window, 0);
+  return B * QH * ceil_div(window, split > 0 ? split : kSplitTokens) * (kHeadDim + 2) * (int64_t)sizeof(float);
 }
 
 // The LDS-table kernels copy code records and tables in 16-byte pieces.
@@ -1764,9 +1758,12 @@ static void launch_split(const DecodeArgs& a, hipStream_t stream) {
 }
 
 template <int D, int NQ>
-static int launch_decode(DecodeArgs a, bool lds_ok, hipStream_t stream, bool append = false) {
-  const int64_t split = lds_ok && D != 128 && D != 0 ? lds_split_tokens(a.B * a.KVH, a.G, a.S, a.K, NQ, a.window) : 0;
-  const int64_t g8_split = lds_ok && D == 8 ? g8_split_tokens(a.B * a.KVH, a.G, a.S, a.K, NQ, a.window) : 0;
+static int launch_decode(DecodeArgs a, bool lds_ok, int64_t workspace_bytes, hipStream_t stream,
+                         bool append = false) {
+  const int64_t room = workspace_bytes / (NQ * (kHeadDim + 2) * (int64_t)sizeof(float));
+  const int64_t n = a.B * a.KVH;
+  const int64_t split = lds_ok && D != 128 && D != 0 ? lds_split_tokens(n, a.G, a.S, a.K, NQ, a.window, room) : 0;
+  const int64_t g8_split = lds_ok && D == 8 ? g8_split_tokens(n, a.G, a.S, a.K, NQ, a.window, room) : 0;
   if constexpr (D == 128 || D == 0) {
     launch_split<D, NQ>(a, stream);
   } else if (D == 8 && g8_split > 0) {
@@ -1873,8 +1870,8 @@ static int decode_packed(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
   JKV_CHECK_ARG(q && k_codes && v_codes && k_tables && v_tables && lengths && out && rope_table,
                 "null buffer");
   const bool lds_ok = packed_lds_ok(k_codes, v_codes, code_stride_b, code_stride_h, k_tables, v_tables);
-  // what the chosen kernel writes; jkv_decode_workspace_bytes() is an upper
-  // bound of it for every packed geometry
+  // jkv_decode_workspace_bytes() is an upper bound of what any packed
+  // geometry writes; the LDS-table kernels take less, with longer splits
   const int64_t need = packed_partial_bytes(B, QH, G, d, S, K, nq, window, lds_ok);
   JKV_CHECK_ARG(workspace != nullptr && workspace_bytes >= need,
                 "decode attention needs %lld bytes of workspace", (long long)need);
@@ -1909,7 +1906,7 @@ static int decode_packed(const void* q, int64_t q_stride_b, int64_t q_stride_h, 
     a.vc_out = const_cast<uint8_t*>(v_codes);
   }
 #define JKV_DEC(DD, NN) \
-  if (d == DD && nq == NN) return launch_decode<DD, NN>(a, lds_ok, stream, append);
+  if (d == DD && nq == NN) return launch_decode<DD, NN>(a, lds_ok, workspace_bytes, stream, append);
   JKV_DEC(8, 1) JKV_DEC(8, 2) JKV_DEC(8, 4) JKV_DEC(8, 8)
   JKV_DEC(4, 1) JKV_DEC(4, 2) JKV_DEC(4, 4) JKV_DEC(4, 8)
   JKV_DEC(128, 1) JKV_DEC(128, 2) JKV_DEC(128, 4) JKV_DEC(128, 8)
@@ -1987,9 +1984,9 @@ int jkv_decode_attention_noalloc(const void* q, int64_t q_stride_b, int64_t q_st
                                  jkv_stream_t stream) {
   using namespace jkv;
   JKV_CHECK_ARG(B >= 0 && QH > 0 && KVH > 0 && QH % KVH == 0 && window > 0, "invalid head geometry");
-  // the partials of the kernel this call will run: splits of up to 2048
-  // tokens on the LDS-table kernels (group dims 4 and 8), 256-token ones
-  // otherwise
+  // the least that this call's kernel needs: 2048-token splits on the
+  // LDS-table kernels (group dims 4 and 8; shorter ones fit the scratch
+  // too), 256-token ones otherwise
   const bool lds_ok = packed_lds_ok(k_codes, v_codes, code_stride_b, code_stride_h, k_tables, v_tables);
   const int64_t need = packed_partial_bytes(B, QH, G, d, S, K, QH / KVH, window, lds_ok);
   JKV_CHECK_ARG(need <= kNoAllocScratchBytes,
@@ -2046,10 +2043,10 @@ int jkv_decode_attention_window(const void* q, int64_t q_stride_b, int64_t q_str
   a.ws_ml = a.ws_o + B * QH * a.n_splits * kHeadDim;
   a.out = (_Float16*)out;
   switch (nq) {
-    case 1: return launch_decode<0, 1>(a, false, stream);
-    case 2: return launch_decode<0, 2>(a, false, stream);
-    case 4: return launch_decode<0, 4>(a, false, stream);
-    default: return launch_decode<0, 8>(a, false, stream);
+    case 1: return launch_decode<0, 1>(a, false, 0, stream);
+    case 2: return launch_decode<0, 2>(a, false, 0, stream);
+    case 4: return launch_decode<0, 4>(a, false, 0, stream);
+    default: return launch_decode<0, 8>(a, false, 0, stream);
   }
 }
 

@@ -70,6 +70,10 @@ def decode_attention(
     (the codec call and ``LayerCache.append`` of
     evaluate_mistral_longbench.py:94-98, fused; group dim 8 caches).
     Returns ``[B,QH,1,D]`` (or ``[B,QH,D]``) fp16.
+
+    A call repeats bit for bit.  How a window is split follows from the batch
+    size, head counts, ``window`` and ``max_length``, so a row may differ in
+    its last fp16 bits between batches of different sizes.
     """
 
     squeeze = query.ndim == 3
@@ -156,7 +160,9 @@ def prefill_attention(
     codec's reconstructions) at positions ``start + t``, ``repeat_kv``, and
     SDPA with the causal mask and Mistral's ``window``-token sliding window.
     ``start_positions``: an int, a sequence of B ints or an int32 tensor.
-    Returns ``[B,QH,T,128]`` fp16.
+    Returns ``[B,QH,T,128]`` fp16.  Its gradients are deterministic, the order
+    of the key and value gradients' fp32 sums follows from the batch size,
+    head counts, tokens and ``window``.
     """
 
     batch, _qh, tokens, _d = map(int, query.shape)

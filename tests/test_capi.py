@@ -113,6 +113,20 @@ def test_decode_rejects_unsupported_geometry():
     assert rc == _lib.JKV_EINVAL and b"rotary" in lib.jkv_last_error()
 
 
+@pytest.mark.parametrize("batch,qh,kvh,groups,stages,d,window", [
+    (1, 32, 8, 16, 2, 8, 4096), (1, 32, 8, 16, 2, 8, 1501), (2, 8, 8, 16, 1, 8, 8192), (4, 32, 8, 32, 1, 4, 3000),
+    (16, 32, 8, 16, 2, 8, 4096), (170, 64, 8, 16, 2, 8, 4096)])
+def test_decode_takes_a_workspace_of_the_longest_splits(batch, qh, kvh, groups, stages, d, window):
+    # with none the call is refused before a launch and says what it needs
+    lib = _lib.load()
+    rc = lib.jkv_decode_attention(16, 0, 0, 16, 16, 0, 0, window, 16, 16, batch, qh, kvh, groups, d, stages, 256, 16,
+                                  window, 16, 8192, 16, 16, 0, None)
+    assert rc == _lib.JKV_EINVAL
+    need = int(re.search(r"needs (\d+) bytes of workspace", lib.jkv_last_error().decode()).group(1))
+    assert need == batch * qh * -(-window // 2048) * 130 * 4
+    assert need <= lib.jkv_decode_workspace_bytes(batch, qh, 128, window)
+
+
 def test_decode_window_rejects_bad_arguments():
     # validation only: every call below fails before a launch
     lib = _lib.load()

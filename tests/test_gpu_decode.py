@@ -90,6 +90,65 @@ def test_decode_split_rule(device, batch, qh, kvh, groups, stages, d, lengths, w
         assert err <= ATOL, f"row {b} length {lengths[b]}: {err}"
 
 
+def _split_bound(q, kc, vc, kt, vt, length, window, out):
+    """How far two choices of splits may lie apart: a probability is rounded
+    to fp16 under its split's own maximum (2^-11 of it either way), the
+    output once, and the fp32 sums' order is far below both."""
+    start = max(0, length - window)
+    slots = torch.arange(start, length) % kc.shape[2]
+    khat, vhat = (ref.frozen_decode(c[:, :, slots].contiguous(), t, t.shape[1], torch.float16) for c, t in ((kc, kt), (vc, vt)))
+    weight = ref.decode_attention(q, khat, vhat.abs(), length - 1, torch.arange(start, length)).float()
+    return 2.0 ** -10 * (weight + out.float().abs()) + 1e-5
+
+
+# one row alone takes short splits, in a batch that fills the chip the longest:
+# other roundings of the same sums, each call the same on every run
+@pytest.mark.parametrize("groups,stages,d,length", [(16, 2, 8, 1501), (16, 1, 8, 4096), (32, 1, 4, 700)])
+def test_decode_row_alone_and_in_a_batch(device, groups, stages, d, length):
+    batch, qh, kvh, window = 16, 32, 8, 4096
+    print(f"decode row alone G={groups} S={stages} d={d} len={length}", flush=True)
+    q, kc, vc, kt, vt = _case(77 + length, 1, qh, kvh, groups, stages, d, length, window)
+    on = [t.to(device) for t in (q, kc, vc, kt.half(), vt.half())]
+    many = [t.expand(batch, *t.shape[1:]).contiguous() for t in on[:3]] + on[3:]
+    lengths = torch.full((batch,), length, dtype=torch.int32, device=device)
+    alone = jkv.decode_attention(*on, lengths[:1], window=window, max_length=length)
+    rows = jkv.decode_attention(*many, lengths, window=window, max_length=length)
+    for _ in range(3):
+        assert torch.equal(alone, jkv.decode_attention(*on, lengths[:1], window=window, max_length=length))
+        assert torch.equal(rows, jkv.decode_attention(*many, lengths, window=window, max_length=length))
+    assert (rows == rows[:1]).all()
+    bound = _split_bound(q, kc, vc, kt, vt, length, window, alone.cpu())
+    assert bool(((alone.cpu().float() - rows[:1].cpu().float()).abs() <= bound).all())
+
+
+# a workspace for 2048-token splits is enough: the splits are the shortest that
+# fit it
+@pytest.mark.parametrize("batch,groups,stages,d,length", [(1, 16, 2, 8, 4096), (2, 32, 1, 4, 3000), (1, 16, 1, 8, 300)])
+def test_decode_in_less_workspace(device, batch, groups, stages, d, length):
+    qh, kvh, window = 8, 2, 4096
+    print(f"decode workspace B={batch} G={groups} S={stages} d={d} len={length}", flush=True)
+    q, kc, vc, kt, vt = _case(88 + length, batch, qh, kvh, groups, stages, d, length, window)
+    dq, dk, dv, dkt, dvt = (t.to(device) for t in (q, kc, vc, kt.half(), vt.half()))
+    lengths = torch.full((batch,), length, dtype=torch.int32, device=device)
+    want = jkv.decode_attention(dq, dk, dv, dkt, dvt, lengths, window=window, max_length=length)
+    _ops = jkv.attention._ops
+    lib, table = _ops._lib.load(), _ops.rope_table(torch.device(device), 10000.0, length + 1)
+    full = int(lib.jkv_decode_workspace_bytes(batch, qh, 128, length))
+    least = batch * qh * -(-length // 2048) * 130 * 4
+    for size in (least, (least + full) // 2, full):
+        out = torch.empty(batch, qh, 128, dtype=torch.float16, device=device)
+        work = torch.empty(size, dtype=torch.uint8, device=device)
+        _ops._lib.check(lib.jkv_decode_attention(
+            dq.data_ptr(), dq.stride(0), dq.stride(1), dk.data_ptr(), dv.data_ptr(), dk.stride(0), dk.stride(1), window,
+            dkt.data_ptr(), dvt.data_ptr(), batch, qh, kvh, groups, d, stages, 256, lengths.data_ptr(), length,
+            table.data_ptr(), int(table.shape[0]), out.data_ptr(), work.data_ptr(), size,
+            _ops._lib.stream_handle(out.device)))
+        out = out.cpu().reshape(q.shape)
+        assert size < full or torch.equal(out, want.cpu())
+        bound = _split_bound(q, kc, vc, kt, vt, length, window, want.cpu())
+        assert bool(((out.float() - want.cpu().float()).abs() <= bound).all())
+
+
 # eight full-vector stages (eight-byte records): ragged tiles, a ring that
 # wraps, one query head per kv head and GQA 8
 @pytest.mark.parametrize("batch,qh,kvh,length,window,cap", [
