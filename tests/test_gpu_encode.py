@@ -488,20 +488,66 @@ def test_bf16_grouped_encode(device, batch, tokens, dim, stages, scale, strided)
         assert torch.equal(got[rows], want[rows])
 
 
-def test_bf16_grouped_encode_outside_fp16(device):
+def _same_as_fp32_search(states, tables, device):
+    """Codes and every exit of the bf16 encode equal those of the fp32 search
+    of the same values, rounded to bf16."""
+    prefixes = tuple(range(1, tables.shape[2] + 1))
+    exits, codes = jkv.hard_grouped_residual_vq(states.to(device), tables.to(device), prefixes=prefixes)
+    wide, want = jkv.hard_grouped_residual_vq(states.float().to(device), tables.to(device), prefixes=prefixes)
+    assert torch.equal(codes, want)
+    for depth in prefixes:
+        assert exits[depth].dtype == torch.bfloat16
+        assert torch.equal(torch.nan_to_num(exits[depth].float(), nan=1234.5),
+                           torch.nan_to_num(wide[depth].bfloat16().float(), nan=1234.5))
+        assert torch.equal(exits[depth].isinf(), wide[depth].bfloat16().isinf())
+    return codes.cpu()
+
+
+@pytest.mark.parametrize("dim,stages", [(8, 2), (8, 1), (4, 2), (4, 1)])
+def test_bf16_grouped_encode_outside_fp16(device, dim, stages):
     # rows the kernel's fp16 words cannot carry (and a codebook of a problem
     # that overflows them) take its fp32 scan, and the other rows the same
     # codes: every code is the fp32 search's over the same values
+    print(f"bf16 encode outside fp16 d={dim} S={stages}", flush=True)
     gen = _gen(5200)
     states = ref.synthetic_states(gen, 1, 2, 300).float()
     states[0, 0, 3] *= 3e5
     states[0, 0, 64:70] *= 1e20
     states[0, 1, 7, 8:16] = float("inf")
     states[0, 1, 9, 0] = float("nan")
-    states = states.bfloat16()
-    tables = ref.synthetic_tables(gen, (2, 16, 2, 256, 8), (1.0, 0.5), stage_axis=2)
-    tables[1, 5] *= 2e4
-    _, codes = jkv.hard_grouped_residual_vq(states.to(device), tables.to(device), prefixes=(2,))
-    _, want = jkv.hard_grouped_residual_vq(states.float().to(device), tables.to(device), prefixes=(2,))
-    codes, want = codes.cpu(), want.cpu()
-    assert torch.equal(codes, want)
+    states[0, 1, 11, 4:8] = float("-inf")
+    tables = ref.synthetic_tables(gen, (2, 128 // dim, stages, 256, dim), (1.0, 0.5)[:stages], stage_axis=2)
+    tables[1, 5] *= 2e4   # finite and infinite fp16 words
+    tables[1, 6] *= 2e3   # |c|^2 beyond the kernel's own words
+    _same_as_fp32_search(states.bfloat16(), tables, device)
+
+
+@pytest.mark.parametrize("dim", [8, 4])
+def test_bf16_grouped_encode_ties(device, dim):
+    # equal words (a fitted table's dead ones): in one run of eight, in
+    # another, in the other 128 words, in all three; rows on such a word, and
+    # halfway between two words.  The lowest index, as in the fp32 search
+    print(f"bf16 encode ties d={dim}", flush=True)
+    gen = _gen(5300 + dim)
+    groups = 128 // dim
+    tables = ref.synthetic_tables(gen, (2, groups, 2, 256, dim), (1.0, 0.5), stage_axis=2).bfloat16().float()
+    pairs = ((3, 4), (10, 19), (37, 165), (64, 250), (127, 128), (0, 255))
+    for low, high in pairs:
+        tables[:, :, :, high] = tables[:, :, :, low]
+    tables[:, :, :, 200:208] = tables[:, :, :, 40:48]
+    tables[0, 1, 0] = tables[0, 1, 0, 77]       # one word in every place
+    tables[1, :, 1] = 0.0                       # a second stage that adds nothing
+    picks = torch.tensor([p for pair in pairs for p in pair] + list(range(200, 208)) + list(range(40, 48)))
+    on_words = tables[:, :, 0, picks].permute(0, 2, 1, 3).reshape(2, len(picks), 128)
+    words = tables[:, :, 0, torch.randint(0, 256, (2, 90), generator=gen)]      # [2,groups,2,90,dim]
+    between = ((words[:, :, 0] + words[:, :, 1]) / 2).permute(0, 2, 1, 3).reshape(2, 90, 128)
+    zeros = torch.zeros(2, 5, 128)
+    states = torch.cat([on_words, between, zeros], dim=1)[None].bfloat16()
+    codes = _same_as_fp32_search(states, tables, device)
+    lowest = {high: low for low, high in pairs} | {200 + i: 40 + i for i in range(8)}
+    plain = [g for g in range(groups) if g != 1]
+    for row, pick in enumerate(picks.tolist()):
+        assert (codes[0, :, row, plain, 0] == lowest.get(pick, pick)).all()
+    assert (codes[0, 0, :, 1, 0] == 0).all() and (codes[0, 1, :, :, 1] == 0).all()
+    for high in lowest:
+        assert (codes != high).all()
