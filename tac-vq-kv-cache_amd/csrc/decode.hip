@@ -96,7 +96,15 @@ __global__ __launch_bounds__(256) void rvq_decode_kernel(RvqDecodeArgs a) {
 // i / G, i / G + 512 / G, ...: the 16 or 32 threads of a token write its row
 // in one contiguous run.  The same sums in the same order as
 // rvq_decode_kernel.
-static const int kLdsDecodeTokens = 128;  // shortest run
+//
+// Shortest run: 128 tokens, so that small calls fill the CUs (8 heads of
+// 4,096 tokens, S = 2, fp16: 7.5 us against 10.0 with runs of 512; 8,192: 11.1
+// against 13.2).  Where the fp32 masters of all heads exceed an XCD's L2,
+// staging them is the time and fewer, longer runs win: S = 2, 32 heads of
+// 1,024 tokens 10.9 us with 512 against 14.5 with 128, of 2,048 14.1 against
+// 15.8; 128 heads of 256, S = 1, 7.6 against 9.3.
+static const int kLdsDecodeTokens = 128;
+static const int kLdsDecodeFarTokens = 512;
 template <int DT, bool F16>
 __global__ __launch_bounds__(512) void rvq_decode_lds_kernel(RvqDecodeArgs a) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -206,15 +214,24 @@ static int rvq_decode_impl(const uint8_t* codes, int64_t code_stride_b, int64_t 
   };
   const int cw = aligned(8) ? 8 : aligned(4) ? 4 : 1;
   // 8-dim groups whose head tables fit 128 KiB of LDS: gathers from LDS, once
-  // the rows pay for staging the tables (S = 2, 8 heads: 6.2 us against 3.4
-  // from L2 at 777 tokens, 7.2 both at 32,768 rows, 19 against 36 at 262,144)
+  // the rows pay for staging the tables.  8 heads, staged against gathered,
+  // us: fp16 tables and results, S = 2: 6.3 and 3.5 at 777 tokens, 7.5 and 7.4
+  // at 4,096 (the line), 11.1 and 11.4 at 8,192, 20.8 and 35.9 at 32,768.
+  // S = 1 and fp32 tables or results cross between 4,096 and 8,192 tokens:
+  // fp16 S = 1 5.9 and 5.4, then 8.0 and 7.9; fp32 S = 2 11.4 and 10.4, then
+  // 16.8 and 17.5; fp32 S = 1 9.1 and 7.8, then 13.9 and 13.5
   const bool lds = B * H * T >= 32768 && d == 8 && K == 256 && G * S <= 32 && 512 % G == 0 && cw == 8 && depth <= 2 &&
                    (uintptr_t)tables % 16 == 0 && B * H * ceil_div(T, kLdsDecodeTokens) < ((int64_t)1 << 31);
   if (lds) {
     // runs long enough for one round of workgroups over 256 CUs (each holds
     // one: 128 KiB of tables), so each CU stages its tables once
     const int64_t runs_per_slice = std::max<int64_t>(1, 256 / (B * H));
-    a.run_tokens = (int32_t)std::max<int64_t>(kLdsDecodeTokens, ceil_div(T, runs_per_slice));
+    // masters of H G S x 8 KiB, of which a workgroup reads G S x 8: the line
+    // lies between 16 and 32 heads at S = 2 (16 heads of 3,072 tokens: 12.0 us
+    // with 128, 12.5 with 512) and 64 and 128 at S = 1 (64 of 768: 9.0, 9.8)
+    const bool far = !tables_f16 && H * (G * S) * (G * S) > 16384;
+    a.run_tokens = (int32_t)std::max<int64_t>(far ? kLdsDecodeFarTokens : kLdsDecodeTokens,
+                                              ceil_div(T, runs_per_slice));
     switch (out_dtype) {
       case JKV_F16:
         tables_f16 ? launch_decode_lds<JKV_F16, true>(a, stream) : launch_decode_lds<JKV_F16, false>(a, stream);

@@ -453,6 +453,18 @@ def test_rvq_decode_staging_rule(device, tokens, tables_f16):
     assert torch.equal(got.cpu(), ref.frozen_decode(codes, tables, 2, torch.float16))
 
 
+# either side of the heads from which fp32 masters are staged for longer runs,
+# with a partial last run
+@pytest.mark.parametrize("heads,tokens,stages", [(16, 2100, 2), (17, 2100, 2), (40, 1030, 2), (65, 520, 1)])
+def test_rvq_decode_runs_of_many_heads(device, heads, tokens, stages):
+    gen = _gen(6464 + heads)
+    tables = ref.synthetic_tables(gen, (heads * 16, stages, 256, 8), (1.0, 0.5)[:stages], stage_axis=1)
+    codes = torch.randint(0, 256, (1, heads, tokens, 16, stages), generator=gen, dtype=torch.uint8)
+    for dtype in (torch.float16, torch.float32):
+        got = jkv.closed_loop_vq._ops.rvq_decode(codes.to(device), tables.to(device), depth=stages, dtype=dtype)
+        assert torch.equal(got.cpu(), ref.frozen_decode(codes, tables, stages, dtype))
+
+
 # bf16 states on the grouped MFMA kernel: slabs of 64 rows, 256 per workgroup
 # pass; one row, tile and slab edges, rows that straddle batch entries, strided
 # [B,T,H,D] views, both group widths, codebooks far from unit scale
