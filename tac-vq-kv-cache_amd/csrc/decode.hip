@@ -219,8 +219,15 @@ static int rvq_decode_impl(const uint8_t* codes, int64_t code_stride_b, int64_t 
   // at 4,096 (the line), 11.1 and 11.4 at 8,192, 20.8 and 35.9 at 32,768.
   // S = 1 and fp32 tables or results cross between 4,096 and 8,192 tokens:
   // fp16 S = 1 5.9 and 5.4, then 8.0 and 7.9; fp32 S = 2 11.4 and 10.4, then
-  // 16.8 and 17.5; fp32 S = 1 9.1 and 7.8, then 13.9 and 13.5
-  const bool lds = B * H * T >= 32768 && d == 8 && K == 256 && G * S <= 32 && 512 % G == 0 && cw == 8 && depth <= 2 &&
+  // 16.8 and 17.5; fp32 S = 1 9.1 and 7.8, then 13.9 and 13.5.
+  // Tables beyond an XCD's L2 make gathers dear from about half the rows on:
+  // 64 heads of 256 tokens, S = 2, 7.8 and 10.3 fp32, 7.8 and 8.6 fp16; of
+  // 128 6.7 and 4.8; 128 heads of 200, fp16 S = 1, 5.8 and 7.3, of 128 5.2 and
+  // 4.6 (32 heads, fp32 S = 2, come out even: 10.1 and 11.9 at 768 tokens with
+  // fp16 results, 13.8 and 12.7 with fp32)
+  const int64_t table_bytes = H * G * S * K * d * (tables_f16 ? 2 : 4);
+  const int64_t lds_rows = table_bytes <= ((int64_t)4 << 20) ? 32768 : G * S > 16 ? 16384 : 24576;
+  const bool lds = B * H * T >= lds_rows && d == 8 && K == 256 && G * S <= 32 && 512 % G == 0 && cw == 8 && depth <= 2 &&
                    (uintptr_t)tables % 16 == 0 && B * H * ceil_div(T, kLdsDecodeTokens) < ((int64_t)1 << 31);
   if (lds) {
     // runs long enough for one round of workgroups over 256 CUs (each holds
