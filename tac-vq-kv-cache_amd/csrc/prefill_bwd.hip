@@ -896,12 +896,12 @@ __global__ __launch_bounds__(256) void value_grad_reduce_kernel(const float* __r
 }
 
 // Tiles per chunk and partial slots of the key-block kernels (blocks of
-// `keys` keys, n = B KVH slices): chunks of 16 tiles, of an eighth of the
-// longest block's rows when that is more, or shorter where the grid is small
-// and the workspace holds their slots (up to max_slots); the slots are the
-// most chunks one block meets.
-static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, int64_t max_slots, int* chunk_tiles,
-                              int* slots) {
+// `keys` keys, n = B KVH slices of nq query heads, nout outputs): chunks of
+// 16 tiles, of an eighth of the longest block's rows when that is more, or
+// shorter where the grid is small and the workspace holds their slots (up to
+// max_slots); the slots are the most chunks one block meets.
+static void value_grad_chunks(int64_t n, int64_t nq, int64_t T, int64_t window, int keys, int nout,
+                              int64_t max_slots, int* chunk_tiles, int* slots) {
   int64_t rows = (int64_t)keys - 1 + window;
   if (rows > T || rows < 0) rows = T;
   const int64_t span = ceil_div(rows, kBRows);  // tiles of the longest block (blocks start on a tile)
@@ -912,22 +912,42 @@ static void value_grad_chunks(int64_t n, int64_t T, int64_t window, int keys, in
     const int64_t most = ceil_div(span - 1, p) + 1;
     return all < most ? all : most;
   };
-  // shorter chunks while a launch has fewer walks than these (a block meets
-  // about half of the slots): the longest walk is the launch's time there,
-  // against partial slots to write and sum.  us per call, 16 tiles against
-  // the chosen ones: full backward [1,32/8,777] 142 -> 94, [2,512] 127 -> 80,
-  // [2,1024] 186 -> 158; value gradient alone [1,777] 76 -> 36, [2,1024]
-  // 83 -> 57, [1,2048] 101 -> 82; [2,2048] (1,280 and 640 walks) keeps 16
-  // (442; shorter ones 450)
+  // Shorter chunks while a launch has fewer walks than these (a block meets
+  // about half of the slots), and of those the least estimate: the longest
+  // walk at 1 us per tile and head, 5 us per walk on each of 256 CUs (its
+  // start and its sums' store), and for several chunks the second launch (2
+  // us an output) and the slots' traffic (70 ps a row).  us per call, 16 tiles
+  // against the chosen ones: full backward [1,32/8,777] 142 -> 94, [2,512]
+  // 127 -> 80, [2,1024] 186 -> 158; value gradient alone [1,777] 76 -> 36,
+  // [2,1024] 83 -> 57, [1,2048] 101 -> 82; [2,2048] (1,280 and 640 walks)
+  // keeps 16 (442; shorter ones 450).  Windows and single query heads keep 16
+  // where the count alone took 8 or fewer: [3,32/32,364] in a window of 64 51
+  // us both gradients and 24 the value's (8 tiles: 72 and 34), [8,8/8,503]
+  // value 30 (4 tiles: 42).  Over 1,375 drawn calls the choice is within 1 %
+  // of the best chunk length in the mean; 16 tiles alone are 15 % off.
+  const double seen = (double)rows * (1.0 - 0.5 * (double)rows / (double)T) / kBRows + keys / (2.0 * kBRows);
+  auto estimate = [&](int64_t p) {
+    const int64_t s = slots_of(p);
+    const double met = std::min((double)s, seen / (double)p + 1.0);
+    const double walks = (double)(n * ceil_div(T, (int64_t)keys)) * met;
+    const double reduce = s > 1 ? 2.0 * nout + 7e-5 * (double)(nout * s) * (double)(n * T) : 0.0;
+    return (double)(nq * std::min(p, span)) + 5.0 / 256 * walks + reduce;
+  };
+  double least = estimate(per);
+  int64_t best = per;
   while (per > 2) {
     const int64_t walks = n * ceil_div(T, (int64_t)keys) * (slots_of(per) + 1) / 2;
     if (walks >= (per >= 16 ? 640 : per >= 8 ? 400 : 250)) break;
-    const int64_t next = std::max<int64_t>(per / 2, 2);
-    if (slots_of(next) > 1 && slots_of(next) > max_slots) break;
-    per = next;
+    per = std::max<int64_t>(per / 2, 2);
+    if (slots_of(per) > 1 && slots_of(per) > max_slots) break;
+    const double t = estimate(per);
+    if (t <= least) {
+      least = t;
+      best = per;
+    }
   }
-  *chunk_tiles = (int)per;
-  *slots = (int)slots_of(per);
+  *chunk_tiles = (int)best;
+  *slots = (int)slots_of(best);
 }
 
 static const int64_t kAnySlots = (int64_t)1 << 62;
@@ -936,9 +956,9 @@ static const int64_t kAnySlots = (int64_t)1 << 62;
 // outputs (none where one chunk writes the results): of the chunks that the
 // rule wants, or with max_slots = 0 of the 16-tile ones, the least that a call
 // takes
-static int64_t slot_area(int64_t n, int64_t T, int64_t window, int keys, int nout, int64_t max_slots) {
+static int64_t slot_area(int64_t n, int64_t nq, int64_t T, int64_t window, int keys, int nout, int64_t max_slots) {
   int chunk_tiles, chunks;
-  value_grad_chunks(n, T, window, keys, max_slots, &chunk_tiles, &chunks);
+  value_grad_chunks(n, nq, T, window, keys, nout, max_slots, &chunk_tiles, &chunks);
   return chunks > 1 ? (int64_t)nout * chunks * n * T * kBD * (int64_t)sizeof(float) : 0;
 }
 
@@ -947,7 +967,7 @@ static int64_t slot_area(int64_t n, int64_t T, int64_t window, int keys, int nou
 // multiples of 256 bytes)
 static int64_t value_grad_workspace(int64_t B, int64_t QH, int64_t KVH, int64_t T, int64_t window,
                                     int64_t max_slots) {
-  return slot_area(B * KVH, T, window, kBKeys, 1, max_slots) + B * QH * T * kBD * 2;
+  return slot_area(B * KVH, QH / KVH, T, window, kBKeys, 1, max_slots) + B * QH * T * kBD * 2;
 }
 
 // bytes of the full backward's workspace: delta, the rotated keys and queries,
@@ -960,7 +980,7 @@ static int64_t backward_workspace(int64_t B, int64_t QH, int64_t KVH, int64_t T,
   const int64_t rot = B * (KVH + QH) * T * kBD * 2;
   const int64_t q = B * QH * T * kBD * (int64_t)sizeof(float);
   const int64_t v = value_grad_workspace(B, QH, KVH, T, window, max_slots);
-  const int64_t kv = slot_area(B * KVH, T, window, 64, 2, max_slots);
+  const int64_t kv = slot_area(B * KVH, QH / KVH, T, window, 64, 2, max_slots);
   return delta + rot + std::max(q, std::max(v, kv));
 }
 
@@ -1026,7 +1046,7 @@ static int launch_kv_grad(ValueGradArgs a, int64_t D, const int64_t (&strides)[1
   // that the rule wants and whose slots fit
   const int64_t n = B * KVH * T * kBD;
   const int64_t q_rot_bytes = q_rot_given != nullptr ? 0 : B * QH * T * kBD * 2;
-  const int64_t need = slot_area(B * KVH, T, a.window, keys, nout, 0) + q_rot_bytes;
+  const int64_t need = slot_area(B * KVH, NQ, T, a.window, keys, nout, 0) + q_rot_bytes;
   if (need > 0) {
     JKV_CHECK_ARG(workspace != nullptr && workspace_bytes >= need,
                   "prefill gradient workspace too small: %lld bytes, need %lld", (long long)workspace_bytes,
@@ -1035,7 +1055,8 @@ static int launch_kv_grad(ValueGradArgs a, int64_t D, const int64_t (&strides)[1
   }
   int chunk_tiles, chunks;
   const int64_t held = workspace != nullptr ? workspace_bytes - q_rot_bytes : 0;
-  value_grad_chunks(B * KVH, T, a.window, keys, held / (nout * n * (int64_t)sizeof(float)), &chunk_tiles, &chunks);
+  value_grad_chunks(B * KVH, NQ, T, a.window, keys, nout, held / (nout * n * (int64_t)sizeof(float)), &chunk_tiles,
+                    &chunks);
   a.chunk_tiles = chunk_tiles;
   a.slots = chunks;
   const int64_t slot_bytes = chunks > 1 ? (int64_t)chunks * n * (int64_t)sizeof(float) : 0;

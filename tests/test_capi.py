@@ -289,3 +289,11 @@ def test_backward_workspace_is_what_its_legs_use(batch, qh, kvh, tokens):
     # no factor of the key blocks' runs on the queries (it made these 2 to 5
     # times as large)
     assert size <= 150e6
+
+
+@pytest.mark.parametrize("batch,qh,kvh,tokens,window", [(3, 32, 32, 364, 64), (8, 8, 8, 503, 4096), (4, 64, 32, 351, 64)])
+def test_short_walks_are_not_split(batch, qh, kvh, tokens, window):
+    # one query head a walk, or a window of few tiles: runs of their own would
+    # cost more than they share out, so no partial slots, the rotated queries only
+    size = _lib.load().jkv_prefill_value_grad_workspace_bytes(batch, qh, kvh, tokens, window)
+    assert size == batch * qh * tokens * 128 * 2

@@ -193,6 +193,8 @@ def test_key_grad_entry_matches_backward_key_leg(device, batch, qh, kvh, tokens,
     (4, 32, 8, 512, 4096),     # four tiles; 512 query blocks, folded
     (2, 32, 8, 1000, 4096),    # eight tiles, ragged
     (32, 8, 8, 200, 4096),     # sixteen tiles: one chunk, no slots
+    (3, 32, 32, 364, 64),      # one head, a short window: sixteen on a small grid
+    (8, 8, 8, 503, 4096),      # one head: one chunk of all sixteen tiles
 ])
 def test_backward_chunk_rule_and_fp16_outputs(device, batch, qh, kvh, tokens, window):
     print(f"backward chunks B={batch} QH={qh} KVH={kvh} T={tokens} win={window}", flush=True)
