@@ -543,14 +543,21 @@ static int launch_prefill(PrefillArgs& a, int cs, const void* q, int64_t q_sb, i
   // of the order pair up (below).  [1,32/8,T]: T = 333 23.2 -> 17.7 us, 777
   // 40.0 -> 32.2, 2,048 91 -> 81; [2,1024] 52.9 -> 46.0; larger grids take
   // the same time or (2 x 2,048: 121 against 133) longer in four-wave form.
-  const int64_t n8 = ceil_div(T, 32 * (int64_t)(8 / a.heads_per_wg)) * KVH * (NQ / a.heads_per_wg) * B;
-  const int waves = cs == 0 && n8 <= 256 ? 4 : 8;
+  // Where a window binds, blocks are of one length, and where the slices do
+  // not spread over the XCDs no order pairs them: then, past about one block a
+  // CU, four-wave blocks of four heads stage each tile once more for nothing
+  // ([1,16/4,3673] in a window of 1,000 58 us with eight waves, 63 with four;
+  // [2,4/1,6330] of 1,676 78 and 86).
+  const int64_t slices = KVH * (NQ / a.heads_per_wg) * B;
+  const int64_t n8 = ceil_div(T, 32 * (int64_t)(8 / a.heads_per_wg)) * slices;
+  const int64_t n4 = ceil_div(T, 32 * (int64_t)std::max(1, 4 / a.heads_per_wg)) * slices;
+  const bool even = a.heads_per_wg == 4 && slices % 8 != 0 && window < T - T / 5 && n4 > 280;
+  const int waves = cs == 0 && n8 <= 256 && !even ? 4 : 8;
   a.row_sets = waves / a.heads_per_wg;
   a.head_groups = (int32_t)(NQ / a.heads_per_wg);
   const int64_t nqb = ceil_div(T, 32 * (int64_t)a.row_sets);
-  const int64_t blocks = nqb * KVH * a.head_groups * B;
+  const int64_t blocks = nqb * slices;
   JKV_CHECK_ARG(blocks < ((int64_t)1 << 31), "prefill grid too large");
-  const int64_t slices = KVH * a.head_groups * B;
   a.group = 1;
   a.fold = 0;
   if (slices % 8 == 0) {

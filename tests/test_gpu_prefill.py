@@ -51,6 +51,7 @@ def test_prefill_matches_oracle(device, batch, qh, kvh, tokens, starts, window):
     (3, 8, 1, 300, (0, 1, 2), 4096),      # six slices (GQA 8): no runs
     (8, 8, 8, 300, (5,) * 8, 4096),       # one head per block, runs of eight slices
     (6, 32, 8, 770, (0,) * 6, 4096),      # eight waves, runs of several slices
+    (3, 16, 4, 800, (0, 1, 2), 128),      # twelve slices, a window that binds: eight waves on a small grid
 ])
 def test_prefill_grid_forms(device, batch, qh, kvh, tokens, starts, window):
     print(f"prefill forms B={batch} QH={qh} KVH={kvh} T={tokens} win={window}", flush=True)
