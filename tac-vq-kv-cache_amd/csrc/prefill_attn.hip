@@ -565,8 +565,14 @@ static int launch_prefill(PrefillArgs& a, int cs, const void* q, int64_t q_sb, i
     // half of its 4 MiB L2 (slice by slice, each began with long blocks while
     // the one before ended: [4,32/8,1024] 94 -> 72 us, [16,2048] 922 -> 883,
     // [64,512] 438 -> 390); four-wave blocks that all reside at once fold
-    // ([2,1024] 56.6 -> 46.0, [4,512] 35.0 -> 29.1)
-    const int64_t per = slices / 8, cap = std::max<int64_t>(1, (2 << 20) / (T * 512));
+    // ([2,1024] 56.6 -> 46.0, [4,512] 35.0 -> 29.1).  Codes: a slice's tables
+    // (128 KiB a stage) and records count too (12 rows of 191 tokens, 128/32
+    // heads, two stages: 104 us slice by slice, 113 with more slices than
+    // tables fit, 101 so)
+    const int64_t per = slices / 8;
+    int64_t bytes = T * 512;
+    if (cs > 0) bytes = std::max<int64_t>(bytes, cs * (131072 + T * 32));
+    const int64_t cap = std::max<int64_t>(1, (2 << 20) / bytes);
     for (int64_t g = 1; g <= per && g <= cap; ++g)
       if (per % g == 0) a.group = (int32_t)g;
     if (waves == 4 && blocks > 256 && blocks <= 512) a.fold = 32;
