@@ -115,7 +115,9 @@ __global__ __launch_bounds__(64 * NWV) void prefill_attn_kernel(PrefillArgs a) {
   const int ln = lane & 15, lg = lane >> 4;
   const int HW = a.heads_per_wg, RS = a.row_sets;
   const int64_t block_rows = 32 * (int64_t)RS;
-  const int64_t nqb = ceil_div(a.T, block_rows);
+  // (block, slice and token counts fit 32 bits, host-checked: 64-bit divisions
+  // here are 0.2 us of a small call)
+  const uint32_t nqb = ((uint32_t)a.T + (uint32_t)block_rows - 1u) / (uint32_t)block_rows;
   // logical block: an XCD's blocks are runs of `group` (batch row, kv head,
   // head group) slices, each run longest key ranges first over all its
   // slices.  xcd_remap keeps the query blocks of one slice on one XCD, so its
@@ -127,14 +129,13 @@ __global__ __launch_bounds__(64 * NWV) void prefill_attn_kernel(PrefillArgs a) {
     const uint32_t per = gridDim.x >> 3, at = bid % per, first = (uint32_t)a.fold;
     if (at >= first) bid += per - 1 - at + first - at;  // at -> first + (per - 1 - at)
   }
-  const int64_t gy = a.KVH * a.head_groups;
-  const uint32_t run = (uint32_t)a.group * (uint32_t)nqb, in_run = bid % run;
-  const int64_t qblk = nqb - 1 - (int64_t)(in_run / (uint32_t)a.group);
-  const int64_t yz = (int64_t)(bid / run) * a.group + in_run % (uint32_t)a.group;
-  const int64_t kvh = (yz % gy) / a.head_groups;
-  const int64_t hg = (yz % gy) % a.head_groups;
-  const int64_t b = yz / gy;
-  const int64_t NQ = a.QH / a.KVH;
+  const uint32_t group = (uint32_t)a.group, run = group * nqb, run_at = bid / run, in_run = bid - run_at * run;
+  const uint32_t back = in_run / group, yz = run_at * group + (in_run - back * group);
+  const int64_t qblk = (int64_t)(nqb - 1u - back);
+  const uint32_t hgs = (uint32_t)a.head_groups, gy = (uint32_t)a.KVH * hgs;
+  const uint32_t b32 = yz / gy, in_b = yz - b32 * gy, kvh32 = in_b / hgs;
+  const int64_t b = b32, kvh = kvh32, hg = in_b - kvh32 * hgs;
+  const int64_t NQ = (int64_t)HW * a.head_groups;
   const int64_t head = kvh * NQ + hg * HW + wave % HW;
   const int64_t wg_row0 = qblk * block_rows;
   int64_t wg_row1 = wg_row0 + block_rows;
