@@ -914,9 +914,11 @@ static void value_grad_chunks(int64_t n, int64_t nq, int64_t T, int64_t window, 
   };
   // Shorter chunks while a launch has fewer walks than these (a block meets
   // about half of the slots), and of those the least estimate: the longest
-  // walk at 1 us per tile and head, 5 us per walk on each of 256 CUs (its
-  // start and its sums' store), and for several chunks the second launch (2
-  // us an output) and the slots' traffic (70 ps a row).  us per call, 16 tiles
+  // walk at 1 us per tile and head (15 % more where walks outnumber the three
+  // that a CU holds: [4,128/32,393] in a window of 300, value 91 us with one
+  // chunk, 106 with two), 5 us per walk on each of 256 CUs (its start and its
+  // sums' store), and for several chunks the second launch (2 us an output)
+  // and the slots' traffic (70 ps a row).  us per call, 16 tiles
   // against the chosen ones: full backward [1,32/8,777] 142 -> 94, [2,512]
   // 127 -> 80, [2,1024] 186 -> 158; value gradient alone [1,777] 76 -> 36,
   // [2,1024] 83 -> 57, [1,2048] 101 -> 82; [2,2048] (1,280 and 640 walks)
@@ -931,7 +933,8 @@ static void value_grad_chunks(int64_t n, int64_t nq, int64_t T, int64_t window, 
     const double met = std::min((double)s, seen / (double)p + 1.0);
     const double walks = (double)(n * ceil_div(T, (int64_t)keys)) * met;
     const double reduce = s > 1 ? 2.0 * nout + 7e-5 * (double)(nout * s) * (double)(n * T) : 0.0;
-    return (double)(nq * std::min(p, span)) + 5.0 / 256 * walks + reduce;
+    const double crowd = walks > 3 * 256 ? 1.15 : 1.0;
+    return crowd * (double)(nq * std::min(p, span)) + 5.0 / 256 * walks + reduce;
   };
   double least = estimate(per);
   int64_t best = per;
