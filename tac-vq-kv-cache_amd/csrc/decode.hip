@@ -224,9 +224,10 @@ static int rvq_decode_impl(const uint8_t* codes, int64_t code_stride_b, int64_t 
   // 64 heads of 256 tokens, S = 2, 7.8 and 10.3 fp32, 7.8 and 8.6 fp16; of
   // 128 6.7 and 4.8; 128 heads of 200, fp16 S = 1, 5.8 and 7.3, of 128 5.2 and
   // 4.6 (32 heads, fp32 S = 2, come out even: 10.1 and 11.9 at 768 tokens with
-  // fp16 results, 13.8 and 12.7 with fp32)
+  // fp16 results, 13.8 and 12.7 with fp32).  Fewer stages than are staged
+  // gather less: 64 heads of 333, one of two fp32 stages, 10.2 and 7.0
   const int64_t table_bytes = H * G * S * K * d * (tables_f16 ? 2 : 4);
-  const int64_t lds_rows = table_bytes <= ((int64_t)4 << 20) ? 32768 : G * S > 16 ? 16384 : 24576;
+  const int64_t lds_rows = table_bytes <= ((int64_t)4 << 20) || depth < S ? 32768 : G * S > 16 ? 16384 : 24576;
   const bool lds = B * H * T >= lds_rows && d == 8 && K == 256 && G * S <= 32 && 512 % G == 0 && cw == 8 && depth <= 2 &&
                    (uintptr_t)tables % 16 == 0 && B * H * ceil_div(T, kLdsDecodeTokens) < ((int64_t)1 << 31);
   if (lds) {
@@ -237,8 +238,13 @@ static int rvq_decode_impl(const uint8_t* codes, int64_t code_stride_b, int64_t 
     // lies between 16 and 32 heads at S = 2 (16 heads of 3,072 tokens: 12.0 us
     // with 128, 12.5 with 512) and 64 and 128 at S = 1 (64 of 768: 9.0, 9.8)
     const bool far = !tables_f16 && H * (G * S) * (G * S) > 16384;
-    a.run_tokens = (int32_t)std::max<int64_t>(far ? kLdsDecodeFarTokens : kLdsDecodeTokens,
-                                              ceil_div(T, runs_per_slice));
+    // equal runs, none of a few tokens, which would stage the tables all the
+    // same (2 rows of 64 heads and 157 tokens, fp32 results: 9.3 us in one run
+    // each, 11.8 in runs of 128 and 29)
+    const int64_t wanted = far ? ceil_div(T, kLdsDecodeFarTokens)
+                               : std::max<int64_t>(1, (T + kLdsDecodeTokens / 2) / kLdsDecodeTokens);
+    const int64_t runs = std::min(runs_per_slice, wanted);
+    a.run_tokens = (int32_t)ceil_div(T, runs);
     switch (out_dtype) {
       case JKV_F16:
         tables_f16 ? launch_decode_lds<JKV_F16, true>(a, stream) : launch_decode_lds<JKV_F16, false>(a, stream);

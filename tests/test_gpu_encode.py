@@ -457,7 +457,8 @@ def test_rvq_decode_staging_rule(device, tokens, tables_f16):
 # with a partial last run
 # and either side of the rows from which many heads' tables are staged
 @pytest.mark.parametrize("heads,tokens,stages", [(16, 2100, 2), (17, 2100, 2), (40, 1030, 2), (65, 520, 1),
-                                                 (40, 409, 2), (40, 410, 2), (70, 351, 1), (70, 352, 1)])
+                                                 (40, 409, 2), (40, 410, 2), (70, 351, 1), (70, 352, 1),
+                                                 (130, 157, 2), (100, 191, 2), (100, 192, 2)])
 def test_rvq_decode_runs_of_many_heads(device, heads, tokens, stages):
     gen = _gen(6464 + heads)
     tables = ref.synthetic_tables(gen, (heads * 16, stages, 256, 8), (1.0, 0.5)[:stages], stage_axis=1)
