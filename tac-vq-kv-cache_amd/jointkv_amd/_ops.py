@@ -8,6 +8,7 @@ on the current HIP stream.  Nothing here computes on the CPU.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Sequence
 
 import torch
@@ -21,6 +22,16 @@ def _encode_states_strides(states: torch.Tensor) -> tuple[torch.Tensor, tuple[in
         states = states.contiguous()
         strides = states.stride()
     return states, strides[:3]
+
+
+def _plain(like: torch.Tensor):
+    """Allocator of plain tensors beside ``like``, of its dtype unless told
+    otherwise: ``new_empty`` costs the host 0.7 us less than ``torch.empty``
+    but hands a subclass on."""
+
+    if type(like) is torch.Tensor:
+        return like.new_empty
+    return functools.partial(torch.empty, dtype=like.dtype, device=like.device)
 
 
 def rvq_encode(
@@ -52,14 +63,15 @@ def rvq_encode(
         raise ValueError(f"at most {_lib.MAX_EXITS} exits per call")
     lib = _lib.load()
     states, (sb, sh, st) = _encode_states_strides(states)
+    empty = _plain(states)
     if codes_out is None:
-        codes = torch.empty((batch, heads, tokens, groups, stages), dtype=torch.uint8, device=device)
+        codes = empty((batch, heads, tokens, groups, stages), dtype=torch.uint8)
     else:
         codes = codes_out
         if (codes.dtype != torch.uint8 or tuple(codes.shape) != (batch, heads, tokens, groups, stages)
                 or codes.stride(-1) != 1 or codes.stride(-2) != stages or codes.device != device):
             raise ValueError("codes_out must be uint8 [B,H,T,G,S] with a contiguous (G,S) block")
-    recon = [torch.empty((batch, heads, tokens, dim), dtype=states.dtype, device=device) for _ in exits]
+    recon = [empty((batch, heads, tokens, dim)) for _ in exits]
     if whiteners is not None:
         whiteners = whiteners.detach().float().contiguous()
         if tuple(whiteners.shape) != (problems, d, d):
@@ -113,10 +125,11 @@ def rvq_encode_kv(
         key, strides = _encode_states_strides(key.contiguous())
         value, vstrides = _encode_states_strides(value.contiguous())
     codes = []
+    empty = _plain(key)
     shape = (batch, heads, tokens, groups, stages)
     for out in (key_codes_out, value_codes_out):
         if out is None:
-            out = torch.empty(shape, dtype=torch.uint8, device=device)
+            out = empty(shape, dtype=torch.uint8)
         elif (out.dtype != torch.uint8 or tuple(out.shape) != shape
               or out.stride(-1) != 1 or out.stride(-2) != stages or out.device != device):
             raise ValueError("codes_out must be uint8 [B,H,T,G,S] with a contiguous (G,S) block")
@@ -124,8 +137,8 @@ def rvq_encode_kv(
     code_strides = codes[0].stride()[:3]
     if code_strides != codes[1].stride()[:3]:
         raise ValueError("K and V code outputs must share their strides")
-    recon_k = [torch.empty((batch, heads, tokens, dim), dtype=key.dtype, device=device) for _ in exits]
-    recon_v = [torch.empty((batch, heads, tokens, dim), dtype=key.dtype, device=device) for _ in exits]
+    recon_k = [empty((batch, heads, tokens, dim)) for _ in exits]
+    recon_v = [empty((batch, heads, tokens, dim)) for _ in exits]
     lib = _lib.load()
     ws_bytes = _lib.workspace_bytes("jkv_rvq_encode_workspace_bytes", heads, groups, stages, clusters, d, 0)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device) if ws_bytes else None
@@ -604,7 +617,7 @@ def decode_attention(
     # shorter than the model's window)
     span = max(1, min(int(window), int(max_length)))
     lib = _lib.load()
-    out = torch.empty((batch, qheads, dim), dtype=torch.float16, device=device)
+    out = _plain(q)((batch, qheads, dim))
     ws_bytes = _lib.workspace_bytes("jkv_decode_workspace_bytes", batch, qheads, dim, span)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     if key_new is None and value_new is None:
@@ -677,7 +690,7 @@ def decode_attention_window(
     table = rope_table(device, rope_theta, int(max_length) + 1)
     span = max(1, min(int(window), int(max_length)))
     lib = _lib.load()
-    out = torch.empty((batch, qheads, dim), dtype=torch.float16, device=device)
+    out = _plain(q)((batch, qheads, dim))
     ws_bytes = _lib.workspace_bytes("jkv_decode_workspace_bytes", batch, qheads, dim, span)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=device)
     code = lib.jkv_decode_attention_window(
@@ -741,7 +754,7 @@ def prefill_attention(
                             or not lse.is_contiguous() or lse.device != q.device):
         raise ValueError("lse must be a contiguous fp32 [B,QH,T] tensor on the query's device")
     table = rope_table(device, rope_theta, int(max_position) + 1)
-    out = torch.empty((batch, qheads, tokens, 128), dtype=torch.float16, device=device)
+    out = _plain(q)((batch, qheads, tokens, 128))
     code = _lib.load().jkv_prefill_attention(
         q.data_ptr(), *q.stride()[:3], key.data_ptr(), *key.stride()[:3], value.data_ptr(),
         *value.stride()[:3], batch, qheads, kvheads, tokens, 128, start_positions.data_ptr(),
@@ -818,7 +831,7 @@ def prefill_attention_codes(
             t = t.to(torch.float16).contiguous()
         tables.append(t)
     table = rope_table(device, rope_theta, int(max_position) + 1)
-    out = torch.empty((batch, qheads, tokens, 128), dtype=torch.float16, device=device)
+    out = _plain(q)((batch, qheads, tokens, 128))
     kc, vc = codes
     code = _lib.load().jkv_prefill_attention_codes(
         q.data_ptr(), *q.stride()[:3], kc.data_ptr(), vc.data_ptr(), *kc.stride()[:3], tables[0].data_ptr(),
